@@ -388,44 +388,37 @@ struct AdvMuT {
   int k1, kde, j0, j1, i0, i1;
 };
 
-// Operands are loaded into registers before the arithmetic so that the loads
-// of one level are in flight together.
-__device__ inline float mut_dvdxi(const Dims& D, const AdvMuT& a, int k, int j, int i) {
-  const float vn = AT(a.v, k, j + 1, i), mvn = AT2(a.muv, j + 1, i), v1n = AT(a.v_1, k, j + 1, i);
-  const float xn = AT2(a.msfvx_inv, j + 1, i);
-  const float vs = AT(a.v, k, j, i), mvs = AT2(a.muv, j, i), v1s = AT(a.v_1, k, j, i), xs = AT2(a.msfvx_inv, j, i);
-  const float ue = AT(a.u, k, j, i + 1), mue = AT2(a.muu, j, i + 1), u1e = AT(a.u_1, k, j, i + 1);
-  const float ye = AT2(a.msfuy, j, i + 1);
-  const float uw = AT(a.u, k, j, i), muw = AT2(a.muu, j, i), u1w = AT(a.u_1, k, j, i), yw = AT2(a.msfuy, j, i);
-  const float mx = AT2(a.msftx, j, i), my = AT2(a.msfty, j, i);
-  float vy = (vn + mvn * v1n * xn) - (vs + mvs * v1s * xs);
-  float ux = (ue + mue * u1e / ye) - (uw + muw * u1w / yw);
-  return mx * my * (a.rdy * vy + a.rdx * ux);
-}
-
 // Column block: a 512-thread workgroup owns TI consecutive i-columns of one
-// row j and all levels.  The divergence dvdxi of every (k, i) is computed by
-// all threads and staged in LDS; one thread per column then forms the column
-// sum, the column-mass update and the eta-velocity recurrence from LDS; all
-// threads finally apply the theta update level by level (coalesced in i).
-// Columns outside the update box copy their inputs (clone semantics).
+// row j and all levels; wave `grp` takes levels grp, grp + TG, ...  The
+// divergence dvdxi of every (k, i) is computed by all waves and staged in LDS;
+// the column sum, the column-mass update and the eta-velocity recurrence
+// follow from LDS; all waves finally apply the theta update.  Columns outside
+// the update box copy their inputs (clone semantics).
+//
+// What bounds it is memory latency: the grid's blocks are all resident at once
+// and reach each phase together, so every phase that loads costs a full
+// round trip.  Each wave therefore loads everything it will need, for all of
+// its LPT levels, before the first barrier (no load is under a branch; level
+// indices are clamped to k1 - 1), and keeps five values a level in registers
+// across the serial part; after it there are only stores.  Each level's
+// vertical theta flux is formed once and passed to the level below in LDS.
 #define TI 64
 #define TB 512
 #define TG (TB / TI)
 
 #define CB_MAXNZ 128   // column blocks hold at most 64 KB of per-level LDS, so nz <= 128
 
+// the wave's number, known to the compiler to be the same in all its lanes
+__device__ __forceinline__ int wave_of_block() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x / TI); }
+
+template <int LPT>
 __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
   extern __shared__ float sm[];
-  __shared__ float s_dnw[CB_MAXNZ], s_fnm[CB_MAXNZ], s_fnp[CB_MAXNZ], s_rdnw[CB_MAXNZ];
   __shared__ float s_part[(CB_MAXNZ / 16 + 1) * TI];
-  const int nz = D.nz;
-  for (int t = threadIdx.x; t < nz; t += TB) {
-    s_dnw[t] = a.dnw[t]; s_fnm[t] = a.fnm[t]; s_fnp[t] = a.fnp[t]; s_rdnw[t] = a.rdnw[t];
-  }
-  float* s_dv = sm;             // [nz][TI] dvdxi
+  const int nz = D.nz, k1 = a.k1;
+  float* s_dv = sm;             // [nz][TI] dvdxi, then the eta-velocity decrements, then the theta fluxes
   float* s_ww = sm + nz * TI;   // [nz][TI] eta velocity before subtracting ww_1
-  const int lane = threadIdx.x % TI, grp = threadIdx.x / TI;
+  const int lane = threadIdx.x % TI, grp = wave_of_block();
   int bx, by;
 #if PW_COL_XCD
   xcd_block_2d(bx, by);
@@ -434,71 +427,100 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
 #endif
   const int j = by, i = bx * TI + lane;
   const bool vi = i < D.nx;
-  const bool h = vi && j >= a.j0 && j < a.j1 && i >= a.i0 && i < a.i1;
-  const long q2 = vi ? D.ix2(j, i) : 0;
-  for (int k = grp; k < nz; k += TG) {
-    if (!vi) continue;
-    long q = D.ix(k, j, i);
-    if (!h) {
-      a.ww[q] = a.ww_in[q];
-      a.t[q] = a.t_in[q];
-      a.t_ave[q] = a.t_ave_in[q];
-      continue;
+  const bool row = j >= a.j0 && j < a.j1 && a.i0 < a.i1;
+  const bool h = vi && row && i >= a.i0 && i < a.i1;
+  if (vi && !h) {
+    for (int k = grp; k < nz; k += TG) {
+      const long q = D.ix(k, j, i);
+      const float x = a.ww_in[q], y = a.t_in[q], z = a.t_ave_in[q];
+      a.ww[q] = x;
+      a.t[q] = y;
+      a.t_ave[q] = z;
     }
-    s_dv[k * TI + lane] = k < a.k1 ? mut_dvdxi(D, a, k, j, i) : 0.0f;
+    if (grp == 0) {
+      const long q = D.ix2(j, i);
+      const float x = a.muave_in[q], y = a.muts_in[q], z = a.mudf_in[q], m = a.mu_in[q];
+      a.muave[q] = x;
+      a.muts[q] = y;
+      a.mudf[q] = z;
+      a.mu[q] = m;
+    }
   }
-  if (vi && !h && grp == 0) {
-    a.muave[q2] = a.muave_in[q2];
-    a.muts[q2] = a.muts_in[q2];
-    a.mudf[q2] = a.mudf_in[q2];
-    a.mu[q2] = a.mu_in[q2];
+  if (!row) return;   // the whole block
+  const int ic = imin(imax(i, a.i0), a.i1 - 1);   // lanes outside the box load (and drop) its edge column's values
+  const long q2 = D.ix2(j, ic);
+  const float mvn = AT2(a.muv, j + 1, ic), xn = AT2(a.msfvx_inv, j + 1, ic), mvs = a.muv[q2], xs = a.msfvx_inv[q2];
+  const float mue = AT2(a.muu, j, ic + 1), ye = AT2(a.msfuy, j, ic + 1), muw = a.muu[q2], yw = a.msfuy[q2];
+  const float mx = a.msftx[q2], my = a.msfty[q2], mt = a.mu_tend[q2], mu_old = a.mu_in[q2], mut = a.mut[q2];
+  const float ww0 = AT(a.ww_in, 0, j, ic);
+  float r_t[LPT], r_p[LPT], r_h[LPT], r_c[LPT], r_w1[LPT];
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = imin(grp + m * TG, k1 - 1), kd = imax(k - 1, 0);
+    const float vn = AT(a.v, k, j + 1, ic), v1n = AT(a.v_1, k, j + 1, ic), vs = AT(a.v, k, j, ic), v1s = AT(a.v_1, k, j, ic);
+    const float ue = AT(a.u, k, j, ic + 1), u1e = AT(a.u_1, k, j, ic + 1), uw = AT(a.u, k, j, ic), u1w = AT(a.u_1, k, j, ic);
+    const float tin = AT(a.t_in, k, j, ic), ftq = AT(a.ft, k, j, ic), t1 = AT(a.t_1, k, j, ic), t1d = AT(a.t_1, kd, j, ic);
+    const float tn = AT(a.t_1, k, j + 1, ic), ts = AT(a.t_1, k, j - 1, ic);
+    const float te = AT(a.t_1, k, j, ic + 1), tw = AT(a.t_1, k, j, ic - 1);
+    r_w1[m] = AT(a.ww_1, k, j, ic);
+    const float vy = (vn + mvn * v1n * xn) - (vs + mvs * v1s * xs);
+    const float ux = (ue + mue * u1e / ye) - (uw + muw * u1w / yw);
+    const float dv = mx * my * (a.rdy * vy + a.rdx * ux);
+    if (grp + m * TG < k1) s_dv[k * TI + lane] = dv;
+    const float yterm = a.hrdy * (vn * (tn + t1) - vs * (t1 + ts));
+    const float xterm = a.hrdx * (ue * (te + t1) - uw * (t1 + tw));
+    r_t[m] = tin + 0.0f;
+    r_p[m] = tin + my * a.dts * ftq;
+    r_h[m] = mx * (yterm + xterm);
+    r_c[m] = a.fnm[k] * t1 + a.fnp[k] * t1d;
   }
   __syncthreads();
   // The column sum dmdt in torch's order (torch_outer_sum with nz <= 128:
   // blocks of 16 levels summed from +0 one after the other, the tail from +0,
-  // tail + (sum of the block sums) + 0 + 0): each block's chain and the
-  // tail's are independent, so the groups form them side by side.
+  // tail + (sum of the block sums) + 0 + 0; levels from k1 on add +0, which
+  // changes no partial sum): each block's chain and the tail's are
+  // independent, so the waves form them side by side.
   const int nb = nz >> 4;
   for (int c = grp; c <= nb; c += TG) {
+    const int k0 = c << 4, ke = imin(imin(k0 + 16, nz), k1);
     float acc = 0.0f;
-    if (h) {
-      const int k0 = c << 4, k1 = imin(k0 + 16, nz);
-      for (int k = k0; k < k1; ++k) acc += k < a.k1 ? s_dnw[k] * s_dv[k * TI + lane] : 0.0f;
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      const int k = imin(k0 + m, k1 - 1);
+      const float x = a.dnw[k] * s_dv[k * TI + lane];
+      acc += k0 + m < ke ? x : 0.0f;
     }
     s_part[c * TI + lane] = acc;
   }
   __syncthreads();
+  // every wave forms the column's dmdt from the block sums (the same floats)
+  float blocks = 0.0f;
+  for (int c = 0; c < nb; ++c) blocks += s_part[c * TI + lane];
+  float dmdt = s_part[nb * TI + lane] + blocks;
+  dmdt = dmdt + 0.0f;
+  dmdt = dmdt + 0.0f;
   if (grp == 0 && h) {
-    float blocks = 0.0f;
-    for (int c = 0; c < nb; ++c) blocks += s_part[c * TI + lane];
-    float dmdt = s_part[nb * TI + lane] + blocks;
-    dmdt = dmdt + 0.0f;
-    dmdt = dmdt + 0.0f;
-    float mt = a.mu_tend[q2];
-    float mu_old = a.mu_in[q2];
-    float mu = mu_old + a.dts * (dmdt + mt);
+    const float mu = mu_old + a.dts * (dmdt + mt);
     a.mu[q2] = mu;
     a.mudf[q2] = dmdt + mt;
-    a.muts[q2] = a.mut[q2] + mu;
+    a.muts[q2] = mut + mu;
     a.muave[q2] = 0.5f * (a.ep1 * mu + a.em1 * (mu_old + 0.0f));
-    s_part[lane] = dmdt;
+  }
+  // the eta-velocity decrements dnw(k) (dmdt + dvdxi(k) + mu_tend) / msfty of
+  // every level at once, in place of dvdxi(k) (this wave's own entries)
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = grp + m * TG;
+    if (k < k1) s_dv[k * TI + lane] = a.dnw[k] * (dmdt + s_dv[k * TI + lane] + mt) / my;
   }
   __syncthreads();
-  // the eta-velocity decrements dnw(k-1) (dmdt + dvdxi(k-1) + mu_tend) / msfty
-  // of every level at once (in place of dvdxi(k-1), which nothing reads again)
-  if (h) {
-    const float dmdt = s_part[lane], mt = a.mu_tend[q2], my = a.msfty[q2];
-    for (int k = 1 + grp; k < a.k1; k += TG)
-      s_dv[(k - 1) * TI + lane] = s_dnw[k - 1] * (dmdt + s_dv[(k - 1) * TI + lane] + mt) / my;
-  }
-  __syncthreads();
-  if (grp == 0 && h) {
+  if (grp == 0) {
     // the decrements 8 levels at a time into registers first (s_dv and s_ww
     // share one LDS buffer, so a read after a store to s_ww would wait for it)
-    float wk = a.ww_in[D.ix(0, j, i)];
+    float wk = ww0;
     s_ww[lane] = wk;
     int k = 1;
-    for (; k + 7 < a.k1; k += 8) {
+    for (; k + 7 < k1; k += 8) {
       float dv[8];
 #pragma unroll
       for (int m = 0; m < 8; ++m) dv[m] = s_dv[(k - 1 + m) * TI + lane];
@@ -508,57 +530,40 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
         s_ww[(k + m) * TI + lane] = wk;
       }
     }
-    for (; k < a.k1; ++k) {
+    for (; k < k1; ++k) {
       wk = wk - s_dv[(k - 1) * TI + lane];
       s_ww[k * TI + lane] = wk;
     }
   }
   __syncthreads();
-  if (!h) return;
-  const float my = a.msfty[q2], mx = a.msftx[q2];
-  // theta and eta velocity of level k < k1 from loads only (indices clamped;
-  // the values taken at clamped indices are not used)
-  auto level = [&](int k, float& o_ww, float& o_t) {
-    const long q = D.ix(k, j, i);
-    const int ku = imin(k + 1, nz - 1), kd = imax(k - 1, 0);
-    const float tin = a.t_in[q], ftq = a.ft[q], t1 = a.t_1[q], w1k = a.ww_1[q];
-    const float vn = AT(a.v, k, j + 1, i), vs = AT(a.v, k, j, i), ue = AT(a.u, k, j, i + 1), uw = AT(a.u, k, j, i);
-    const float tn = AT(a.t_1, k, j + 1, i), ts = AT(a.t_1, k, j - 1, i);
-    const float te = AT(a.t_1, k, j, i + 1), tw = AT(a.t_1, k, j, i - 1);
-    const bool up = k + 1 < a.k1, dn = k > 0;   // where the eta fluxes wdtn(k + 1), wdtn(k) are nonzero
-    const float w1u = AT(a.ww_1, ku, j, i), t1u = AT(a.t_1, ku, j, i), t1d = AT(a.t_1, kd, j, i);
-    const float wwk = s_ww[k * TI + lane] - w1k;
-    o_ww = wwk;
-    float t = tin + my * a.dts * ftq;
-    const float wdu = up ? (s_ww[ku * TI + lane] - w1u) * (s_fnm[ku] * t1u + s_fnp[ku] * t1) : 0.0f;
-    const float wdk = dn ? wwk * (s_fnm[k] * t1 + s_fnp[k] * t1d) : 0.0f;
-    float yterm = a.hrdy * (vn * (tn + t1) - vs * (t1 + ts));
-    float xterm = a.hrdx * (ue * (te + t1) - uw * (t1 + tw));
-    o_t = t - a.dts * my * (mx * (yterm + xterm) + s_rdnw[k] * (wdu - wdk));
-  };
-  // two of the thread's levels at a time, every load before the stores (the
-  // second level clamped to the last one below k1 and stored only if real)
-  for (int k = grp; k < a.k1; k += 2 * TG) {
-    const int k2 = imin(k + TG, a.k1 - 1);
-    float w0, t0, w1, t1;
-    level(k, w0, t0);
-    level(k2, w1, t1);
-    const long q = D.ix(k, j, i), qb = D.ix(k2, j, i);
-    const float ta0 = a.t_in[q] + 0.0f, ta1 = a.t_in[qb] + 0.0f;
-    a.ww[q] = w0;
-    a.t_ave[q] = ta0;
-    a.t[q] = t0;
-    if (k + TG < a.k1) {
-      a.ww[qb] = w1;
-      a.t_ave[qb] = ta1;
-      a.t[qb] = t1;
+  // the vertical theta flux wdtn(k) of each level (zero at k = 0) into s_dv
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = grp + m * TG;
+    if (k < k1) {
+      const float wwk = s_ww[k * TI + lane] - r_w1[m];
+      r_w1[m] = wwk;
+      r_c[m] = k > 0 ? wwk * r_c[m] : 0.0f;
+      s_dv[k * TI + lane] = r_c[m];
     }
   }
-  for (int k = a.k1 + grp; k < nz; k += TG) {   // levels at and above k1 copy their inputs
+  __syncthreads();
+  if (!h) return;
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = grp + m * TG;
+    if (k >= k1) continue;
+    const float wdu = k + 1 < k1 ? s_dv[(k + 1) * TI + lane] : 0.0f;
+    AT(a.ww, k, j, i) = r_w1[m];
+    AT(a.t_ave, k, j, i) = r_t[m];
+    AT(a.t, k, j, i) = r_p[m] - a.dts * my * (r_h[m] + a.rdnw[k] * (wdu - r_c[m]));
+  }
+  for (int k = k1 + grp; k < nz; k += TG) {   // levels at and above k1 copy their inputs
     const long q = D.ix(k, j, i);
-    a.ww[q] = a.ww_in[q];
-    a.t[q] = a.t_in[q];
-    a.t_ave[q] = a.t_ave_in[q];
+    const float x = a.ww_in[q], y = a.t_in[q], z = a.t_ave_in[q];
+    a.ww[q] = x;
+    a.t[q] = y;
+    a.t_ave[q] = z;
   }
 }
 
@@ -587,7 +592,9 @@ extern "C" int pywrf_advance_mu_t(const pywrf_grid_t* g, const float* ww_in, con
               imax(g->its, g->ids + 1), imin(g->ite, g->ide - 2)};
   if (column_block_launch_check(g, 2)) return PYWRF_E_RANGE;
   dim3 grid((g->nx + TI - 1) / TI, g->ny);
-  hipLaunchKernelGGL(k_advance_mu_t, grid, dim3(TB), 2 * g->nz * TI * sizeof(float), (hipStream_t)s, dims_of(g), a);
+  // levels a wave keeps in registers: 5 covers the model's 40 mass levels
+  auto kern = a.k1 <= 5 * TG ? k_advance_mu_t<5> : a.k1 <= 8 * TG ? k_advance_mu_t<8> : k_advance_mu_t<16>;
+  hipLaunchKernelGGL(kern, grid, dim3(TB), 2 * g->nz * TI * sizeof(float), (hipStream_t)s, dims_of(g), a);
   PW_RET();
 }
 
@@ -601,29 +608,26 @@ struct AdvW {
   int k1, j0, j1, i0, i1;
 };
 
-// Column block as in advance_mu_t.  Phase 1 (all threads): t_2ave and the
-// phi right-hand side rhs for every (k, i), staged in LDS with the
-// tridiagonal factors a, alpha, gamma.  Phase 2 (all threads): surface w and
-// the explicit w predictor from the LDS rhs / t_2ave.  Phase 3 (one thread
-// per column): Thomas forward sweep and back substitution in LDS.  Phase 4
-// (all threads): Rayleigh damping and the new phi, written back coalesced.
-#ifndef AW_UNROLL
-#define AW_UNROLL 2
-#endif
+// Column block as in advance_mu_t, bound the same way: every operand of a
+// wave's LPT levels (1 + grp, 1 + grp + TG, ... up to k1) is loaded before the
+// first barrier and what the later phases need of it stays in registers (ten
+// values a level; the outputs may be the inputs' own arrays); level 0, whose w is the surface condition, belongs to one
+// wave.  Four LDS arrays are used in turn: wd holds the geopotential
+// advection wdwn, then the pressure term of each half level, then a; rhs the
+// phi right-hand side, then w; yp the buoyancy term c2a alt t_2ave of each half
+// level, then gamma; al alpha.  Each term is formed once and read by the two
+// levels that difference it.  One wave then runs the Thomas sweeps out of
+// LDS, and all waves apply the Rayleigh damping (its weights formed before the
+// first barrier) and store.
+template <int LPT>
 __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
   extern __shared__ float sm[];
-  __shared__ float s_fnm[CB_MAXNZ], s_fnp[CB_MAXNZ], s_rdnw[CB_MAXNZ], s_rdn[CB_MAXNZ];
   const int nz = D.nz, k1 = a.k1;
-  for (int t = threadIdx.x; t < nz; t += TB) {
-    s_fnm[t] = a.fnm[t]; s_fnp[t] = a.fnp[t]; s_rdnw[t] = a.rdnw[t]; s_rdn[t] = a.rdn[t];
-  }
-  float* s_t2a = sm;
+  float* s_wd = sm;
   float* s_rhs = sm + 1 * nz * TI;
-  float* s_w = sm + 2 * nz * TI;
-  float* s_a = sm + 3 * nz * TI;
-  float* s_al = sm + 4 * nz * TI;
-  float* s_ga = sm + 5 * nz * TI;
-  const int lane = threadIdx.x % TI, grp = threadIdx.x / TI;
+  float* s_yp = sm + 2 * nz * TI;
+  float* s_al = sm + 3 * nz * TI;
+  const int lane = threadIdx.x % TI, grp = wave_of_block();
   int bx, by;
 #if PW_COL_XCD
   xcd_block_2d(bx, by);
@@ -632,108 +636,149 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
 #endif
   const int j = by, i = bx * TI + lane;
   const bool vi = i < D.nx;
-  const bool h = vi && j >= a.j0 && j < a.j1 && i >= a.i0 && i < a.i1;
-  const long q2 = vi ? D.ix2(j, i) : 0;
+  const bool row = j >= a.j0 && j < a.j1 && a.i0 < a.i1;
+  const bool h = vi && row && i >= a.i0 && i < a.i1;
+  if (vi && !h) {
+    for (int k = grp; k < nz; k += TG) {
+      const long q = D.ix(k, j, i);
+      const float x = a.t_2ave_in[q], y = a.w_in[q], z = a.ph_in[q];
+      a.t_2ave[q] = x;
+      a.w[q] = y;
+      a.ph[q] = z;
+    }
+  }
+  if (!row) return;   // the whole block
+  const int ic = imin(imax(i, a.i0), a.i1 - 1);   // lanes outside the box load (and drop) its edge column's values
+  const long q2 = D.ix2(j, ic);
   const float G = F(pw::g);
-  float mut = 0.0f, muts = 0.0f, muave = 0.0f, my = 1.0f, mx = 1.0f;
-  if (h) {
-    mut = a.mut[q2]; muts = a.muts[q2]; muave = a.muave[q2]; my = a.msfty[q2]; mx = a.msftx[q2];
-  }
+  const float mut = a.mut[q2], muts = a.muts[q2], muave = a.muave[q2], my = a.msfty[q2], mx = a.msftx[q2];
   const float mi = 1.0f / my;
-  __syncthreads();   // level arrays staged
-  // phase 1 (operands loaded before the arithmetic, so one level's loads are in
-  // flight together; no global store in the loop, so the levels can overlap)
-#pragma unroll AW_UNROLL
-  for (int k = grp; k < nz; k += TG) {
-    if (!vi) continue;
-    long q = D.ix(k, j, i);
-    if (!h) {
-      a.t_2ave[q] = a.t_2ave_in[q];
-      a.w[q] = a.w_in[q];
-      a.ph[q] = a.ph_in[q];
-      continue;
+  auto theta_ave = [&](float t2i, float t2, float t1) -> float {
+    const float t = 0.5f * (a.ep1 * t2 + a.em1 * t2i);
+    return (t + muave * a.t0) / (muts * (a.t0 + t1));
+  };
+  const float htop = (AT(a.ph_1, k1, j, ic) + AT(a.phb, k1, j, ic)) / G;
+  const float hbot = htop - a.hdepth;
+  const int ktw = (k1 - 1) % TG, k0w = ktw == TG - 2 ? TG - 3 : TG - 2;   // the waves that own the top level and level 0
+  float r_a[LPT], r_ga[LPT], r_w[LPT], r_cq[LPT], r_cb[LPT], r_e[LPT], r_rhs[LPT], r_phi[LPT], r_hk[LPT];
+  float r_ws[LPT], r_t2a[LPT], t2a_sfc = 0.0f, z_a = 0.0f, z_e = 0.0f, z_b = 0.0f;
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = imin(1 + grp + m * TG, k1), kl = imin(k, k1 - 1);   // kl: the half level above k, where there is one
+    const float t2i = AT(a.t_2ave_in, k, j, ic), t2 = AT(a.t_2, kl, j, ic), t1 = AT(a.t_1, kl, j, ic);
+    const float pht = AT(a.ph_tend, k, j, ic), win = AT(a.w_in, k, j, ic);
+    const float phi = AT(a.ph_in, k, j, ic), php = AT(a.ph_in, kl + 1, j, ic);
+    const float ww0 = AT(a.ww, k, j, ic), wwm = AT(a.ww, k - 1, j, ic);
+    const float p10 = AT(a.ph_1, k, j, ic), p1m = AT(a.ph_1, k - 1, j, ic);
+    const float pb0 = AT(a.phb, k, j, ic), pbm = AT(a.phb, k - 1, j, ic);
+    const float c2 = AT(a.c2a, kl, j, ic), alt = AT(a.alt, kl, j, ic), cq = AT(a.cqw, kl, j, ic);
+    const float rwt = AT(a.rw_tend, k, j, ic);
+    r_ws[m] = AT(a.w_save, k, j, ic);
+    r_a[m] = AT(a.a, k, j, ic);
+    const float al = AT(a.alpha, k, j, ic);
+    r_ga[m] = AT(a.gamma, k, j, ic);
+    // wdwn(k) = 0.5 (ww[k] + ww[k-1]) rdnw[k-1] (ph_1[k] - ph_1[k-1] + phb[k] - phb[k-1])
+    const float wd = 0.5f * (ww0 + wwm) * a.rdnw[k - 1] * (p10 - p1m + pb0 - pbm);
+    const float t2a = k < k1 ? theta_ave(t2i, t2, t1) : t2i;
+    if (1 + grp + m * TG <= k1) {
+      s_wd[k * TI + lane] = wd;
+      s_yp[k * TI + lane] = c2 * alt * t2a;   // read below k1 only
+      s_al[k * TI + lane] = al;
     }
-    const bool lo = k < k1, rk = k >= 1 && k <= k1, wd = rk && k < k1;
-    const float t2i = a.t_2ave_in[q], t2 = lo ? a.t_2[q] : 0.0f, t1 = lo ? a.t_1[q] : 0.0f;
-    const float pht = rk ? a.ph_tend[q] : 0.0f, win = rk ? a.w_in[q] : 0.0f, phi = rk ? a.ph_in[q] : 0.0f;
-    const float ca = a.a[q], cal = a.alpha[q], cga = a.gamma[q];
-    float wwp = 0.0f, ww0 = 0.0f, wwm = 0.0f, p1p = 0.0f, p10 = 0.0f, p1m = 0.0f, pbp = 0.0f, pb0 = 0.0f, pbm = 0.0f;
-    if (wd) {
-      wwp = AT(a.ww, k + 1, j, i); ww0 = AT(a.ww, k, j, i); wwm = AT(a.ww, k - 1, j, i);
-      p1p = AT(a.ph_1, k + 1, j, i); p10 = AT(a.ph_1, k, j, i); p1m = AT(a.ph_1, k - 1, j, i);
-      pbp = AT(a.phb, k + 1, j, i); pb0 = AT(a.phb, k, j, i); pbm = AT(a.phb, k - 1, j, i);
-    }
-    float t = t2i;
-    if (lo) {
-      t = 0.5f * (a.ep1 * t2 + a.em1 * t);
-      t = (t + muave * a.t0) / (muts * (a.t0 + t1));
-    }
-    s_t2a[k * TI + lane] = t;
-    float r = 0.0f;
-    if (rk) {
-      r = a.dts * (pht + a.hgem1 * win);
-      if (wd) {
-        // wdwn(kk) = 0.5 (ww[kk] + ww[kk-1]) rdnw[kk-1] (ph_1[kk] - ph_1[kk-1] + phb[kk] - phb[kk-1])
-        const float wup = 0.5f * (wwp + ww0) * s_rdnw[k] * (p1p - p10 + pbp - pb0);
-        const float wdn = 0.5f * (ww0 + wwm) * s_rdnw[k - 1] * (p10 - p1m + pb0 - pbm);
-        r = r - a.dts * (s_fnm[k] * wup + s_fnp[k] * wdn);
-      }
-      r = phi + my * r / mut;
-    }
+    r_t2a[m] = t2a;
+    r_w[m] = win + a.dts * rwt;
+    r_cq[m] = mi * cq;
+    r_cb[m] = c2 * a.rdnw[kl] / mut;
+    r_e[m] = a.em1 * (php - phi);
+    r_rhs[m] = a.dts * (pht + a.hgem1 * win);
+    r_phi[m] = phi;
+    r_hk[m] = (p10 + pb0) / G;
+  }
+  if (grp == ktw) {
+    const float c2m = AT(a.c2a, k1 - 1, j, ic), alm = AT(a.alt, k1 - 1, j, ic);
+    const float ph0 = AT(a.ph_in, k1, j, ic), phm = AT(a.ph_in, k1 - 1, j, ic), rn = a.rdnw[k1 - 1];
+    const float t2a = theta_ave(AT(a.t_2ave_in, k1 - 1, j, ic), AT(a.t_2, k1 - 1, j, ic), AT(a.t_1, k1 - 1, j, ic));
+    z_a = a.mhdtsg / mut * (rn * rn) * 2.0f * c2m;
+    z_e = a.em1 * (ph0 - phm);
+    z_b = a.dtsg * (2.0f * rn * c2m * alm * t2a + muave);
+  }
+  float z_cb = 0.0f, w_sfc = 0.0f, ph_sfc = 0.0f;
+  if (grp == k0w) {
+    const float cf1 = a.cf[0], cf2 = a.cf[1], cf3 = a.cf[2];
+    auto V3 = [&](int jj, int ii) {
+      return cf1 * AT(a.v, 0, jj, ii) + cf2 * AT(a.v, 1, jj, ii) + cf3 * AT(a.v, 2, jj, ii);
+    };
+    auto U3 = [&](int jj, int ii) {
+      return cf1 * AT(a.u, 0, jj, ii) + cf2 * AT(a.u, 1, jj, ii) + cf3 * AT(a.u, 2, jj, ii);
+    };
+    const float c2 = AT(a.c2a, 0, j, ic), alt = AT(a.alt, 0, j, ic), php = AT(a.ph_in, 1, j, ic);
+    const float t2i = AT(a.t_2ave_in, 0, j, ic), t2 = AT(a.t_2, 0, j, ic), t1 = AT(a.t_1, 0, j, ic);
+    ph_sfc = AT(a.ph_in, 0, j, ic);
+    const float htc = AT2(a.ht, j, ic);
+    const float ty = (AT2(a.ht, j + 1, ic) - htc) * V3(j + 1, ic) + (htc - AT2(a.ht, j - 1, ic)) * V3(j, ic);
+    const float tx = (AT2(a.ht, j, ic + 1) - htc) * U3(j, ic + 1) + (htc - AT2(a.ht, j, ic - 1)) * U3(j, ic);
+    w_sfc = my * 0.5f * a.rdy * ty + mx * 0.5f * a.rdx * tx;
+    t2a_sfc = theta_ave(t2i, t2, t1);
+    s_yp[lane] = c2 * alt * t2a_sfc;
+    z_cb = c2 * a.rdnw[0] / mut;
+    z_e = a.em1 * (php - ph_sfc);
+    s_rhs[lane] = 0.0f;
+  }
+  __syncthreads();
+  // the phi right-hand side
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = 1 + grp + m * TG;
+    if (k > k1) continue;
+    float r = r_rhs[m];
+    if (k < k1) r = r - a.dts * (a.fnm[k] * s_wd[(k + 1) * TI + lane] + a.fnp[k] * s_wd[k * TI + lane]);
+    r = r_phi[m] + my * r / mut;
+    r_rhs[m] = r;
     s_rhs[k * TI + lane] = r;
-    s_a[k * TI + lane] = ca;
-    s_al[k * TI + lane] = cal;
-    s_ga[k * TI + lane] = cga;
   }
   __syncthreads();
-  auto RHS = [&](int k) -> float { return s_rhs[k * TI + lane]; };   // rhs[0] is 0
-  // phase 2
-#pragma unroll AW_UNROLL
-  for (int k = grp; k < nz; k += TG) {
-    if (!h) continue;
-    long q = D.ix(k, j, i);
-    float w;
-    if (k == 0) {
-      float cf1 = a.cf[0], cf2 = a.cf[1], cf3 = a.cf[2];
-      auto V3 = [&](int jj, int ii) {
-        return cf1 * AT(a.v, 0, jj, ii) + cf2 * AT(a.v, 1, jj, ii) + cf3 * AT(a.v, 2, jj, ii);
-      };
-      auto U3 = [&](int jj, int ii) {
-        return cf1 * AT(a.u, 0, jj, ii) + cf2 * AT(a.u, 1, jj, ii) + cf3 * AT(a.u, 2, jj, ii);
-      };
-      float htc = AT2(a.ht, j, i);
-      float ty = (AT2(a.ht, j + 1, i) - htc) * V3(j + 1, i) + (htc - AT2(a.ht, j - 1, i)) * V3(j, i);
-      float tx = (AT2(a.ht, j, i + 1) - htc) * U3(j, i + 1) + (htc - AT2(a.ht, j, i - 1)) * U3(j, i);
-      w = my * 0.5f * a.rdy * ty + mx * 0.5f * a.rdx * tx;
-    } else if (k < k1) {
-      const float c2 = a.c2a[q], c2m = AT(a.c2a, k - 1, j, i), al0 = a.alt[q], alm = AT(a.alt, k - 1, j, i);
-      const float win = a.w_in[q], rwt = a.rw_tend[q], cq = a.cqw[q];
-      const float php = AT(a.ph_in, k + 1, j, i), ph0 = a.ph_in[q], phm = AT(a.ph_in, k - 1, j, i);
-      float X = a.hdtsg * s_rdn[k] *
-                (c2 * s_rdnw[k] / mut * (a.ep1 * (RHS(k + 1) - RHS(k)) + a.em1 * (php - ph0)) -
-                 c2m * s_rdnw[k - 1] / mut * (a.ep1 * (RHS(k) - RHS(k - 1)) + a.em1 * (ph0 - phm)));
-      float Y = s_rdn[k] * (c2 * al0 * s_t2a[k * TI + lane] - c2m * alm * s_t2a[(k - 1) * TI + lane]) - muave;
-      w = win + a.dts * rwt + mi * cq * X + a.dtsg * mi * Y;
+  // the pressure term of each half level, and the top level's w
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = 1 + grp + m * TG;
+    if (k < k1) {
+      s_wd[k * TI + lane] = r_cb[m] * (a.ep1 * (s_rhs[(k + 1) * TI + lane] - r_rhs[m]) + r_e[m]);
     } else if (k == k1) {
-      const float c2m = AT(a.c2a, k1 - 1, j, i), alm = AT(a.alt, k1 - 1, j, i);
-      const float win = a.w_in[q], rwt = a.rw_tend[q];
-      const float ph0 = a.ph_in[q], phm = AT(a.ph_in, k1 - 1, j, i);
-      float rn = s_rdnw[k1 - 1];
-      float Z = a.mhdtsg / mut * (rn * rn) * 2.0f * c2m * (a.ep1 * (RHS(k1) - RHS(k1 - 1)) + a.em1 * (ph0 - phm)) -
-                a.dtsg * (2.0f * rn * c2m * alm * s_t2a[(k1 - 1) * TI + lane] + muave);
-      w = win + a.dts * rwt + mi * Z;
-    } else {
-      w = a.w_in[q];
+      r_w[m] = r_w[m] + mi * (z_a * (a.ep1 * (r_rhs[m] - s_rhs[(k1 - 1) * TI + lane]) + z_e) - z_b);
     }
-    s_w[k * TI + lane] = w;
+  }
+  if (grp == k0w) s_wd[lane] = z_cb * (a.ep1 * (s_rhs[TI + lane] - 0.0f) + z_e);
+  __syncthreads();
+  // the explicit w predictor
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = 1 + grp + m * TG;
+    if (k > k1) continue;
+    float w = r_w[m];
+    if (k < k1) {
+      const float X = a.hdtsg * a.rdn[k] * (s_wd[k * TI + lane] - s_wd[(k - 1) * TI + lane]);
+      const float Y = a.rdn[k] * (s_yp[k * TI + lane] - s_yp[(k - 1) * TI + lane]) - muave;
+      w = w + r_cq[m] * X + a.dtsg * mi * Y;
+    }
+    s_rhs[k * TI + lane] = w;
+  }
+  if (grp == k0w) s_rhs[lane] = w_sfc;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = 1 + grp + m * TG;
+    if (k > k1) continue;
+    s_wd[k * TI + lane] = r_a[m];
+    s_yp[k * TI + lane] = r_ga[m];
   }
   __syncthreads();
-  // phase 3
   // The sweeps take their operands 8 levels at a time into registers before
-  // the dependent arithmetic: s_w, s_a, s_al, s_ga are runtime offsets into
-  // one LDS buffer, so a read placed after a store to s_w would be made to
-  // wait for it.
-  if (grp == 0 && h) {
+  // the dependent arithmetic: the LDS arrays are runtime offsets into one
+  // buffer, so a read placed after a store to s_rhs would be made to wait for
+  // it.  The other waves form their damping weights meanwhile.
+  if (grp == 0) {
+    float* s_w = s_rhs;
+    const float *s_a = s_wd, *s_ga = s_yp;
     float wm = s_w[lane];
     int k = 1;
     for (; k + 7 <= k1; k += 8) {
@@ -769,36 +814,38 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
       s_w[k * TI + lane] = wp;
     }
   }
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    float dw = 0.0f;
+    if (r_hk[m] >= hbot) {
+      const float sn = sinf(a.hpi * (r_hk[m] - hbot) / a.hdepth);
+      dw = a.dampmag * (sn * sn);
+    }
+    r_ws[m] = dw * mut * r_ws[m];
+    r_hk[m] = 1.0f + dw;
+  }
   __syncthreads();
   if (!h) return;
-  // phase 4: the new w and phi of this thread's levels into LDS (s_w, s_rhs),
-  // then written out with t_2ave in a loop of stores only
-  float htop = (AT(a.ph_1, k1, j, i) + AT(a.phb, k1, j, i)) / G;
-  float hbot = htop - a.hdepth;
-#pragma unroll AW_UNROLL
-  for (int k = grp; k < nz; k += TG) {
-    long q = D.ix(k, j, i);
-    float w = s_w[k * TI + lane];
-    if (k == 0 || k > k1) {
-      s_rhs[k * TI + lane] = a.ph_in[q];
-    } else {
-      const float p1 = a.ph_1[q], pb = a.phb[q], ws = a.w_save[q];
-      float hk = (p1 + pb) / G;
-      float dw = 0.0f;
-      if (hk >= hbot) {
-        float sn = sinf(a.hpi * (hk - hbot) / a.hdepth);
-        dw = a.dampmag * (sn * sn);
-      }
-      w = (w - dw * mut * ws) / (1.0f + dw);
-      s_w[k * TI + lane] = w;
-      s_rhs[k * TI + lane] = s_rhs[k * TI + lane] + my * 0.5f * a.dts * G * a.ep1 * w / muts;
-    }
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int k = 1 + grp + m * TG;
+    if (k > k1) continue;
+    const float w = (s_rhs[k * TI + lane] - r_ws[m]) / r_hk[m];
+    AT(a.t_2ave, k, j, i) = r_t2a[m];
+    AT(a.w, k, j, i) = w;
+    AT(a.ph, k, j, i) = r_rhs[m] + my * 0.5f * a.dts * G * a.ep1 * w / muts;
   }
-  for (int k = grp; k < nz; k += TG) {
-    long q = D.ix(k, j, i);
-    a.w[q] = s_w[k * TI + lane];
-    a.ph[q] = s_rhs[k * TI + lane];
-    a.t_2ave[q] = s_t2a[k * TI + lane];
+  if (grp == k0w) {
+    AT(a.t_2ave, 0, j, i) = t2a_sfc;
+    AT(a.w, 0, j, i) = w_sfc;
+    AT(a.ph, 0, j, i) = ph_sfc;
+  }
+  for (int k = k1 + 1 + grp; k < nz; k += TG) {   // levels above k1 copy their inputs
+    const long q = D.ix(k, j, i);
+    const float x = a.t_2ave_in[q], y = a.w_in[q], z = a.ph_in[q];
+    a.t_2ave[q] = x;
+    a.w[q] = y;
+    a.ph[q] = z;
   }
 }
 
@@ -821,9 +868,11 @@ extern "C" int pywrf_advance_w(const pywrf_grid_t* g, const float* w_in, const f
             F(dts), F(t0), F(1. + epssm), F(1. - epssm), F(0.5 * G * (1. - epssm)), F(rdx), F(rdy),
             F(0.5 * dts * G), F(dts * G), F(-0.5 * dts * G), F(dts * 0.2), F(0.5 * pi_), F(5000.), g->kte - 1,
             imax(g->jts, g->jds + 1), imin(g->jte, g->jde - 2), imax(g->its, g->ids + 1), imin(g->ite, g->ide - 2)};
-  if (column_block_launch_check(g, 6)) return PYWRF_E_RANGE;
+  if (column_block_launch_check(g, 6)) return PYWRF_E_RANGE;   // the LDS of nz levels the entry point has always taken
   dim3 grid((g->nx + TI - 1) / TI, g->ny);
-  hipLaunchKernelGGL(k_advance_w, grid, dim3(TB), 6 * g->nz * TI * sizeof(float), (hipStream_t)s, dims_of(g), p);
+  auto kern = k_advance_w<5>;   // nz <= 42 (column_block_launch_check), so 5 levels a wave hold levels 1 .. 40
+  if (p.k1 > 5 * TG) kern = k_advance_w<6>;
+  hipLaunchKernelGGL(kern, grid, dim3(TB), 4 * g->nz * TI * sizeof(float), (hipStream_t)s, dims_of(g), p);
   PW_RET();
 }
 
