@@ -358,36 +358,7 @@ struct AdvS {
   float rdx, rdy;
 };
 
-__device__ inline float s_yface(const Dims& D, const AdvS& a, const AdvIdx& x, int k, int jf, int i) {
-  auto Q = [&](int o) { return AT(a.f, k, jf + o, i); };
-  float vel = AT(a.rv, k, jf, i);
-  if (jf >= x.jds + 3 && jf < x.jde - 3) return vel * flux5(Q(-3), Q(-2), Q(-1), Q(0), Q(1), Q(2), vel);
-  if (jf == x.jds + 1 || jf == x.jde - 2) return 0.5f * vel * (Q(0) + Q(-1));
-  if (jf == x.jds + 2 || jf == x.jde - 3) return vel * flux3(Q(-2), Q(-1), Q(0), Q(1), vel);
-  return 0.0f;
-}
-
-__device__ inline float s_xface(const Dims& D, const AdvS& a, const AdvIdx& x, int k, int j, int f) {
-  auto Q = [&](int o) { return AT(a.f, k, j, f + o); };
-  float vel = AT(a.ru, k, j, f);
-  if (f >= x.ids + 3 && f < x.ide - 3) return vel * flux5(Q(-3), Q(-2), Q(-1), Q(0), Q(1), Q(2), vel);
-  if (f == x.ids + 1 || f == x.ide - 2) return 0.5f * vel * (Q(0) + Q(-1));
-  if (f == x.ids + 2) return vel * flux3(Q(-2), Q(-1), Q(0), Q(1), vel);
-  if (f == x.ide - 3) return vel * flux3(Q(-2), Q(-1), Q(0), Q(1), AT(a.ru, k, j, f + 1));  // sign from ru[ide-2]
-  return 0.0f;
-}
-
-__device__ inline float s_zface(const Dims& D, const AdvS& a, const AdvIdx& x, int kf, int j, int i) {
-  auto Q = [&](int o) { return AT(a.f, kf + o, j, i); };
-  if (kf < 1 || kf >= x.ktf) return 0.0f;
-  float vel = AT(a.rom, kf, j, i);
-  if (kf >= 3 && kf < x.ktf - 2) return vel * flux5(Q(-3), Q(-2), Q(-1), Q(0), Q(1), Q(2), -vel);
-  if (kf == 1 || kf == x.ktf - 1) return vel * (a.fzm[kf] * Q(0) + a.fzp[kf] * Q(-1));
-  return vel * flux3(Q(-2), Q(-1), Q(0), Q(1), -vel);  // kf == 2 or ktf-2
-}
-
-
-// The same faces from operand values: Q[0..5] are the field at offsets -3..2
+// The scalar faces from operand values: Q[0..5] are the field at offsets -3..2
 // from the face (rows for y, levels for z), vel the face velocity.
 __device__ inline float s_yface_v(const AdvIdx& x, int jf, float vel, const float* Q) {
   if (jf >= x.jds + 3 && jf < x.jde - 3) return vel * flux5(Q[0], Q[1], Q[2], Q[3], Q[4], Q[5], vel);
@@ -426,125 +397,146 @@ struct ScalarTend {
   float *adv_tend, *sc_tend, *h_t, *z_t;
   long n3;
   int scs, sce, rk1, moist_step, accumulate;
-  Box bzero, badv, by, bx, bh, bv, span;
-  // a second species array over the same fluxes and index set (scalar2 null:
-  // none); species groups [0, nsg1) are the first array's, the rest the second's
+  Box bzero, badv, by, bx, bh, bv;
+  // a second species array over the same fluxes and index set (scalar2 null: none)
   const float* scalar2;
   float *adv_tend2, *sc_tend2;
-  int scs2, sce2, moist_step2, nsg1;
+  int scs2, sce2, moist_step2;
 };
 
-// Tile of 63 i x 4 j points per workgroup (lane l of a row evaluates the x-face
-// at i0 + l; the point takes its right-hand face from lane l + 1 by a lane
-// shuffle), marching SA_KC levels up the column and carrying each z-face to
-// the level above.  Face values and the tendency arithmetic are those of the
-// one-thread-per-point form (s_yface, s_xface, s_zface in the reference's
-// y, x, z order), so the results are the same floats; each x- and z-face is
-// evaluated about once instead of by both neighbours.
-#define SA_OX 63
-#ifndef SA_KC
-#define SA_KC 8
-#endif
-#ifndef SA_SPW
-#define SA_SPW 1   // species per wave
-#endif
-__global__ void __launch_bounds__(PW_TX * PW_TY) k_scalar_adv(Dims D, ScalarTend a) {
-  const Box& b = a.bzero;   // points that receive a tendency
-  const Box& sp = a.span;   // launch region: b, or the whole array when h_t / z_t are zeroed as well
-  const int i = sp.i0 + (int)(blockIdx.x * SA_OX + threadIdx.x);
-  const int j = sp.j0 + (int)(blockIdx.y * PW_TY + threadIdx.y);
-  if (j >= sp.j1) return;                     // a whole wave (one row) leaves together
-  const int nkc = (sp.nk() + SA_KC - 1) / SA_KC;
-  const int kc = (int)blockIdx.z % nkc, sg = (int)blockIdx.z / nkc;   // level chunk, species group
-  const int k0 = sp.k0 + kc * SA_KC, k1 = imin(k0 + SA_KC, sp.k1);
-  const bool second = sg >= a.nsg1;                                   // the second species array
-  const int scs = second ? a.scs2 : a.scs, sce = second ? a.sce2 : a.sce;
-  const int ms = scs + (second ? sg - a.nsg1 : sg) * SA_SPW, me = imin(sce, ms + SA_SPW - 1);
-  const float* const sbase = second ? a.scalar2 : a.scalar;
-  float* const tbase = second ? a.adv_tend2 : a.adv_tend;
-  const bool mine = threadIdx.x < SA_OX && i < sp.i1;
-  if (a.h_t && mine && sg == 0)
-    for (int k = k0; k < k1; ++k) {
+// One wave owns SA_OX consecutive columns of R consecutive rows (lane l holds
+// column i0 - 3 + l, three halo columns on the left and three on the right)
+// and marches SA_KC levels.  A level's values of its own rows are in the
+// registers that slide up the columns for the vertical faces, so the level
+// loads only the six halo rows, the R new top values and the mass fluxes; the
+// x-stencil comes from the neighbouring lanes by DPP shifts; the R + 1 y-faces
+// serve the R rows; each x- and z-face is evaluated once.  j and k are the
+// same in a whole wave, so which rule a y- or z-face follows is decided in
+// scalar registers.  The arithmetic and its order are those of the reference.
+//
+// What bounds it is VALU work (a 5th-order face is 26 operations): 2 + (R+1)/R
+// faces a point with R rows against 4 with one row a wave.  Eight species at
+// 240x240x41: 128 -> 102 us a launch, theta 21.5 -> 20.4 us; the six launches of a step at 40x40x41 15.1 -> 8.8 us each.
+#define SA_OX 58
+#define SA_KC 8   // levels a wave (14 and 21: 0.4-0.8 % of a step slower)
+
+// The part of the launch that zeroes: h_tendency and z_tendency everywhere, and
+// the points of a fresh tendency outside the advection box.  One level a
+// block slab, the slab's blocks striding over its rows and columns.
+__device__ inline void scalar_adv_fill(const Dims& D, const ScalarTend& a, int k) {
+  const int nsp1 = a.sce - a.scs + 1, nsp = nsp1 + (a.scalar2 ? a.sce2 - a.scs2 + 1 : 0);
+  for (int j = (int)(blockIdx.y * PW_TY + threadIdx.y); j < D.ny; j += (int)gridDim.y * PW_TY)
+    for (int i = (int)(blockIdx.x * PW_TX + threadIdx.x); i < D.nx; i += (int)gridDim.x * PW_TX) {
       const int q = D.ix(k, j, i);
-      a.h_t[q] = 0.0f;
-      a.z_t[q] = 0.0f;
-    }
-  if (j < b.j0 || j >= b.j1) return;          // whole wave: no tendency points in this row
-  const bool live = i < D.nx;                 // may evaluate faces
-  const bool own = mine && i >= b.i0 && i < b.i1;
-  const float mx = (own && a.badv.has2(j, i)) ? AT2(a.adv.msftx, j, i) : 0.0f;
-#pragma unroll 1
-  for (int im = ms; im <= me; ++im) {
-    AdvS ad = a.adv;
-    ad.f = sbase + im * a.n3;
-    // the column's values at levels kf-3 .. kf+2 around the current z-face kf,
-    // slid up one level per step (one new load per level); levels outside the
-    // array are never used by the face formulas and are not loaded
-    // (indices clamped into the array so that every load is unconditional; the
-    // clamped values are never used)
-    const int ic = imin(i, D.nx - 1);
-    auto ZQ = [&](int kk) { return AT(ad.f, imin(imax(kk, 0), D.nz - 1), j, ic); };
-    float wz[6];
-#pragma unroll
-    for (int o = 0; o < 6; ++o) wz[o] = ZQ(k0 - 3 + o);
-    float zlo = live ? s_zface_v(ad, a.x, k0, AT(ad.rom, imin(imax(k0, 0), D.nz - 1), j, ic), wz) : 0.0f;
-    // every operand of a level is loaded before its arithmetic and outside
-    // the branches (indices clamped into the array; values at clamped indices
-    // are never used), so that a level waits on memory once
-    const int jn = imin(j + 1, D.ny - 1);
-    int xi[6], yj[7];
-#pragma unroll
-    for (int o = 0; o < 6; ++o) xi[o] = imin(imax(ic - 3 + o, 0), D.nx - 1);
-#pragma unroll
-    for (int o = 0; o < 7; ++o) yj[o] = imin(imax(j - 3 + o, 0), D.ny - 1);
-    const int ic1 = imin(ic + 1, D.nx - 1);
-#pragma unroll 1
-    for (int k = k0; k < k1; ++k) {
-      float xq[6], r[7];
-#pragma unroll
-      for (int o = 0; o < 6; ++o) xq[o] = AT(ad.f, k, j, xi[o]);
-#pragma unroll
-      for (int o = 0; o < 7; ++o) r[o] = AT(ad.f, k, yj[o], ic);
-      const float xvel = AT(ad.ru, k, j, ic), xvel1 = AT(ad.ru, k, j, ic1);
-      const float rvl = AT(ad.rv, k, j, ic), rvh = AT(ad.rv, k, jn, ic);
-      const int kf = k + 1;
-      const float romv = AT(ad.rom, imin(kf, D.nz - 1), j, ic);
-      const float wnew = ZQ(k + 3);
-      const float told = a.accumulate ? tbase[im * a.n3 + D.ix(k, j, ic)] : 0.0f;
-      const float rdz = k < b.k1 ? ad.rdzw[k] : 0.0f;
-      const float xf = live ? s_xface_v(a.x, i, xvel, xvel1, xq) : 0.0f;
-      const float xr = __shfl_down(xf, 1, PW_TX);
-#pragma unroll
-      for (int o = 0; o < 5; ++o) wz[o] = wz[o + 1];
-      wz[5] = wnew;
-      const float zhi = live ? s_zface_v(ad, a.x, kf, romv, wz) : 0.0f;
-      if (own && k >= b.k0 && k < b.k1) {
-        const int q = im * a.n3 + D.ix(k, j, i);
-        float t = told;
-        if (a.badv.has(k, j, i)) {
-          if (a.by.has(k, j, i)) {
-            // rows j-3 .. j+3 serve the faces at j (rows j-3 .. j+2) and j+1 (rows j-2 .. j+3)
-            const float yhi = s_yface_v(a.x, j + 1, rvh, r + 1);
-            const float ylo = s_yface_v(a.x, j, rvl, r);
-            t = t - (mx * ad.rdy) * (yhi - ylo);
-          }
-          if (a.bx.has(k, j, i)) t = t - (mx * ad.rdx) * (xr - xf);
-          t = t - rdz * (zhi - zlo);
-        }
-        tbase[q] = t;
+      if (a.h_t) {
+        a.h_t[q] = 0.0f;
+        a.z_t[q] = 0.0f;
       }
-      zlo = zhi;
+      if (!a.accumulate && a.bzero.has(k, j, i) && !a.badv.has(k, j, i))
+        for (int s = 0; s < nsp; ++s) {
+          if (s < nsp1) a.adv_tend[(a.scs + s) * (int)a.n3 + q] = 0.0f;
+          else a.adv_tend2[(a.scs2 + s - nsp1) * (int)a.n3 + q] = 0.0f;
+        }
+    }
+}
+
+template <int R>
+__global__ void __launch_bounds__(PW_TX * PW_TY) k_scalar_adv(Dims D, ScalarTend a, int kc_len, int nkc, int nadv) {
+  if ((int)blockIdx.z >= nadv) {
+    scalar_adv_fill(D, a, (int)blockIdx.z - nadv);
+    return;
+  }
+  const Box& b = a.badv;
+  const int kc = (int)blockIdx.z % nkc, sg = (int)blockIdx.z / nkc;   // level chunk, species
+  const int k0 = b.k0 + kc * kc_len, k1 = imin(k0 + kc_len, b.k1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+  const int j0 = b.j0 + ((int)blockIdx.y * PW_TY + wave) * R;
+  if (j0 >= b.j1) return;
+  const int nsp1 = a.sce - a.scs + 1;
+  const bool second = sg >= nsp1;                                     // the second species array
+  const int im = second ? a.scs2 + sg - nsp1 : a.scs + sg;
+  AdvS ad = a.adv;
+  ad.f = (second ? a.scalar2 : a.scalar) + im * a.n3;
+  float* const tend = (second ? a.adv_tend2 : a.adv_tend) + im * a.n3;
+  const int lane = (int)threadIdx.x, i = b.i0 + (int)blockIdx.x * SA_OX - 3 + lane;
+  // indices are clamped into the array so that every load is unconditional;
+  // the values taken at clamped indices are never used by a face that counts
+  const int ic = imin(imax(i, 0), D.nx - 1);
+  const bool own = lane >= 3 && lane < 3 + SA_OX && i < b.i1;
+  const bool inx = i >= a.bx.i0 && i < a.bx.i1;
+  int jr[R + 6];   // the rows j0 - 3 .. j0 + R + 2
+#pragma unroll
+  for (int o = 0; o < R + 6; ++o) jr[o] = imin(imax(j0 - 3 + o, 0), D.ny - 1);
+  float wz[R][6], zlo[R], mx[R];   // wz: levels k-3 .. k+2 of each row, around the z-face k
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int o = 0; o < 6; ++o) wz[r][o] = AT(ad.f, imin(imax(k0 - 3 + o, 0), D.nz - 1), jr[r + 3], ic);
+    mx[r] = AT2(ad.msftx, jr[r + 3], ic);
+    zlo[r] = s_zface_v(ad, a.x, k0, AT(ad.rom, k0, jr[r + 3], ic), wz[r]);
+  }
+#pragma unroll 1
+  for (int k = k0; k < k1; ++k) {
+    const int kn = imin(k + 1, D.nz - 1), k3 = imin(k + 3, D.nz - 1);
+    float q[R + 6], wnew[R], xv[R], yv[R + 1], zv[R], told[R];
+#pragma unroll
+    for (int o = 0; o < R + 6; ++o) q[o] = o >= 3 && o < R + 3 ? wz[o - 3][3] : AT(ad.f, k, jr[o], ic);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      wnew[r] = AT(ad.f, k3, jr[r + 3], ic);
+      xv[r] = AT(ad.ru, k, jr[r + 3], ic);
+      zv[r] = AT(ad.rom, kn, jr[r + 3], ic);
+      told[r] = a.accumulate ? AT(tend, k, jr[r + 3], ic) : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r <= R; ++r) yv[r] = AT(ad.rv, k, jr[r + 3], ic);
+    const float rdz = ad.rdzw[k];
+    float ylo = s_yface_v(a.x, j0, yv[0], q);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int j = j0 + r;
+      float x[6];
+      x[3] = q[r + 3];
+      x[2] = lane_below(x[3]); x[1] = lane_below(x[2]); x[0] = lane_below(x[1]);
+      x[4] = lane_above(x[3]); x[5] = lane_above(x[4]);
+      const float xf = s_xface_v(a.x, i, xv[r], lane_above(xv[r]), x);
+      const float xr = lane_above(xf);
+      const float yhi = s_yface_v(a.x, j + 1, yv[r + 1], q + r + 1);
+#pragma unroll
+      for (int o = 0; o < 5; ++o) wz[r][o] = wz[r][o + 1];
+      wz[r][5] = wnew[r];
+      const float zhi = s_zface_v(ad, a.x, k + 1, zv[r], wz[r]);
+      float t = told[r];
+      if (j >= a.by.j0 && j < a.by.j1) t = t - (mx[r] * ad.rdy) * (yhi - ylo);
+      if (inx) t = t - (mx[r] * ad.rdx) * (xr - xf);
+      t = t - rdz * (zhi - zlo[r]);
+      if (own && j < b.j1) AT(tend, k, j, i) = t;
+      ylo = yhi;
+      zlo[r] = zhi;
     }
   }
 }
 
 static void pw_launch_scalar_adv(const pywrf_grid_t* g, const ScalarTend& a, pywrf_stream_t s) {
-  const Box& sp = a.span;
-  if (sp.size() <= 0) return;
-  dim3 grid((unsigned)((sp.ni() + SA_OX - 1) / SA_OX), (unsigned)((sp.nj() + PW_TY - 1) / PW_TY),
-            (unsigned)((sp.nk() + SA_KC - 1) / SA_KC *
-                       (a.nsg1 + (a.scalar2 ? (a.sce2 - a.scs2 + SA_SPW) / SA_SPW : 0))));
-  hipLaunchKernelGGL(k_scalar_adv, grid, dim3(PW_TX, PW_TY), 0, (hipStream_t)s, dims_of(g), a);
+  const Box& b = a.badv;
+  const int nsp = (a.sce - a.scs + 1) + (a.scalar2 ? a.sce2 - a.scs2 + 1 : 0);
+  const bool any = b.size() > 0, fill = a.h_t || a.bzero.size() > imax(0, (int)b.size());
+  if (!any && !fill) return;
+  // Rows a wave: more rows share more y-faces but make fewer, longer waves, so
+  // four need eight waves for each of the 1024 SIMDs and two need four (eight
+  // species at 240x240x41: 4 rows 28 us a step faster than 2, 12 than 1; six at
+  // 203x237x41: 2 rows 62 us a launch, 4 rows 67, 1 row 69); below that one row,
+  // and half as many levels a wave (a step at 40x40x41: 925 -> 899 us).
+  auto waves = [&](int R, int kc) {
+    return (long)((b.ni() + SA_OX - 1) / SA_OX) * ((b.nj() + R - 1) / R) * ((b.nk() + kc - 1) / kc) * nsp;
+  };
+  const int R = waves(4, SA_KC) >= 1024L * 8 ? 4 : waves(2, SA_KC) >= 1024L * 4 ? 2 : 1;
+  const int kc_len = R == 1 ? SA_KC / 2 : SA_KC;
+  const int nkc = any ? (b.nk() + kc_len - 1) / kc_len : 1, nadv = any ? nkc * nsp : 0;
+  auto kern = R == 1 ? k_scalar_adv<1> : R == 2 ? k_scalar_adv<2> : k_scalar_adv<4>;
+  dim3 grid((unsigned)imax(1, (b.ni() + SA_OX - 1) / SA_OX), (unsigned)imax(1, (b.nj() + R * PW_TY - 1) / (R * PW_TY)),
+            (unsigned)(nadv + (fill ? g->nz : 0)));
+  hipLaunchKernelGGL(kern, grid, dim3(PW_TX, PW_TY), 0, (hipStream_t)s, dims_of(g), a, kc_len, nkc, nadv);
 }
 
 // zero_box 1: first zero the tendency on [kts, kte) x [jts, jte) x [its, ite)
@@ -566,10 +558,8 @@ int pw_advect_scalar_box(const pywrf_grid_t* g, const float* field, float* tende
   t.adv = a; t.x = x;
   t.scalar = field; t.adv_tend = tendency; t.n3 = 0; t.scs = 0; t.sce = 0; t.accumulate = zero_box ? 0 : 1;
   t.scalar2 = nullptr; t.adv_tend2 = t.sc_tend2 = nullptr; t.scs2 = 0; t.sce2 = -1; t.moist_step2 = 0;
-  t.nsg1 = 1;
   t.bzero = zero_box == 2 ? whole(g) : zero_box ? mkbox(g->kts, g->kte, g->jts, g->jte, g->its, g->ite) : badv;
   t.badv = badv; t.by = by; t.bx = bx;
-  t.span = t.bzero;
   t.h_t = nullptr;
   t.z_t = nullptr;
   pw_launch_scalar_adv(g, t, s);
@@ -704,7 +694,6 @@ int pw_rk_scalar_tend_fused(const pywrf_grid_t* g, int scs, int sce, int rk_step
   a.n3 = (long)g->nz * g->ny * g->nx;
   if ((long)(sce + 1) * a.n3 >= (1L << 31)) return PYWRF_E_RANGE;   // species offsets are 32-bit
   a.scs = scs; a.sce = sce; a.rk1 = rk_step == 1; a.moist_step = moist_step; a.accumulate = 0;
-  a.nsg1 = (sce - scs + SA_SPW) / SA_SPW;
   a.scalar2 = scalar2; a.sc_tend2 = scalar_tends2; a.adv_tend2 = advect_tend2;
   a.scs2 = scs2; a.sce2 = sce2; a.moist_step2 = moist_step2;
   if (scalar2 && (scs2 < 0 || sce2 < scs2 || (long)(sce2 + 1) * a.n3 >= (1L << 31) || !scalar_tends2 ||
@@ -718,7 +707,6 @@ int pw_rk_scalar_tend_fused(const pywrf_grid_t* g, int scs, int sce, int rk_step
   a.bh = mkbox(g->kts, ktf, imax(g->jds + 1, g->jts), imin(g->jde - 2, g->jte), imax(g->ids + 1, g->its),
                imin(g->ide - 2, g->ite));
   a.bv = mkbox(g->kts + 1, ktf, g->jts, jtf, g->its, itf);
-  a.span = mkbox(0, g->nz, 0, g->ny, 0, g->nx);   // h_tendency and z_tendency are zeroed everywhere
   pw_launch_scalar_adv(g, a, s);
   if (a.rk1 && a.bzero.size() > 0) {
     const Box& bz = a.bzero;

@@ -136,34 +136,50 @@ __device__ inline float sgn1(float x) { return x >= 0.0f ? 1.0f : -1.0f; }
 // The divisions by 60 and 12 give the correctly rounded quotient x / d of an
 // IEEE division, computed as a product by r = RN(1/d) and one fma correction
 // (Markstein's correction step): q = RN(x r), e = x - q d (exact in an fma),
-// RN(q + e r).  An exhaustive run over every float (the float_div_const check
+// RN(q + e r).  An exhaustive run over every float (the float_div_value check
 // of the test suite) shows that for d = 60 and d = 12 this equals RN(x / d)
-// bit for bit whenever |x| is finite and at least 2^-124, and for +-0 once the
-// sign of x is copied onto it.  Inputs outside that range (subnormal x,
-// infinities) and results that are subnormal or NaN take the true division,
-// so the function equals x / d for every input.  It costs 4 VALU operations
-// where the division sequence costs 11, one of them a quarter-rate rcp.
+// unless it comes out NaN or subnormal (only a zero's sign may differ, which
+// the sums below drop); those results, which include every infinite x, are
+// taken from the true division, once for the two quotients of a face.  A face
+// costs 3 VALU operations and a class test per quotient where the division
+// sequence costs 11, one of them a quarter-rate rcp.  The upwind sign is taken
+// after the quotient (the quotient is odd in x): 26 operations a 5th-order face
+// where testing x as well and multiplying by the sign took 32 (the advection
+// kernels are VALU-bound).
 template <int D>
-__device__ inline float div_const(float x) {
+__device__ inline void div_const2(float x0, float x1, float& y0, float& y1) {
   constexpr float d = (float)D;
   constexpr float r = 1.0f / d;
-  float q = x * r;
-  float e = __builtin_fmaf(-q, d, x);
-  float y = __builtin_copysignf(__builtin_fmaf(e, r, q), x);
-  // fpclass bits: 1|2 NaN, 4|512 infinity, 16|128 subnormal
-  if (__builtin_expect(__builtin_isfpclass(x, 4 | 16 | 128 | 512) | __builtin_isfpclass(y, 1 | 2 | 16 | 128), 0))
-    y = x / d;
-  return y;
+  const float q0 = x0 * r, q1 = x1 * r;
+  y0 = __builtin_fmaf(__builtin_fmaf(-q0, d, x0), r, q0);
+  y1 = __builtin_fmaf(__builtin_fmaf(-q1, d, x1), r, q1);
+  // fpclass bits: 1|2 NaN, 16|128 subnormal
+  if (__builtin_expect(__builtin_isfpclass(y0, 1 | 2 | 16 | 128) | __builtin_isfpclass(y1, 1 | 2 | 16 | 128), 0)) {
+    y0 = x0 / d;
+    y1 = x1 / d;
+  }
 }
 __device__ inline float flux5(float qm3, float qm2, float qm1, float q0, float qp1, float qp2, float ua) {
-  float f6 = div_const<60>(37.0f * (q0 + qm1) - 8.0f * (qp1 + qm2) + (qp2 + qm3));
-  float d = (qp2 - qm3) - 5.0f * (qp1 - qm2) + 10.0f * (q0 - qm1);
-  return f6 - div_const<60>(sgn1(ua) * d);
+  float f6, q;
+  div_const2<60>(37.0f * (q0 + qm1) - 8.0f * (qp1 + qm2) + (qp2 + qm3),
+                 (qp2 - qm3) - 5.0f * (qp1 - qm2) + 10.0f * (q0 - qm1), f6, q);
+  return f6 - (ua >= 0.0f ? q : -q);
 }
 __device__ inline float flux3(float qm2, float qm1, float q0, float qp1, float ua) {
-  float f4 = div_const<12>(7.0f * (q0 + qm1) - (qp1 + qm2));
-  float d = (qp1 - qm2) - 3.0f * (q0 - qm1);
-  return f4 + div_const<12>(sgn1(ua) * d);
+  float f4, q;
+  div_const2<12>(7.0f * (q0 + qm1) - (qp1 + qm2), (qp1 - qm2) - 3.0f * (q0 - qm1), f4, q);
+  return f4 + (ua >= 0.0f ? q : -q);
+}
+
+// The value of the next lower / higher lane of the wave (DPP wave shifts, one
+// VALU operation; the end lane keeps its own).  All 64 lanes must be active.
+__device__ __forceinline__ float lane_below(float x) {
+  const int v = __builtin_bit_cast(int, x);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false));   // wave_shr:1
+}
+__device__ __forceinline__ float lane_above(float x) {
+  const int v = __builtin_bit_cast(int, x);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false));   // wave_shl:1
 }
 
 // Offsets are 32-bit: every entry point rejects arrays of 2^30 or more points
