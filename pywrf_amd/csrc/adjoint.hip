@@ -1,12 +1,7 @@
 // Adjoints (transposes) of linear parts of the step, for gradients through it.
 //
-// * advect_scalar (wrf_dynamics.py:1841-2028): with the mass fluxes fixed the
-//   tendency is linear in the field, T = A q, the face value of each face
-//   being vel * sum_o c_o(face, sign) q(face + o).  k_advect_scalar_adj forms
-//   A^T lam by gathering, for every point, the faces whose stencils hold it
-//   (six in each direction), each face's sensitivity being formed from the
-//   adjoint tendencies of the two points it separates.  No atomics; every
-//   output point is written by one thread.
+// (the advection tendencies' are in adv_adj.hip)
+//
 // * rk_update_scalar (wrf_dynamics.py:4055-4119): pointwise.
 // * The column tridiagonal solve of advance_w (wrf_dynamics.py:3758-3765):
 //   forward elimination w[k] = (w[k] - a[k] w[k-1]) alpha[k], k = 1..K, then
@@ -21,135 +16,6 @@
 
 int pw_check_grid(const pywrf_grid_t* g, int r);
 #define CHECK(g, r) do { int _e = pw_check_grid((g), (r)); if (_e) return _e; } while (0)
-
-// ------------------------------------------------------------------ advect_scalar^T
-struct AdjS {
-  const float *lam, *ru, *rv, *rom, *msftx, *fzm, *fzp, *rdzw;
-  float* out;
-  float rdx, rdy;
-  int ids, ide, jds, jde, ktf, accumulate;
-  Box badv, by, bx;   // the forward's boxes: all terms, the y-term, the x-term
-};
-
-// d(face value) / d(q at face + o), o = -3..2, without the velocity factor:
-// the 5th-order face (flux5) with upwind sign s = +-1.
-__device__ inline float c5(int o, float s) {
-  switch (o) {
-    case -3: return (1.0f + s) / 60.0f;
-    case -2: return (-8.0f - 5.0f * s) / 60.0f;
-    case -1: return (37.0f + 10.0f * s) / 60.0f;
-    case 0: return (37.0f - 10.0f * s) / 60.0f;
-    case 1: return (-8.0f + 5.0f * s) / 60.0f;
-    case 2: return (1.0f - s) / 60.0f;
-  }
-  return 0.0f;
-}
-// the 3rd-order face (flux3), o = -2..1
-__device__ inline float c3(int o, float s) {
-  switch (o) {
-    case -2: return (-1.0f - s) / 12.0f;
-    case -1: return (7.0f + 3.0f * s) / 12.0f;
-    case 0: return (7.0f - 3.0f * s) / 12.0f;
-    case 1: return (-1.0f + s) / 12.0f;
-  }
-  return 0.0f;
-}
-
-// Coefficient of q(face + o) in the value of the horizontal face f of a row
-// or column whose domain is [d0, d1) (y: jds, jde; x: ids, ide): the
-// reference's face rules (5th order inside, 2nd order next to the edge, 3rd
-// order one further in; zero flux elsewhere).  s_lo / s_hi: the upwind signs
-// the 3rd-order faces at d0 + 2 and d1 - 3 use.
-__device__ inline float hface_coef(int f, int o, int d0, int d1, float s, float s_lo, float s_hi) {
-  if (f >= d0 + 3 && f < d1 - 3) return c5(o, s);
-  if (f == d0 + 1 || f == d1 - 2) return (o == 0 || o == -1) ? 0.5f : 0.0f;
-  if (f == d0 + 2) return c3(o, s_lo);
-  if (f == d1 - 3) return c3(o, s_hi);
-  return 0.0f;
-}
-
-__global__ void k_advect_scalar_adj(Box all, Dims D, AdjS a) {
-  int k, j, i;
-  if (!box_point(all, k, j, i)) return;
-  float acc = 0.0f;
-  // y-faces jf = j - o hold q(k, j, i) at offset o
-  if (k >= a.badv.k0 && k < a.badv.k1 && i >= a.badv.i0 && i < a.badv.i1) {
-#pragma unroll
-    for (int o = -3; o <= 2; ++o) {
-      const int jf = j - o;
-      if (jf < 1 || jf >= D.ny) continue;
-      // sensitivity of the face value: the points jf (face on its low side)
-      // and jf - 1 (face on its high side) that take the y-term
-      float gF = 0.0f;
-      if (a.by.has(k, jf, i)) gF += (AT2(a.msftx, jf, i) * a.rdy) * AT(a.lam, k, jf, i);
-      if (a.by.has(k, jf - 1, i)) gF -= (AT2(a.msftx, jf - 1, i) * a.rdy) * AT(a.lam, k, jf - 1, i);
-      if (gF == 0.0f) continue;
-      const float vel = AT(a.rv, k, jf, i);
-      const float s = sgn1(vel);
-      acc += gF * vel * hface_coef(jf, o, a.jds, a.jde, s, s, s);
-    }
-  }
-  // x-faces f = i - o
-  if (k >= a.badv.k0 && k < a.badv.k1 && j >= a.badv.j0 && j < a.badv.j1) {
-#pragma unroll
-    for (int o = -3; o <= 2; ++o) {
-      const int f = i - o;
-      if (f < 1 || f >= D.nx) continue;
-      float gF = 0.0f;
-      if (a.bx.has(k, j, f)) gF += (AT2(a.msftx, j, f) * a.rdx) * AT(a.lam, k, j, f);
-      if (a.bx.has(k, j, f - 1)) gF -= (AT2(a.msftx, j, f - 1) * a.rdx) * AT(a.lam, k, j, f - 1);
-      if (gF == 0.0f) continue;
-      const float vel = AT(a.ru, k, j, f);
-      const float s = sgn1(vel);
-      // the face at ide - 3 takes its upwind sign from ru at ide - 2
-      const float s_hi = (f == a.ide - 3 && f + 1 < D.nx) ? sgn1(AT(a.ru, k, j, f + 1)) : s;
-      acc += gF * vel * hface_coef(f, o, a.ids, a.ide, s, s, s_hi);
-    }
-  }
-  // z-faces kf = k - o (upwind sign from -rom)
-  if (j >= a.badv.j0 && j < a.badv.j1 && i >= a.badv.i0 && i < a.badv.i1) {
-#pragma unroll
-    for (int o = -3; o <= 2; ++o) {
-      const int kf = k - o;
-      if (kf < 1 || kf >= a.ktf || kf >= D.nz) continue;
-      float gF = 0.0f;
-      if (kf < a.badv.k1) gF += a.rdzw[kf] * AT(a.lam, kf, j, i);
-      if (kf - 1 >= a.badv.k0) gF -= a.rdzw[kf - 1] * AT(a.lam, kf - 1, j, i);
-      if (gF == 0.0f) continue;
-      const float vel = AT(a.rom, kf, j, i);
-      const float s = sgn1(-vel);
-      float c;
-      if (kf >= 3 && kf < a.ktf - 2) c = c5(o, s);
-      else if (kf == 1 || kf == a.ktf - 1) c = o == 0 ? a.fzm[kf] : (o == -1 ? a.fzp[kf] : 0.0f);
-      else c = c3(o, s);   // kf == 2 or ktf - 2
-      acc += gF * vel * c;
-    }
-  }
-  // (each face sensitivity above already carries the sign with which the
-  // forward subtracts the face difference from the tendency)
-  float* out = &AT(a.out, k, j, i);
-  *out = a.accumulate ? *out + acc : acc;
-}
-
-extern "C" int pywrf_advect_scalar_adjoint(const pywrf_grid_t* g, const float* lam_tend, const float* ru,
-                                           const float* rv, const float* rom, const float* msftx, const float* fzm,
-                                           const float* fzp, double rdx, double rdy, const float* rdzw,
-                                           float* lam_field, int accumulate, pywrf_stream_t s) {
-  if (!pw_size_ok(g)) return PYWRF_E_RANGE;
-  CHECK(g, 4);
-  AdjS a;
-  a.lam = lam_tend; a.ru = ru; a.rv = rv; a.rom = rom; a.msftx = msftx; a.fzm = fzm; a.fzp = fzp; a.rdzw = rdzw;
-  a.out = lam_field; a.rdx = F(rdx); a.rdy = F(rdy); a.accumulate = accumulate;
-  a.ids = g->ids; a.ide = g->ide; a.jds = g->jds; a.jde = g->jde; a.ktf = imin(g->kte, g->kde - 1);
-  if (g->kts != 0 || a.ktf + 1 > g->nz || g->kte > g->nz) return PYWRF_E_RANGE;
-  const int i0 = g->its, i1 = imin(g->ite, g->ide - 1), j0 = g->jts, j1 = imin(g->jte, g->jde - 1);
-  a.badv = mkbox(g->kts, a.ktf, j0, j1, i0, i1);
-  a.by = mkbox(g->kts, a.ktf, imax(g->jts, g->jds + 1), imin(g->jte, g->jde - 2), i0, i1);
-  a.bx = mkbox(g->kts, a.ktf, j0, j1, imax(g->ids + 1, g->its), imin(g->ide - 2, g->ite));
-  Box all = whole(g);
-  PW_LAUNCH_BOX(k_advect_scalar_adj, all, s, dims_of(g), a);
-  PW_RET();
-}
 
 // ------------------------------------------------------------------ rk_update_scalar^T
 struct AdjU {
@@ -1315,333 +1181,5 @@ extern "C" int pywrf_small_step_finish_adjoint(
               g->jte, g->ite};
   Box pl = mkbox(0, 1, 0, g->ny, 0, g->nx);
   PW_LAUNCH_COLS(k_ssfinish_adj, pl, s, dims_of(g), a);
-  PW_RET();
-}
-
-// ------------------------------------------------------------------ advect_u^T
-// advect_u (wrf_dynamics.py:1112-1307) with the mass fluxes fixed is linear in
-// u except at the two x-faces next to the edges, whose upwind value is chosen
-// by the sign of u itself (piecewise linear: the forward's branch is taken).
-// Scatter form: each tendency point hands its sensitivity, through the
-// coefficients of its six faces' rules, to the u points those faces read
-// (atomic adds onto the zeroed output).
-struct AdjAdvU {
-  const float *lam, *u, *ru, *rv, *rom, *msfux, *fzm, *fzp, *rdzw;
-  float* gu;
-  float rdx, rdy;
-  int ids, ide, jds, jde, ktf;
-  Box b, by;
-};
-
-// the y-face jf of u column (k, i): weight w times d(face)/d(u at row jf + o)
-__device__ inline void u_yface_adj(const AdjAdvU& a, int jf, float rvs, float w, float* acc) {
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (jf >= a.jds + 3 && jf < a.jde - 3) {
-    const float vel = 0.5f * rvs, s = sgn1(vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else if (jf == a.jds + 1 || jf == a.jde - 2) {
-    put(0, 0.25f * rvs);
-    put(-1, 0.25f * rvs);
-  } else if (jf == a.jds + 2 || jf == a.jde - 3) {
-    const float vel = 0.5f * rvs, s = jf == a.jds + 2 ? sgn1(vel) : sgn1(0.0f);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  }
-}
-
-__device__ inline void u_xface_adj(const AdjAdvU& a, const Dims& D, int k, int j, int f, float rus, float w, float* acc) {
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (f >= a.ids + 3 && f < a.ide - 2) {
-    const float vel = 0.5f * rus, s = sgn1(vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else if (f == a.ids + 1) {
-    if (AT(a.u, k, j, f) < 0.0f) put(0, 0.5f * rus);
-    else { put(0, 0.25f * rus); put(-1, 0.25f * rus); }
-  } else if (f == a.ids + 2 || f == a.ide - 2) {
-    const float vel = 0.5f * rus, s = sgn1(vel);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  } else if (f == a.ide - 1) {
-    if (AT(a.u, k, j, f - 1) > 0.0f) put(-1, 0.5f * rus);
-    else { put(-1, 0.25f * rus); put(0, 0.25f * rus); }
-  }
-}
-
-__device__ inline void u_zface_adj(const AdjAdvU& a, int kf, float vel, float w, float* acc) {
-  if (kf < 1 || kf >= a.ktf) return;
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (kf >= 3 && kf < a.ktf - 2) {
-    const float s = sgn1(-vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else if (kf == 1 || kf == a.ktf - 1) {
-    put(0, vel * a.fzm[kf]);
-    put(-1, vel * a.fzp[kf]);
-  } else {
-    const float s = sgn1(-vel);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  }
-}
-
-__global__ void k_advect_u_adj(Box all, Dims D, AdjAdvU a) {
-  int k, j, i;
-  if (!box_point(all, k, j, i)) return;
-  const float lam = AT(a.lam, k, j, i);
-  if (lam == 0.0f) return;
-  const float msf = AT2(a.msfux, j, i), rdz = a.rdzw[k];
-  // the two faces of each direction read overlapping stencils: their shares
-  // are summed per target (offsets -3..3 from the point) before the atomics
-  float ay[7] = {}, ax[7] = {}, az[7] = {};
-  if (a.by.has(k, j, i)) {
-    const float wy = msf * a.rdy * lam;
-    u_yface_adj(a, j + 1, AT(a.rv, k, j + 1, i) + AT(a.rv, k, j + 1, i - 1), -wy, ay + 4);
-    u_yface_adj(a, j, AT(a.rv, k, j, i) + AT(a.rv, k, j, i - 1), wy, ay + 3);
-  }
-  const float wx = msf * a.rdx * lam;
-  u_xface_adj(a, D, k, j, i + 1, AT(a.ru, k, j, i + 1) + AT(a.ru, k, j, i), -wx, ax + 4);
-  u_xface_adj(a, D, k, j, i, AT(a.ru, k, j, i) + AT(a.ru, k, j, i - 1), wx, ax + 3);
-  const float wz = rdz * lam;
-  u_zface_adj(a, k + 1, 0.5f * (AT(a.rom, k + 1, j, i - 1) + AT(a.rom, k + 1, j, i)), -wz, az + 4);
-  u_zface_adj(a, k, 0.5f * (AT(a.rom, k, j, i - 1) + AT(a.rom, k, j, i)), wz, az + 3);
-  for (int m = 0; m < 7; ++m) {          // a nonzero share is one a face stencil read: in bounds
-    atomic_add(&AT(a.gu, k, j + m - 3, i), ay[m]);
-    atomic_add(&AT(a.gu, k, j, i + m - 3), ax[m]);
-    atomic_add(&AT(a.gu, k + m - 3, j, i), az[m]);
-  }
-}
-
-extern "C" int pywrf_advect_u_adjoint(const pywrf_grid_t* g, const float* lam_tendency, const float* u,
-                                      const float* ru, const float* rv, const float* rom, const float* msfux,
-                                      const float* fzm, const float* fzp, double rdx, double rdy,
-                                      const float* rdzw, float* lam_u, pywrf_stream_t s) {
-  if (!pw_size_ok(g)) return PYWRF_E_RANGE;
-  CHECK(g, 4);
-  const int ktf = imin(g->kte, g->kde - 1);
-  if (g->kts != 0 || ktf + 1 > g->nz) return PYWRF_E_RANGE;
-  const int i0 = imax(g->ids + 1, g->its), i1 = imin(g->ide - 1, g->ite);
-  const int j0 = g->jts, j1 = imin(g->jte, g->jde - 1);
-  AdjAdvU a;
-  a.lam = lam_tendency; a.u = u; a.ru = ru; a.rv = rv; a.rom = rom; a.msfux = msfux; a.fzm = fzm; a.fzp = fzp;
-  a.rdzw = rdzw; a.gu = lam_u; a.rdx = F(rdx); a.rdy = F(rdy);
-  a.ids = g->ids; a.ide = g->ide; a.jds = g->jds; a.jde = g->jde; a.ktf = ktf;
-  a.b = mkbox(g->kts, ktf, j0, j1, i0, i1);
-  a.by = mkbox(g->kts, ktf, imax(g->jts, g->jds + 1), imin(g->jte, g->jde - 2), i0, i1);
-  hipLaunchKernelGGL(k_zero_n, dim3(1024), dim3(256), 0, (hipStream_t)s, lam_u, (long)g->nz * g->ny * g->nx);
-  PW_LAUNCH_BOX(k_advect_u_adj, a.b, s, dims_of(g), a);
-  PW_RET();
-}
-
-// ------------------------------------------------------------------ advect_v^T
-// advect_v (wrf_dynamics.py:1332-1532), as advect_u's transpose with the roles
-// of x and y exchanged: the upwind choice by the sign of v at the edge
-// y-faces, the symmetric rules at the x-faces, the z term scaled by
-// msfvy / msfvx, and the reference's +v sign at the z-face ktf-2.
-struct AdjAdvV {
-  const float *lam, *v, *ru, *rv, *rom, *msfvx, *msfvy, *fzm, *fzp, *rdzw;
-  float* gv;
-  float rdx, rdy;
-  int ids, ide, jds, jde, ktf;
-  Box b, bx;
-};
-
-__device__ inline void v_yface_adj(const AdjAdvV& a, const Dims& D, int k, int f, int i, float rvs, float w, float* acc) {
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (f >= a.jds + 3 && f < a.jde - 2) {
-    const float vel = 0.5f * rvs, s = sgn1(vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else if (f == a.jds + 1) {
-    if (AT(a.v, k, f, i) < 0.0f) put(0, 0.5f * rvs);
-    else { put(0, 0.25f * rvs); put(-1, 0.25f * rvs); }
-  } else if (f == a.jds + 2 || f == a.jde - 2) {
-    const float vel = 0.5f * rvs, s = sgn1(vel);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  } else if (f == a.jde - 1) {
-    if (AT(a.v, k, f - 1, i) > 0.0f) put(-1, 0.5f * rvs);
-    else { put(-1, 0.25f * rvs); put(0, 0.25f * rvs); }
-  }
-}
-
-__device__ inline void v_xface_adj(const AdjAdvV& a, const Dims& D, int k, int j, int f, float rus, float w, float* acc) {
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (f >= a.ids + 3 && f < a.ide - 3) {
-    const float vel = 0.5f * rus, s = sgn1(vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else if (f == a.ids + 1 || f == a.ide - 2) {
-    put(0, 0.25f * rus);
-    put(-1, 0.25f * rus);
-  } else if (f == a.ids + 2 || f == a.ide - 3) {
-    const float vel = 0.5f * rus, s = sgn1(vel);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  }
-}
-
-__device__ inline void v_zface_adj(const AdjAdvV& a, const Dims& D, int kf, int j, int i, float vel, float w, float* acc) {
-  if (kf < 1 || kf >= a.ktf) return;
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (kf >= 3 && kf < a.ktf - 2) {
-    const float s = sgn1(-vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else if (kf == 1 || kf == a.ktf - 1) {
-    put(0, vel * a.fzm[kf]);
-    put(-1, vel * a.fzp[kf]);
-  } else {
-    const float s = kf == 2 ? sgn1(-vel) : sgn1(vel);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  }
-}
-
-__global__ void k_advect_v_adj(Box all, Dims D, AdjAdvV a) {
-  int k, j, i;
-  if (!box_point(all, k, j, i)) return;
-  const float lam = AT(a.lam, k, j, i);
-  if (lam == 0.0f) return;
-  const float my = AT2(a.msfvy, j, i), mvx = AT2(a.msfvx, j, i), rdz = a.rdzw[k];
-  // shares summed per target (offsets -3..3 from the point) before the atomics
-  float ay[7] = {}, ax[7] = {}, az[7] = {};
-  const float wy = my * a.rdy * lam;
-  v_yface_adj(a, D, k, j + 1, i, AT(a.rv, k, j + 1, i) + AT(a.rv, k, j, i), -wy, ay + 4);
-  v_yface_adj(a, D, k, j, i, AT(a.rv, k, j, i) + AT(a.rv, k, j - 1, i), wy, ay + 3);
-  if (a.bx.has(k, j, i)) {
-    const float wx = my * a.rdx * lam;
-    v_xface_adj(a, D, k, j, i + 1, AT(a.ru, k, j, i + 1) + AT(a.ru, k, j - 1, i + 1), -wx, ax + 4);
-    v_xface_adj(a, D, k, j, i, AT(a.ru, k, j, i) + AT(a.ru, k, j - 1, i), wx, ax + 3);
-  }
-  const float wz = (my / mvx) * rdz * lam;
-  v_zface_adj(a, D, k + 1, j, i, 0.5f * (AT(a.rom, k + 1, j, i) + AT(a.rom, k + 1, j - 1, i)), -wz, az + 4);
-  v_zface_adj(a, D, k, j, i, 0.5f * (AT(a.rom, k, j, i) + AT(a.rom, k, j - 1, i)), wz, az + 3);
-  for (int m = 0; m < 7; ++m) {          // a nonzero share is one a face stencil read: in bounds
-    atomic_add(&AT(a.gv, k, j + m - 3, i), ay[m]);
-    atomic_add(&AT(a.gv, k, j, i + m - 3), ax[m]);
-    atomic_add(&AT(a.gv, k + m - 3, j, i), az[m]);
-  }
-}
-
-extern "C" int pywrf_advect_v_adjoint(const pywrf_grid_t* g, const float* lam_tendency, const float* v,
-                                      const float* ru, const float* rv, const float* rom, const float* msfvx,
-                                      const float* msfvy, const float* fzm, const float* fzp, double rdx, double rdy,
-                                      const float* rdzw, float* lam_v, pywrf_stream_t s) {
-  if (!pw_size_ok(g)) return PYWRF_E_RANGE;
-  CHECK(g, 4);
-  const int ktf = imin(g->kte, g->kde - 1);
-  if (g->kts != 0 || ktf + 1 > g->nz) return PYWRF_E_RANGE;
-  const int i0 = g->its, i1 = imin(g->ite, g->ide - 1);
-  const int j0 = imax(g->jts, g->jds + 1), j1 = imin(g->jte, g->jde - 1);
-  AdjAdvV a;
-  a.lam = lam_tendency; a.v = v; a.ru = ru; a.rv = rv; a.rom = rom; a.msfvx = msfvx; a.msfvy = msfvy;
-  a.fzm = fzm; a.fzp = fzp; a.rdzw = rdzw; a.gv = lam_v; a.rdx = F(rdx); a.rdy = F(rdy);
-  a.ids = g->ids; a.ide = g->ide; a.jds = g->jds; a.jde = g->jde; a.ktf = ktf;
-  a.b = mkbox(g->kts, ktf, j0, j1, i0, i1);
-  a.bx = mkbox(g->kts, ktf, j0, j1, imax(g->ids + 1, g->its), imin(g->ide - 2, g->ite));
-  hipLaunchKernelGGL(k_zero_n, dim3(1024), dim3(256), 0, (hipStream_t)s, lam_v, (long)g->nz * g->ny * g->nx);
-  PW_LAUNCH_BOX(k_advect_v_adj, a.b, s, dims_of(g), a);
-  PW_RET();
-}
-
-// ------------------------------------------------------------------ advect_w^T
-// advect_w (wrf_dynamics.py:1535-1838) is linear in w with the mass fluxes
-// fixed (the horizontal ones interpolated to w levels, extrapolated at the
-// top; the vertical faces' rules from 2nd order at the ends to 5th inside,
-// with the reference's +w sign at the face ktf-1; at the top level only the
-// face below, doubled).  Scatter form as advect_u's.
-struct AdjAdvW {
-  const float *lam, *ru, *rv, *rom, *msftx, *fzm, *fzp, *rdzu;
-  float* gw;
-  float rdx, rdy;
-  int ids, ide, jds, jde, ktf;
-  Box b, by, bx;
-};
-
-__device__ inline float w_level_flux_a(const AdjAdvW& a, int k, float rA, float rB) {
-  if (k < a.ktf) return a.fzm[k] * rA + a.fzp[k] * rB;
-  return (2.0f - a.fzm[a.ktf - 1]) * rA - a.fzp[a.ktf - 1] * rB;
-}
-
-// the horizontal face f of a row or column [lo, hi): d(face) / d(w at f + o), times w
-template <class Put>
-__device__ inline void w_hface_adj(int f, int lo, int hi, float vel, float w, Put put) {
-  if (f >= lo + 3 && f < hi - 3) {
-    const float s = sgn1(vel);
-    for (int o = -3; o <= 2; ++o) put(o, w * vel * c5(o, s));
-  } else if (f == lo + 1 || f == hi - 2) {
-    put(0, w * 0.5f * vel);
-    put(-1, w * 0.5f * vel);
-  } else if (f == lo + 2 || f == hi - 3) {
-    const float s = sgn1(vel);
-    for (int o = -2; o <= 1; ++o) put(o, w * vel * c3(o, s));
-  }
-}
-
-__device__ inline void w_zface_adj(const AdjAdvW& a, int kf, float rs, float w, float* acc) {
-  if (kf < 1 || kf > a.ktf) return;
-  auto put = [&](int o, float c) { acc[o] += w * c; };
-  if (kf == 1 || kf == a.ktf) {
-    put(0, 0.25f * rs);
-    put(-1, 0.25f * rs);
-    return;
-  }
-  const float vel = 0.5f * rs;
-  if (kf >= 3 && kf < a.ktf - 1) {
-    const float s = sgn1(-vel);
-    for (int o = -3; o <= 2; ++o) put(o, vel * c5(o, s));
-  } else {
-    const float s = kf == 2 ? sgn1(-vel) : sgn1(vel);
-    for (int o = -2; o <= 1; ++o) put(o, vel * c3(o, s));
-  }
-}
-
-__global__ void k_advect_w_adj(Box all, Dims D, AdjAdvW a) {
-  int k, j, i;
-  if (!box_point(all, k, j, i)) return;
-  const float lam = AT(a.lam, k, j, i);
-  if (lam == 0.0f) return;
-  const int ktf = a.ktf, top = k >= ktf;
-  const int kA = top ? ktf - 1 : k, kB = imax(top ? ktf - 2 : k - 1, 0);
-  const float mx = AT2(a.msftx, j, i), rdz = a.rdzu[top ? ktf - 1 : k];
-  // shares summed per target (offsets -3..3 from the point) before the atomics
-  float ay[7] = {}, ax[7] = {}, az[7] = {};
-  auto into = [](float* acc) { return [acc](int o, float c) { acc[o] += c; }; };
-  if (a.by.has(k, j, i)) {
-    const float wy = mx * a.rdy * lam;
-    w_hface_adj(j + 1, a.jds, a.jde, w_level_flux_a(a, k, AT(a.rv, kA, j + 1, i), AT(a.rv, kB, j + 1, i)), -wy,
-                into(ay + 4));
-    w_hface_adj(j, a.jds, a.jde, w_level_flux_a(a, k, AT(a.rv, kA, j, i), AT(a.rv, kB, j, i)), wy, into(ay + 3));
-  }
-  if (a.bx.has(k, j, i)) {
-    const float wx = mx * a.rdx * lam;
-    w_hface_adj(i + 1, a.ids, a.ide, w_level_flux_a(a, k, AT(a.ru, kA, j, i + 1), AT(a.ru, kB, j, i + 1)), -wx,
-                into(ax + 4));
-    w_hface_adj(i, a.ids, a.ide, w_level_flux_a(a, k, AT(a.ru, kA, j, i), AT(a.ru, kB, j, i)), wx, into(ax + 3));
-  }
-  const float rm0 = AT(a.rom, k, j, i), rmb = AT(a.rom, imax(k - 1, 0), j, i);
-  if (!top) {
-    const float rmn = AT(a.rom, imin(k + 1, D.nz - 1), j, i);
-    w_zface_adj(a, k + 1, rmn + rm0, -rdz * lam, az + 4);
-    w_zface_adj(a, k, rm0 + rmb, rdz * lam, az + 3);
-  } else {
-    w_zface_adj(a, k, rm0 + rmb, 2.0f * rdz * lam, az + 3);
-  }
-  for (int m = 0; m < 7; ++m) {          // a nonzero share is one a face stencil read: in bounds
-    atomic_add(&AT(a.gw, k, j + m - 3, i), ay[m]);
-    atomic_add(&AT(a.gw, k, j, i + m - 3), ax[m]);
-    atomic_add(&AT(a.gw, k + m - 3, j, i), az[m]);
-  }
-}
-
-extern "C" int pywrf_advect_w_adjoint(const pywrf_grid_t* g, const float* lam_tendency, const float* ru,
-                                      const float* rv, const float* rom, const float* msftx, const float* fzm,
-                                      const float* fzp, double rdx, double rdy, const float* rdzu, float* lam_w,
-                                      pywrf_stream_t s) {
-  if (!pw_size_ok(g)) return PYWRF_E_RANGE;
-  CHECK(g, 4);
-  const int ktf = imin(g->kte, g->kde - 1);
-  if (g->kts != 0 || ktf + 1 > g->nz || ktf < 3) return PYWRF_E_RANGE;
-  const int i0 = g->its, i1 = imin(g->ite, g->ide - 1);
-  const int j0 = g->jts, j1 = imin(g->jte, g->jde - 1);
-  AdjAdvW a;
-  a.lam = lam_tendency; a.ru = ru; a.rv = rv; a.rom = rom; a.msftx = msftx; a.fzm = fzm; a.fzp = fzp;
-  a.rdzu = rdzu; a.gw = lam_w; a.rdx = F(rdx); a.rdy = F(rdy);
-  a.ids = g->ids; a.ide = g->ide; a.jds = g->jds; a.jde = g->jde; a.ktf = ktf;
-  a.b = mkbox(g->kts + 1, ktf + 1, j0, j1, i0, i1);
-  a.by = mkbox(g->kts + 1, ktf + 1, imax(g->jts, g->jds + 1), imin(g->jte, g->jde - 2), i0, i1);
-  a.bx = mkbox(g->kts + 1, ktf + 1, j0, j1, imax(g->ids + 1, g->its), imin(g->ide - 2, g->ite));
-  hipLaunchKernelGGL(k_zero_n, dim3(1024), dim3(256), 0, (hipStream_t)s, lam_w, (long)g->nz * g->ny * g->nx);
-  PW_LAUNCH_BOX(k_advect_w_adj, a.b, s, dims_of(g), a);
   PW_RET();
 }

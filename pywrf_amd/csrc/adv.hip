@@ -378,7 +378,7 @@ __device__ inline float s_xface_v(const AdvIdx& x, int f, float vel, float vel1,
 __device__ inline float s_zface_v(const AdvS& a, const AdvIdx& x, int kf, float vel, const float* Q) {
   if (kf < 1 || kf >= x.ktf) return 0.0f;
   if (kf >= 3 && kf < x.ktf - 2) return vel * flux5(Q[0], Q[1], Q[2], Q[3], Q[4], Q[5], -vel);
-  if (kf == 1 || kf == x.ktf - 1) return vel * (a.fzm[kf] * Q[3] + a.fzp[kf] * Q[2]);
+  if (kf == 1 || kf == x.ktf - 1) return vel * (level(a.fzm, kf) * Q[3] + level(a.fzp, kf) * Q[2]);
   return vel * flux3(Q[1], Q[2], Q[3], Q[4], -vel);  // kf == 2 or ktf-2
 }
 
@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(PW_TX * PW_TY) k_scalar_adv(Dims D, ScalarTend
     }
 #pragma unroll
     for (int r = 0; r <= R; ++r) yv[r] = AT(ad.rv, k, jr[r + 3], ic);
-    const float rdz = ad.rdzw[k];
+    const float rdz = level(ad.rdzw, k);
     float ylo = s_yface_v(a.x, j0, yv[0], q);
 #pragma unroll
     for (int r = 0; r < R; ++r) {

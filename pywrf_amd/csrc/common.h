@@ -171,6 +171,14 @@ __device__ inline float flux3(float qm2, float qm1, float q0, float qp1, float u
   return f4 + (ua >= 0.0f ? q : -q);
 }
 
+// Entry k of a level array (k the same in the whole wave) by a scalar load.  A
+// kernel never writes the level arrays, which the constant address space says
+// to the compiler: after a store to another array it would take a plain read
+// for a vector load that has to wait for the store.
+__device__ __forceinline__ float level(const float* p, int k) {
+  return ((const __attribute__((address_space(4))) float*)p)[k];
+}
+
 // The value of the next lower / higher lane of the wave (DPP wave shifts, one
 // VALU operation; the end lane keeps its own).  All 64 lanes must be active.
 __device__ __forceinline__ float lane_below(float x) {

@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
     r_t[m] = tin + 0.0f;
     r_p[m] = tin + my * a.dts * ftq;
     r_h[m] = mx * (yterm + xterm);
-    r_c[m] = a.fnm[k] * t1 + a.fnp[k] * t1d;
+    r_c[m] = level(a.fnm, k) * t1 + level(a.fnp, k) * t1d;
   }
   __syncthreads();
   // The column sum dmdt in torch's order (torch_outer_sum with nz <= 128:
@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
       const int k = imin(k0 + m, k1 - 1);
-      const float x = a.dnw[k] * s_dv[k * TI + lane];
+      const float x = level(a.dnw, k) * s_dv[k * TI + lane];
       acc += k0 + m < ke ? x : 0.0f;
     }
     s_part[c * TI + lane] = acc;
@@ -511,7 +511,7 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
 #pragma unroll
   for (int m = 0; m < LPT; ++m) {
     const int k = grp + m * TG;
-    if (k < k1) s_dv[k * TI + lane] = a.dnw[k] * (dmdt + s_dv[k * TI + lane] + mt) / my;
+    if (k < k1) s_dv[k * TI + lane] = level(a.dnw, k) * (dmdt + s_dv[k * TI + lane] + mt) / my;
   }
   __syncthreads();
   if (grp == 0) {
@@ -556,7 +556,7 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a) {
     const float wdu = k + 1 < k1 ? s_dv[(k + 1) * TI + lane] : 0.0f;
     AT(a.ww, k, j, i) = r_w1[m];
     AT(a.t_ave, k, j, i) = r_t[m];
-    AT(a.t, k, j, i) = r_p[m] - a.dts * my * (r_h[m] + a.rdnw[k] * (wdu - r_c[m]));
+    AT(a.t, k, j, i) = r_p[m] - a.dts * my * (r_h[m] + level(a.rdnw, k) * (wdu - r_c[m]));
   }
   for (int k = k1 + grp; k < nz; k += TG) {   // levels at and above k1 copy their inputs
     const long q = D.ix(k, j, i);
@@ -678,7 +678,7 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
     const float al = AT(a.alpha, k, j, ic);
     r_ga[m] = AT(a.gamma, k, j, ic);
     // wdwn(k) = 0.5 (ww[k] + ww[k-1]) rdnw[k-1] (ph_1[k] - ph_1[k-1] + phb[k] - phb[k-1])
-    const float wd = 0.5f * (ww0 + wwm) * a.rdnw[k - 1] * (p10 - p1m + pb0 - pbm);
+    const float wd = 0.5f * (ww0 + wwm) * level(a.rdnw, k - 1) * (p10 - p1m + pb0 - pbm);
     const float t2a = k < k1 ? theta_ave(t2i, t2, t1) : t2i;
     if (1 + grp + m * TG <= k1) {
       s_wd[k * TI + lane] = wd;
@@ -688,7 +688,7 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
     r_t2a[m] = t2a;
     r_w[m] = win + a.dts * rwt;
     r_cq[m] = mi * cq;
-    r_cb[m] = c2 * a.rdnw[kl] / mut;
+    r_cb[m] = c2 * level(a.rdnw, kl) / mut;
     r_e[m] = a.em1 * (php - phi);
     r_rhs[m] = a.dts * (pht + a.hgem1 * win);
     r_phi[m] = phi;
@@ -696,7 +696,7 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
   }
   if (grp == ktw) {
     const float c2m = AT(a.c2a, k1 - 1, j, ic), alm = AT(a.alt, k1 - 1, j, ic);
-    const float ph0 = AT(a.ph_in, k1, j, ic), phm = AT(a.ph_in, k1 - 1, j, ic), rn = a.rdnw[k1 - 1];
+    const float ph0 = AT(a.ph_in, k1, j, ic), phm = AT(a.ph_in, k1 - 1, j, ic), rn = level(a.rdnw, k1 - 1);
     const float t2a = theta_ave(AT(a.t_2ave_in, k1 - 1, j, ic), AT(a.t_2, k1 - 1, j, ic), AT(a.t_1, k1 - 1, j, ic));
     z_a = a.mhdtsg / mut * (rn * rn) * 2.0f * c2m;
     z_e = a.em1 * (ph0 - phm);
@@ -704,7 +704,7 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
   }
   float z_cb = 0.0f, w_sfc = 0.0f, ph_sfc = 0.0f;
   if (grp == k0w) {
-    const float cf1 = a.cf[0], cf2 = a.cf[1], cf3 = a.cf[2];
+    const float cf1 = level(a.cf, 0), cf2 = level(a.cf, 1), cf3 = level(a.cf, 2);
     auto V3 = [&](int jj, int ii) {
       return cf1 * AT(a.v, 0, jj, ii) + cf2 * AT(a.v, 1, jj, ii) + cf3 * AT(a.v, 2, jj, ii);
     };
@@ -720,7 +720,7 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
     w_sfc = my * 0.5f * a.rdy * ty + mx * 0.5f * a.rdx * tx;
     t2a_sfc = theta_ave(t2i, t2, t1);
     s_yp[lane] = c2 * alt * t2a_sfc;
-    z_cb = c2 * a.rdnw[0] / mut;
+    z_cb = c2 * level(a.rdnw, 0) / mut;
     z_e = a.em1 * (php - ph_sfc);
     s_rhs[lane] = 0.0f;
   }
@@ -731,7 +731,7 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
     const int k = 1 + grp + m * TG;
     if (k > k1) continue;
     float r = r_rhs[m];
-    if (k < k1) r = r - a.dts * (a.fnm[k] * s_wd[(k + 1) * TI + lane] + a.fnp[k] * s_wd[k * TI + lane]);
+    if (k < k1) r = r - a.dts * (level(a.fnm, k) * s_wd[(k + 1) * TI + lane] + level(a.fnp, k) * s_wd[k * TI + lane]);
     r = r_phi[m] + my * r / mut;
     r_rhs[m] = r;
     s_rhs[k * TI + lane] = r;
@@ -756,8 +756,8 @@ __global__ void __launch_bounds__(TB) k_advance_w(Dims D, AdvW a) {
     if (k > k1) continue;
     float w = r_w[m];
     if (k < k1) {
-      const float X = a.hdtsg * a.rdn[k] * (s_wd[k * TI + lane] - s_wd[(k - 1) * TI + lane]);
-      const float Y = a.rdn[k] * (s_yp[k * TI + lane] - s_yp[(k - 1) * TI + lane]) - muave;
+      const float X = a.hdtsg * level(a.rdn, k) * (s_wd[k * TI + lane] - s_wd[(k - 1) * TI + lane]);
+      const float Y = level(a.rdn, k) * (s_yp[k * TI + lane] - s_yp[(k - 1) * TI + lane]) - muave;
       w = w + r_cq[m] * X + a.dtsg * mi * Y;
     }
     s_rhs[k * TI + lane] = w;
