@@ -138,45 +138,87 @@ LEVEL_IN = {"rdzw": "pywrf_advect_"}
 class TensorPtr(ctypes.c_void_p):
     """Device pointer of a tensor argument; `shape` is checked against the
     call's grid before the launch."""
+    __slots__ = ("shape",)
 
 
 class BoundaryPtr(ctypes.c_void_p):
     """Device pointer of a lateral-boundary array (checked by bptr)."""
 
 
+def _roles(name, params):
+    """[(position, parameter name, role)] of an entry point's parameters: the
+    entries a level array needs (0: the grid's nz), -2 for a plane, -3 for a
+    field."""
+    out = []
+    for n, pname in enumerate(params):
+        if pname in LEVEL_PARAMS or (pname in LEVEL_IN and name.startswith(LEVEL_IN[pname])):
+            out.append((n, pname, LEVEL_PARAMS.get(pname) or 0))
+        else:
+            out.append((n, pname, -2 if pname in PLANE_PARAMS else -3))
+    return out
+
+
+_ROLES = {}     # of each entry point's own parameters, by name
+
+
 def check_operands(name, g, params, args):
     """Raise IndexError when an array operand is smaller than the part of it
     the kernel addresses for grid g (a Grid), so that no mismatched operand
     reaches a kernel.  params: the C parameter names, args: the arguments."""
-    nz, ny, nx = g.nz, g.ny, g.nx
-    for pname, a in zip(params, args):
-        if not isinstance(a, TensorPtr):
+    _check_roles(name, (g.nz, g.ny, g.nx), _roles(name, params), args)
+
+
+def _check_roles(name, full, roles, args):
+    plane = full[1:]
+    for n, pname, role in roles:
+        a = args[n] if n < len(args) else None
+        if type(a) is not TensorPtr:
             continue
         shape = a.shape
-        if pname in LEVEL_PARAMS or (pname in LEVEL_IN and name.startswith(LEVEL_IN[pname])):
-            need = LEVEL_PARAMS.get(pname) or nz
-            if pname == "cf" and len(shape) == 0:
+        # the common case of each role first: an operand of exactly the grid's shape
+        if role == -3:
+            if shape == full:
+                continue
+        elif role == -2:
+            if shape == plane:
+                continue
+        else:
+            if len(shape) == 1:
+                if shape[0] >= (role or full[0]):
+                    continue
+            elif pname == "cf" and len(shape) == 0:
                 continue                      # (cf1, cf2, cf3) checked adjacent by the caller
-            n = 1
+            need, m = role or full[0], 1
             for d in shape:
-                n *= d
-            if n < need:
-                raise IndexError("%s: %s has %d entries, the grid needs %d" % (name, pname, n, need))
+                m *= d
+            if m < need:
+                raise IndexError("%s: %s has %d entries, the grid needs %d" % (name, pname, m, need))
             continue
-        if len(shape) < 2 or tuple(shape[-2:]) != (ny, nx):
-            raise IndexError("%s: %s has shape %s, the grid is (%d, %d, %d)" % (name, pname, tuple(shape), nz, ny, nx))
-        if pname in PLANE_PARAMS:
+        if len(shape) < 2 or tuple(shape[-2:]) != plane:
+            raise IndexError("%s: %s has shape %s, the grid is (%d, %d, %d)" % ((name, pname, tuple(shape)) + full))
+        if role == -2:
             continue
         lev = shape[-3] if len(shape) >= 3 else 1
-        if lev < nz:
-            raise IndexError("%s: %s has %d levels, the grid needs %d (shape %s)" % (name, pname, lev, nz,
+        if lev < full[0]:
+            raise IndexError("%s: %s has %d levels, the grid needs %d (shape %s)" % (name, pname, lev, full[0],
                                                                                     tuple(shape)))
 
 
 def call(name, *args):
     if args and isinstance(args[0], _GridPtr):
-        check_operands(name, args[0].contents, PARAMS[name], args)
-    check(name, getattr(LIB, name)(*args))
+        g = args[0]
+        try:
+            full = g.full                     # kept by grid(); g.contents builds a Grid each time
+        except AttributeError:
+            g = g.contents
+            full = (g.nz, g.ny, g.nx)
+        roles = _ROLES.get(name)
+        if roles is None:
+            roles = _ROLES[name] = _roles(name, PARAMS[name])
+        _check_roles(name, full, roles, args)
+    rc = getattr(LIB, name)(*args)
+    if rc:
+        check(name, rc)
 
 
 _grid_cache = {}
@@ -185,7 +227,7 @@ _grid_cache = {}
 def grid(shape, idx):
     """pywrf_grid_t for an array shape and an index tuple of 16, 18 or 24 ints
     (the reference's 2-D, tile-only and patch+tile argument lists)."""
-    key = (tuple(shape), tuple(idx))
+    key = (shape, idx) if type(idx) is tuple else (tuple(shape), tuple(idx))
     g = _grid_cache.get(key)
     if g is not None:
         return g
@@ -210,18 +252,19 @@ def grid(shape, idx):
         # indices' extent (the kernels only use the (j, i) plane)
         v["nz"] = max(1, v["kte"], v["kde"])
     g = ctypes.pointer(Grid(**{n: int(v[n]) for n in _GRID_FIELDS}))
-    _grid_cache[key] = g
+    g.full = (int(v["nz"]), int(v["ny"]), int(v["nx"]))
+    _grid_cache[(tuple(shape), tuple(idx))] = g
     return g
 
 
 def stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _require_device(t):
     if not isinstance(t, torch.Tensor):
         raise TypeError("expected a tensor, got %r" % type(t))
-    if t.device.type != "cuda" or t.dtype != torch.float32:
+    if not t.is_cuda or t.dtype is not torch.float32:
         raise TypeError("expected a float32 CUDA tensor, got %s %s" % (t.device, t.dtype))
 
 
@@ -231,7 +274,7 @@ def ptr(t):
     if not t.is_contiguous():
         raise TypeError("expected a contiguous float32 CUDA tensor, got strides %s" % (t.stride(),))
     p = TensorPtr(t.data_ptr())
-    p.shape = tuple(t.shape)
+    p.shape = t.shape
     return p
 
 
@@ -248,10 +291,10 @@ def boundary_layout(t, kind, kz, n):
     while the array's data and version are unchanged."""
     _require_device(t)
     want = (kz, n, 5) if kind == "x" else (kz, 5, n)
-    if tuple(t.shape) != want:
+    if t.shape != want:
         raise IndexError("boundary array has shape %s, expected %s (spec_bdy_width 5)" % (tuple(t.shape), want))
     strides = (n, 1, kz * n) if kind == "x" else (n, kz * n, 1)
-    if tuple(t.stride()) == strides or t.numel() == 0:
+    if t.stride() == strides or t.numel() == 0:
         return t
     key = (t.data_ptr(), tuple(t.stride()), kind)
     hit = _bdy_copies.get(key)

@@ -11,6 +11,7 @@ torch's current stream; nothing here synchronises the device.
 Tensors are contiguous FP32 CUDA tensors, 3-D (nz, ny, nx), 2-D (ny, nx),
 level arrays (nz,); 0-d tensors for cf1..cf3, cfn, cfn1.
 """
+import functools
 import inspect
 from types import SimpleNamespace
 
@@ -921,9 +922,14 @@ def rk_scalar_tend(scs, sce,
     return scalar_tends, advect_tend, h_tendency, z_tendency
 
 
+@functools.lru_cache(maxsize=None)
+def _names(fn):
+    return tuple(inspect.signature(fn).parameters)
+
+
 def _bind(fn, args):
     """The positional arguments of a call of `fn`, by parameter name."""
-    names = list(inspect.signature(fn).parameters)
+    names = _names(fn)
     if len(args) != len(names):
         raise TypeError("%s takes %d positional arguments, got %d" % (fn.__name__, len(names), len(args)))
     return SimpleNamespace(**dict(zip(names, args)))
@@ -931,7 +937,7 @@ def _bind(fn, args):
 
 def _shared(fn, a, b, own):
     """Raise unless the two bound calls of `fn` agree on every argument outside `own`."""
-    for n in inspect.signature(fn).parameters:
+    for n in _names(fn):
         if n in own:
             continue
         x, y = getattr(a, n), getattr(b, n)
