@@ -551,13 +551,27 @@ int pywrf_mlp_gemm(int epi, int M, int N, int K, const void* A, int lda, const v
 int pywrf_mlp_frag_pack(int N, int K, const void* W, int ldw, void* out, pywrf_stream_t s);
 /* out[c][r] = in[r][c], BF16. */
 int pywrf_mlp_transpose(int R, int C, const void* in, int ldi, void* out, int ldo, pywrf_stream_t s);
+/* The same for n <= 8 matrices in one launch. */
+int pywrf_mlp_transpose_group(int n, const int* R, const int* C, void* const* in, const int* ldi, void* const* out,
+                              const int* ldo, pywrf_stream_t s);
+/* BF16 rows [M x ldo] of the FP32 rows in [M x ldi]: columns [0, N) converted, [N, ldo) zero (ldo a
+ * multiple of 8, out 16-byte aligned). */
+int pywrf_mlp_to_bf16(int M, int N, const float* in, int ldi, void* out, int ldo, pywrf_stream_t s);
 /* out[r] = sum_{c < C} in[r][c] (BF16 in, FP32 out): bias gradients. */
 int pywrf_mlp_rowsum(int R, int C, const void* in, int ld, float* out, pywrf_stream_t s);
+/* The same for n <= 8 matrices in one launch. */
+int pywrf_mlp_rowsum_group(int n, const int* R, const int* C, void* const* in, const int* ld, void* const* out,
+                           pywrf_stream_t s);
 /* Weighted squared error of Y (FP32 [B x ldy]) against T over N outputs:
  * *loss += sum w[n] (Y - T)^2 scale, dY (BF16 [B x lddy]) = 2 w[n] (Y - T) scale
  * (0 in columns N .. lddy). */
 int pywrf_mlp_mse(int B, int N, const float* Y, int ldy, const float* T, int ldt, const float* w, double scale,
                   void* dY, int lddy, float* loss, pywrf_stream_t s);
+/* One Adam step (pywrf_mlp_adam) of n <= 8 parameters in one launch; wb / wtb: arrays of n pointers, each of
+ * which may be null. */
+int pywrf_mlp_adam_group(int n, const int* rows, const int* cols, void* const* w, void* const* g, void* const* m,
+                         void* const* v, double lr, double beta1, double beta2, double eps, double gscale, int t,
+                         void* const* wb, void* const* wtb, pywrf_stream_t s);
 /* One bias-corrected Adam step of an FP32 [rows x cols] parameter with
  * gradient g * gscale (step number t >= 1); wb / wtb (optional) receive its
  * BF16 copy and transposed BF16 copy. */

@@ -1052,24 +1052,26 @@ class SurrogateNet(torch.autograd.Function):
     @staticmethod
     def forward(ctx, X, net):
         M = X.shape[0]
-        ws = _sg.Workspace(M, device=X.device)
-        Xb = torch.zeros(M, _sg.KIN, dtype=torch.bfloat16, device=X.device)
-        Xb[:, :_sg.FIN] = X.to(torch.bfloat16)
-        Y = _sg.forward(net, Xb, ws)
-        ctx.net, ctx.ws = net, ws
-        return Y[:, :_sg.FOUT].clone()
+        if M % 32:
+            raise ValueError("batch size must be a multiple of 32")
+        bf = dict(dtype=torch.bfloat16, device=X.device)
+        H1, H2 = torch.empty(M, _sg.HID, **bf), torch.empty(M, _sg.HID, **bf)
+        Y = torch.empty(M, _sg.FOUT, device=X.device)
+        _sg.gemm(1, _sg.to_bf16(X, _sg.KIN), net.Wb[0], H1, net.b[0])
+        _sg.gemm(1, H1, net.Wb[1], H2, net.b[1])
+        _sg.gemm(0, H2, net.Wb[2][:_sg.FOUT], Y, net.b[2])
+        ctx.net, ctx.H = net, (H1, H2)
+        return Y
 
     @staticmethod
     def backward(ctx, dY):
-        net, ws = ctx.net, ctx.ws
-        M = ws.M
-        dYb = torch.zeros(M, _sg.NO, dtype=torch.bfloat16, device=dY.device)
-        dYb[:, :_sg.FOUT] = dY.to(torch.bfloat16)
-        _sg.gemm(2, dYb, net.Wt[2], ws.dH2, H=ws.H2)        # (dY W3) [H2 > 0]
-        _sg.gemm(2, ws.dH2, net.Wt[1], ws.dH1, H=ws.H1)     # (dH2 W2) [H1 > 0]
-        dX = torch.empty(M, _sg.KIN, dtype=torch.float32, device=dY.device)
-        _sg.gemm(0, ws.dH1, net.Wt[0], dX)                  # dH1 W1
-        return dX[:, :_sg.FIN].clone(), None
+        net, (H1, H2) = ctx.net, ctx.H
+        dH2, dH1 = torch.empty_like(H2), torch.empty_like(H1)
+        _sg.gemm(2, _sg.to_bf16(dY, _sg.NO), net.Wt[2], dH2, H=H2)     # (dY W3) [H2 > 0]
+        _sg.gemm(2, dH2, net.Wt[1], dH1, H=H1)                         # (dH2 W2) [H1 > 0]
+        dX = torch.empty(H1.shape[0], _sg.FIN, device=dY.device)
+        _sg.gemm(0, dH1, net.Wt[0][:_sg.FIN], dX)                      # dH1 W1
+        return dX, None
 
 
 class AcousticStage(torch.autograd.Function):

@@ -28,6 +28,7 @@ import torch
 
 from . import _lib
 from ._lib import call, grid, ptr, stream
+from .wrf_dynamics import zero_group
 
 NLEV, NIN, NOUT = 41, 9, 7
 FIN, FOUT = NLEV * NIN, NLEV * NOUT          # 369, 287
@@ -90,6 +91,42 @@ def transpose(x, out):
     if tuple(out.shape) != (C, R):
         raise IndexError("transpose: %s -> %s" % (tuple(x.shape), tuple(out.shape)))
     call("pywrf_mlp_transpose", R, C, _vp(x), C, _vp(out), R, stream())
+
+
+def _ptrs(ts):
+    return (ctypes.c_void_p * len(ts))(*[t.data_ptr() if t is not None else None for t in ts])
+
+
+def _ints(xs):
+    return (ctypes.c_int * len(xs))(*xs)
+
+
+def transpose_group(pairs):
+    """transpose(x, out) for each (x, out) of up to 8 pairs, one launch."""
+    for x, out in pairs:
+        if tuple(out.shape) != (x.shape[1], x.shape[0]):
+            raise IndexError("transpose: %s -> %s" % (tuple(x.shape), tuple(out.shape)))
+    ins, outs = [x for x, _ in pairs], [o for _, o in pairs]
+    R, C = _ints([x.shape[0] for x in ins]), _ints([x.shape[1] for x in ins])
+    call("pywrf_mlp_transpose_group", len(pairs), R, C, _ptrs(ins), C, _ptrs(outs), R, stream())
+
+
+def rowsum_group(pairs):
+    """rowsum(x, out) for each (x, out) of up to 8 pairs, one launch."""
+    ins, outs = [x for x, _ in pairs], [o for _, o in pairs]
+    C = _ints([x.shape[1] for x in ins])
+    call("pywrf_mlp_rowsum_group", len(pairs), _ints([x.shape[0] for x in ins]), C, _ptrs(ins), C, _ptrs(outs), stream())
+
+
+def to_bf16(x, cols):
+    """BF16 rows [M x cols] of the FP32 matrix x [M x N], zero beyond its N columns."""
+    M, N = x.shape
+    if x.dtype != torch.float32 or x.stride(1) != 1 or x.stride(0) < N:
+        x = x.float().contiguous()
+    _lib._require_device(x)
+    out = torch.empty(M, cols, dtype=torch.bfloat16, device=x.device)
+    call("pywrf_mlp_to_bf16", M, N, _vp(x), x.stride(0), _vp(out), cols, stream())
+    return out
 
 
 def rowsum(x, out):
@@ -178,29 +215,24 @@ def backward(net, X, T, w, ws, wsum, ksplit=None):
     mean squared error sum_n w[n] (Y - T)^2 / (M wsum) of the forward pass
     just run on X (standardised targets T, FP32 [M x 288]; wsum = sum w)."""
     M = ws.M
-    ks = ksplit or max(1, min(64, M // 256))
-    ws.loss.zero_()
+    # splits of a weight gradient's sum over the batch: each adds its tiles with atomics, so no more than give half
+    # the CUs a workgroup (16 tiles of 128 x 128; 8192 columns: 26.8 us a product with 32 splits, 19.5 with 8)
+    ks = ksplit or max(1, min(8, M // 256))
+    zero_group([ws.loss, *ws.gW])
     call("pywrf_mlp_mse", M, FOUT, _vp(ws.Y), NO, _vp(T), NO, _vp(w), 1.0 / (M * wsum), _vp(ws.dY), NO,
          _vp(ws.loss), stream())
     # layer 3: dW3 = dY^T H2, db3 = sum dY, dH2 = (dY W3) [H2 > 0]
-    transpose(ws.dY, ws.dYt)
-    transpose(ws.H2, ws.H2t)
-    for g in ws.gW:
-        g.zero_()
+    transpose_group([(ws.dY, ws.dYt), (ws.H2, ws.H2t), (ws.H1, ws.H1t), (X, ws.Xt)])
     gemm(3, ws.dYt, ws.H2t, ws.gW[2], ksplit=ks)
-    rowsum(ws.dYt, ws.gb[2])
     gemm(2, ws.dY, net.Wt[2], ws.dH2, H=ws.H2)
     # layer 2
     transpose(ws.dH2, ws.dH2t)
-    transpose(ws.H1, ws.H1t)
     gemm(3, ws.dH2t, ws.H1t, ws.gW[1], ksplit=ks)
-    rowsum(ws.dH2t, ws.gb[1])
     gemm(2, ws.dH2, net.Wt[1], ws.dH1, H=ws.H1)
     # layer 1
     transpose(ws.dH1, ws.dH1t)
-    transpose(X, ws.Xt)
     gemm(3, ws.dH1t, ws.Xt, ws.gW[0], ksplit=ks)
-    rowsum(ws.dH1t, ws.gb[0])
+    rowsum_group([(ws.dYt, ws.gb[2]), (ws.dH2t, ws.gb[1]), (ws.dH1t, ws.gb[0])])
     return ws.loss
 
 
@@ -216,13 +248,12 @@ def loss_weights(device="cuda"):
 
 def adam_step(net, ws, lr, beta1=0.9, beta2=0.999, eps=1e-8):
     net.t += 1
-    for n in range(3):
-        W = net.W[n]
-        call("pywrf_mlp_adam", W.shape[0], W.shape[1], _vp(W), _vp(ws.gW[n]), _vp(net.mW[n]), _vp(net.vW[n]),
-             float(lr), beta1, beta2, eps, 1.0, net.t, _vp(net.Wb[n]), _vp(net.Wt[n]), stream())
-        b = net.b[n]
-        call("pywrf_mlp_adam", 1, b.shape[0], _vp(b), _vp(ws.gb[n]), _vp(net.mb[n]), _vp(net.vb[n]), float(lr),
-             beta1, beta2, eps, 1.0, net.t, None, None, stream())
+    W, g = [*net.W, *net.b], [*ws.gW, *ws.gb]
+    m, v = [*net.mW, *net.mb], [*net.vW, *net.vb]
+    none = [None] * len(net.b)
+    call("pywrf_mlp_adam_group", len(W), _ints([x.shape[0] if x.dim() == 2 else 1 for x in W]),
+         _ints([x.shape[-1] for x in W]), _ptrs(W), _ptrs(g), _ptrs(m), _ptrs(v), float(lr), beta1, beta2, eps, 1.0,
+         net.t, _ptrs([*net.Wb, *none]), _ptrs([*net.Wt, *none]), stream())
 
 
 # ----------------------------------------------------------------- data

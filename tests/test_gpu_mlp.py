@@ -148,3 +148,45 @@ def test_adam_matches_torch():
         assert _rel(mine, ref.detach()) < 1e-5
     assert torch.equal(net.Wb[1].cpu(), _bf(net.W[1].cpu()))
     assert torch.equal(net.Wt[2].cpu(), _bf(net.W[2].cpu()).t())
+
+
+@pytest.mark.parametrize("shapes", [[(64, 64)], [(8, 8), (72, 200), (300, 201), (129, 136)]])
+def test_grouped_calls_and_conversion(shapes):
+    """Matrices of aligned and ragged sides in one launch; FP32 rows of any
+    length (and any row stride) into padded BF16 rows: the same bits as torch."""
+    from pywrf_amd import surrogate as sg
+    gen = torch.Generator().manual_seed(len(shapes))
+    xs = [_bf(torch.randn(r, c, generator=gen)).cuda() for r, c in shapes]
+    ts = [torch.zeros(c, r, dtype=torch.bfloat16, device="cuda") for r, c in shapes]
+    sg.transpose_group(list(zip(xs, ts)))
+    rs = [torch.zeros(r, device="cuda") for r, _ in shapes]
+    sg.rowsum_group(list(zip(xs, rs)))
+    for x, t, r in zip(xs, ts, rs):
+        assert torch.equal(t.cpu(), x.cpu().t())
+        # FP32 sums of at most 256 values: c eps / 2 of the sum of magnitudes, far below this
+        assert float((r.cpu() - x.cpu().double().sum(1)).abs().max()) <= 1e-5 * float(x.cpu().double().abs().sum(1).max())
+    for N, cols in ((287, 288), (369, 384), (5, 8), (600, 640)):
+        x = torch.randn(7, N + 3, generator=gen).cuda()[:, :N]
+        for y in (x, x[:1].expand(7, N), x.t().contiguous().t()):
+            want = torch.zeros(7, cols, dtype=torch.bfloat16, device="cuda")
+            want[:, :N] = y.to(torch.bfloat16)
+            assert torch.equal(sg.to_bf16(y, cols), want)
+
+
+@pytest.mark.parametrize("N,ldy", [(287, 288), (7, 9), (1, 4)])
+def test_mse_rows_of_any_length(N, ldy):
+    from pywrf_amd import surrogate as sg
+    from pywrf_amd._lib import call, stream
+    gen = torch.Generator().manual_seed(N)
+    B = 700
+    Y, T = torch.randn(B, ldy, generator=gen).cuda(), torch.randn(B, ldy, generator=gen).cuda()
+    w = torch.rand(ldy, generator=gen).cuda()
+    dY = torch.full((B, ldy), 7.0, dtype=torch.bfloat16, device="cuda")
+    loss = torch.zeros(1, device="cuda")
+    call("pywrf_mlp_mse", B, N, sg._vp(Y), ldy, sg._vp(T), ldy, sg._vp(w), 0.01, sg._vp(dY), ldy, sg._vp(loss), stream())
+    d = (Y - T).double()[:, :N]
+    # positive terms, FP32 sums over at most B N / 256 of them a workgroup: a few hundred roundings
+    assert abs(float(loss) / float((w[:N] * d * d).sum() * 0.01) - 1) < 1e-5
+    want = (2.0 * w[:N] * (Y - T)[:, :N] * 0.01)
+    assert float((dY[:, :N].float() - want).abs().max()) <= 2 ** -8 * float(want.abs().max())
+    assert bool((dY[:, N:] == 0).all())
