@@ -298,6 +298,17 @@ int pywrf_advance_uv(const pywrf_grid_t* g, const float* u_in, const float* ru_t
                      const float* msfvx, const float* msfvx_inv, const float* msfvy, double rdx, double rdy,
                      double dts, const float* cf, const float* fnm, const float* fnp, double emdiv,
                      const float* rdnw, int spec_zone, float* u_out, float* v_out, pywrf_stream_t s);
+/* advance_uv, then spec_bdyupdate (wrf_boundary.py:228-284) of u with ru_tend and of v with rv_tend on grid gz
+ * with step zone_dt, in one launch. */
+int pywrf_advance_uv_zone(const pywrf_grid_t* g, const pywrf_grid_t* gz, const float* u_in,
+                          const float* ru_tend, const float* v_in, const float* rv_tend, const float* p,
+                          const float* pb, const float* ph, const float* php, const float* alt,
+                          const float* al, const float* mu, const float* muu, const float* cqu,
+                          const float* muv, const float* cqv, const float* mudf, const float* msfux,
+                          const float* msfuy, const float* msfvx, const float* msfvx_inv, const float* msfvy,
+                          double rdx, double rdy, double dts, const float* cf, const float* fnm,
+                          const float* fnp, double emdiv, const float* rdnw, int spec_zone, float* u_out,
+                          float* v_out, double zone_dt, pywrf_stream_t s);
 /* advance_mu_t, wrf_dynamics.py:3528-3638 (the seven *_out arrays fresh) */
 int pywrf_advance_mu_t(const pywrf_grid_t* g, const float* ww_in, const float* ww_1, const float* u,
                        const float* u_1, const float* v, const float* v_1, const float* mu_in, const float* mut,
@@ -308,6 +319,19 @@ int pywrf_advance_mu_t(const pywrf_grid_t* g, const float* ww_in, const float* w
                        const float* msfuy, const float* msfvx_inv, const float* msftx, const float* msfty,
                        float* ww_out, float* t_out, float* t_ave_out, float* muave_out, float* muts_out,
                        float* mudf_out, float* mu_out, pywrf_stream_t s);
+/* advance_mu_t, then spec_bdyupdate of t with ft (grid gz) and of mu and muts with mu_tend (grid gz2, 2-D) with
+ * step zone_dt, in one launch. */
+int pywrf_advance_mu_t_zone(const pywrf_grid_t* g, const pywrf_grid_t* gz, const pywrf_grid_t* gz2,
+                            const float* ww_in, const float* ww_1, const float* u, const float* u_1,
+                            const float* v, const float* v_1, const float* mu_in, const float* mut,
+                            const float* muave_in, const float* muts_in, const float* muu, const float* muv,
+                            const float* mudf_in, const float* t_in, const float* t_1, const float* t_ave_in,
+                            const float* ft, const float* mu_tend, double rdx, double rdy, double dts,
+                            double epssm, const float* dnw, const float* fnm, const float* fnp,
+                            const float* rdnw, const float* msfuy, const float* msfvx_inv, const float* msftx,
+                            const float* msfty, float* ww_out, float* t_out, float* t_ave_out,
+                            float* muave_out, float* muts_out, float* mudf_out, float* mu_out, double zone_dt,
+                            pywrf_stream_t s);
 /* advance_w, wrf_dynamics.py:3641-3796 (t_2ave_out, w_out, ph_out fresh) */
 int pywrf_advance_w(const pywrf_grid_t* g, const float* w_in, const float* rw_tend, const float* ww,
                     const float* w_save, const float* u, const float* v, const float* mut, const float* muave,
@@ -323,6 +347,15 @@ int pywrf_sumflux(const pywrf_grid_t* g, const float* ru, const float* rv, const
                   const float* v_lin, const float* ww_lin, const float* muu, const float* muv, float* ru_m,
                   float* rv_m, float* ww_m, const float* msfuy, const float* msfvx_inv, int iteration,
                   int number_of_small_timesteps, pywrf_stream_t s);
+/* sumflux, and on grid gz spec_bdyupdate_ph (ph) and zero_grad_bdy (zg_field), which touch none of its arrays,
+ * in one launch. */
+int pywrf_sumflux_zone(const pywrf_grid_t* g, const pywrf_grid_t* gz, const float* ru, const float* rv,
+                       const float* ww, const float* u_lin, const float* v_lin, const float* ww_lin,
+                       const float* muu, const float* muv, float* ru_m, float* rv_m, float* ww_m,
+                       const float* msfuy, const float* msfvx_inv, int iteration,
+                       int number_of_small_timesteps, const float* ph_save, float* ph, const float* ph_tend,
+                       const float* mu_tend, const float* muts, double dt, char variable_in, float* zg_field,
+                       char zg_variable, pywrf_stream_t s);
 /* calc_mu_uv_1, wrf_dynamics.py:3844-3860 */
 int pywrf_calc_mu_uv_1(const pywrf_grid_t* g, const float* mu, float* muu, float* muv, pywrf_stream_t s);
 /* small_step_finish, wrf_dynamics.py:3863-3930 (u..t_out fresh; ww, mu_2 in place) */

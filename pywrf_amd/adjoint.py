@@ -700,6 +700,10 @@ SUBSTEP_CALLS = ("advance_uv", "spec_bdyupdate_group", "advance_mu_t", "spec_bdy
                  "sumflux", "spec_bdyupdate_ph_zero_grad", "calc_p_rho", "set_physical_bc_group")
 
 
+# calls that merge several of the recorded ones; a recorder does not offer them, so the step makes each call itself
+MERGED = frozenset(("advance_uv_zone", "advance_mu_t_zone", "sumflux_zone"))
+
+
 class _LoopRecorder:
     """The step's functions, keeping copies of the arguments of every call of
     the acoustic loop that starts at the n-th call of advance_uv, up to the
@@ -717,6 +721,8 @@ class _LoopRecorder:
         return a
 
     def __getattr__(self, name):
+        if name in MERGED:
+            raise AttributeError(name)
         f = getattr(self._ops, name)
 
         def rec(*args):
@@ -824,6 +830,8 @@ class _StageRecorder(_LoopRecorder):
     from the n-th small_step_prep through the next small_step_finish."""
 
     def __getattr__(self, name):
+        if name in MERGED:
+            raise AttributeError(name)
         f = getattr(self._ops, name)
 
         def rec(*args):

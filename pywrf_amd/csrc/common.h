@@ -99,10 +99,8 @@ __host__ __device__ inline long edge_count(const Box& b, int w) {
   return 2L * w * b.ni() + 2L * w * (b.nj() - 2 * w);
 }
 
-__device__ inline bool edge_point(const Box& b, int w, int& k, int& j, int& i) {
-  if (w == 0) return box_point(b, k, j, i);
-  int t = (int)(blockIdx.x * PW_EDGE_BLOCK + threadIdx.x);
-  k = b.k0 + (int)blockIdx.z;
+// the t-th point of a level's band
+__device__ inline bool edge_at(const Box& b, int w, int t, int& j, int& i) {
   const int ni = b.ni(), nj = b.nj(), rows = w * ni, h = nj - 2 * w;
   if (t < rows) { j = b.j0 + t / ni; i = b.i0 + t % ni; return true; }
   t -= rows;
@@ -112,6 +110,12 @@ __device__ inline bool edge_point(const Box& b, int w, int& k, int& j, int& i) {
   t -= w * h;
   if (t < w * h) { j = b.j0 + w + t / w; i = b.i1 - w + t % w; return true; }
   return false;
+}
+
+__device__ inline bool edge_point(const Box& b, int w, int& k, int& j, int& i) {
+  if (w == 0) return box_point(b, k, j, i);
+  k = b.k0 + (int)blockIdx.z;
+  return edge_at(b, w, (int)(blockIdx.x * PW_EDGE_BLOCK + threadIdx.x), j, i);
 }
 
 template <class Kern, class... Args>

@@ -177,6 +177,9 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
     bc2 = lambda a, v: o.set_physical_bc2d(a, v, *I2)
     grouped = hasattr(o, "set_physical_bc_group")
     grouped_upd = hasattr(o, "spec_bdyupdate_group")
+    # the forms that merge several calls: where the launch itself counts (a graph's node is about 5 us), and only
+    # there, so that a step made call by call keeps the calls that a caller may replace or record
+    merged = clock is not None and hasattr(o, "advance_uv_zone")
 
     def bcs(*items):
         """A run of consecutive open-boundary fills, items (tensor, flag, is_2d);
@@ -386,24 +389,29 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
                  its, ite, jts, jte, 0, 0)
         # acoustic small steps (solver.py:1349-1493)
         for iteration in range(1, nsmall + 1):
-            s.u, s.v = o.advance_uv(s.u, s.ru_tend, s.v, s.rv_tend, s.p, s.pb, s.ph, s.php, s.alt, s.al, s.mu,
-                                    s.muu, s.cqu, s.muv, s.cqv, s.mudf, s.c1h, s.c2h, s.c1f, s.c2f, s.c3h, s.c4h,
-                                    s.c3f, s.c4f, s.msfux, s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, rdx, rdy, dts_rk,
-                                    s.cf1, s.cf2, s.cf3, s.fnm, s.fnp, EMDIV, s.rdnw, SPEC_ZONE, True, False, *I18)
-            if grouped_upd:
-                o.spec_bdyupdate_group([(s.u, s.ru_tend, 'u', 0), (s.v, s.rv_tend, 'v', 0)], dts_rk, I24, ix_2d)
+            uv_args = (s.u, s.ru_tend, s.v, s.rv_tend, s.p, s.pb, s.ph, s.php, s.alt, s.al, s.mu, s.muu, s.cqu, s.muv,
+                       s.cqv, s.mudf, s.c1h, s.c2h, s.c1f, s.c2f, s.c3h, s.c4h, s.c3f, s.c4f, s.msfux, s.msfuy,
+                       s.msfvx, s.msfvx_inv, s.msfvy, rdx, rdy, dts_rk, s.cf1, s.cf2, s.cf3, s.fnm, s.fnp, EMDIV,
+                       s.rdnw, SPEC_ZONE, True, False, *I18)
+            if merged:
+                s.u, s.v = o.advance_uv_zone(uv_args, dts_rk, I24)
             else:
-                s.u = o.spec_bdyupdate(s.u, s.ru_tend, dts_rk, 'u', SPEC_ZONE, *I24)
-                s.v = o.spec_bdyupdate(s.v, s.rv_tend, dts_rk, 'v', SPEC_ZONE, *I24)
-            (s.ww, s.ww1, s.t, s.t_2save, s.ru_m, s.rv_m, s.ww_m, s.muave, s.muts, s.mudf, s.mu) = o.advance_mu_t(
-                s.ww, s.ww1, s.u, s.u_save, s.v, s.v_save, s.mu, s.mut, s.muave, s.muts, s.muu, s.muv, s.mudf,
-                s.c1h, s.c2h, s.c1f, s.c2f, s.c3h, s.c4h, s.c3f, s.c4f, s.ru_m, s.rv_m, s.ww_m, s.t, s.t_save,
-                s.t_2save, s.t_tend, s.mu_tend, rdx, rdy, dts_rk, EPSSM, s.dnw, s.fnm, s.fnp, s.rdnw, s.msfux,
-                s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.msftx, s.msfty, iteration, *I18)
-            if grouped_upd:
+                s.u, s.v = o.advance_uv(*uv_args)
+                if grouped_upd:
+                    o.spec_bdyupdate_group([(s.u, s.ru_tend, 'u', 0), (s.v, s.rv_tend, 'v', 0)], dts_rk, I24, ix_2d)
+                else:
+                    s.u = o.spec_bdyupdate(s.u, s.ru_tend, dts_rk, 'u', SPEC_ZONE, *I24)
+                    s.v = o.spec_bdyupdate(s.v, s.rv_tend, dts_rk, 'v', SPEC_ZONE, *I24)
+            mt_args = (s.ww, s.ww1, s.u, s.u_save, s.v, s.v_save, s.mu, s.mut, s.muave, s.muts, s.muu, s.muv, s.mudf,
+                       s.c1h, s.c2h, s.c1f, s.c2f, s.c3h, s.c4h, s.c3f, s.c4f, s.ru_m, s.rv_m, s.ww_m, s.t, s.t_save,
+                       s.t_2save, s.t_tend, s.mu_tend, rdx, rdy, dts_rk, EPSSM, s.dnw, s.fnm, s.fnp, s.rdnw, s.msfux,
+                       s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.msftx, s.msfty, iteration, *I18)
+            (s.ww, s.ww1, s.t, s.t_2save, s.ru_m, s.rv_m, s.ww_m, s.muave, s.muts, s.mudf, s.mu) = (
+                o.advance_mu_t_zone(mt_args, dts_rk, I24, ix_2d) if merged else o.advance_mu_t(*mt_args))
+            if not merged and grouped_upd:
                 o.spec_bdyupdate_group([(s.t, s.t_tend, 't', 0), (s.mu, s.mu_tend, 'm', 1),
                                         (s.muts, s.mu_tend, 'm', 1)], dts_rk, I24, ix_2d)
-            else:
+            elif not merged:
                 s.t = o.spec_bdyupdate(s.t, s.t_tend, dts_rk, 't', SPEC_ZONE, *I24)
                 s.mu = o.spec_bdyupdate(s.mu, s.mu_tend, dts_rk, 'm', SPEC_ZONE, *ix_2d)
                 s.muts = o.spec_bdyupdate(s.muts, s.mu_tend, dts_rk, 'm', SPEC_ZONE, *ix_2d)
@@ -412,16 +420,20 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
                 s.c3h, s.c4h, s.c3f, s.c4f, s.t_2save, s.t, s.t_save, s.ph, s.ph_save, s.phb, s.ph_tend, s.ht, s.c2a,
                 s.cqw, s.alt, s.alb, s.a, s.alpha, s.gamma, rdx, rdy, dts_rk, T0, EPSSM, s.dnw, s.fnm, s.fnp, s.rdnw,
                 s.rdn, s.cf1, s.cf2, s.cf3, s.msftx, s.msfty, False, *I18)
-            s.ru_m, s.rv_m, s.ww_m = o.sumflux(s.u, s.v, s.ww, s.u_save, s.v_save, s.ww1, s.muu, s.muv, s.c1h, s.c2h,
-                                               s.c1f, s.c2f, s.c3h, s.c4h, s.c3f, s.c4f, s.ru_m, s.rv_m, s.ww_m, EPSSM,
-                                               s.msfux, s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, iteration, nsmall,
-                                               *I18)
+            sf_args = (s.u, s.v, s.ww, s.u_save, s.v_save, s.ww1, s.muu, s.muv, s.c1h, s.c2h, s.c1f, s.c2f, s.c3h, s.c4h,
+                       s.c3f, s.c4f, s.ru_m, s.rv_m, s.ww_m, EPSSM, s.msfux, s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy,
+                       iteration, nsmall, *I18)
             ph_args = (s.ph_save, s.ph, s.ph_tend, s.mu_tend, s.muts, s.c1f, s.c2f, dts_rk, 'h', SPEC_ZONE, *I24)
-            if hasattr(o, "spec_bdyupdate_ph_zero_grad"):
-                s.ph, s.w = o.spec_bdyupdate_ph_zero_grad(ph_args, (s.w, 'w', SPEC_ZONE, *I24))
+            zg_args = (s.w, 'w', SPEC_ZONE, *I24)
+            if merged:
+                (s.ru_m, s.rv_m, s.ww_m), s.ph, s.w = o.sumflux_zone(sf_args, ph_args, zg_args)
             else:
-                s.ph = o.spec_bdyupdate_ph(*ph_args)
-                s.w = o.zero_grad_bdy(s.w, 'w', SPEC_ZONE, *I24)
+                s.ru_m, s.rv_m, s.ww_m = o.sumflux(*sf_args)
+                if hasattr(o, "spec_bdyupdate_ph_zero_grad"):
+                    s.ph, s.w = o.spec_bdyupdate_ph_zero_grad(ph_args, zg_args)
+                else:
+                    s.ph = o.spec_bdyupdate_ph(*ph_args)
+                    s.w = o.zero_grad_bdy(*zg_args)
             s.al, s.p, s.pm1 = cpr(iteration)
             s.ph, s.al, s.p, s.muts, s.mu, s.mudf = bcs((s.ph, 'w', 0), (s.al, 'p', 0), (s.p, 'p', 0),
                                                         (s.muts, 't', 1), (s.mu, 't', 1), (s.mudf, 't', 1))

@@ -783,6 +783,24 @@ def advance_uv(u_ori, ru_tend, v_ori, rv_tend,
     return u, v
 
 
+def advance_uv_zone(uv_args, dt, idx24):
+    """advance_uv (uv_args: its positional arguments), then spec_bdyupdate
+    (wrf_boundary.py:228-284) of u with ru_tend and of v with rv_tend, step dt
+    and index set idx24, in one launch.  Same result as the three calls.  Not
+    part of the reference API."""
+    (u_ori, ru_tend, v_ori, rv_tend, p, pb, ph, php, alt, al, mu, muu, cqu, muv, cqv, mudf, _, _, _, _, _, _, _, _,
+     msfux, msfuy, msfvx, msfvx_inv, msfvy, rdx, rdy, dts, cf1, cf2, cf3, fnm, fnp, emdiv, rdnw, spec_zone, _, _,
+     *ix) = uv_args
+    g, gz = grid(u_ori.shape, tuple(ix)), grid(u_ori.shape, tuple(idx24))
+    cf, _keep = _cf(cf1, cf2, cf3)
+    u, v = fresh(u_ori), fresh(v_ori)
+    call("pywrf_advance_uv_zone", g, gz, ptr(u_ori), ptr(ru_tend), ptr(v_ori), ptr(rv_tend), ptr(p), ptr(pb), ptr(ph),
+         ptr(php), ptr(alt), ptr(al), ptr(mu), ptr(muu), ptr(cqu), ptr(muv), ptr(cqv), ptr(mudf), ptr(msfux),
+         ptr(msfuy), ptr(msfvx), ptr(msfvx_inv), ptr(msfvy), float(rdx), float(rdy), float(dts), cf, ptr(fnm),
+         ptr(fnp), float(emdiv), ptr(rdnw), int(spec_zone), ptr(u), ptr(v), float(dt), stream())
+    return u, v
+
+
 def advance_mu_t(ww_ori, ww_1, u, u_1, v, v_1,
                  mu_ori, mut, muave_ori, muts_ori, muu, muv, mudf_ori,
                  c1h, c2h, c1f, c2f,
@@ -807,6 +825,25 @@ def advance_mu_t(ww_ori, ww_1, u, u_1, v, v_1,
          ptr(ft), ptr(mu_tend), float(rdx), float(rdy), float(dts), float(epssm), ptr(dnw), ptr(fnm), ptr(fnp),
          ptr(rdnw), ptr(msfuy), ptr(msfvx_inv), ptr(msftx), ptr(msfty), ptr(ww), ptr(t), ptr(t_ave), ptr(muave),
          ptr(muts), ptr(mudf), ptr(mu), stream())
+    return ww, ww_1, t, t_ave, uam, vam, wwam, muave, muts, mudf, mu
+
+
+def advance_mu_t_zone(mt_args, dt, idx24, idx2d):
+    """advance_mu_t (mt_args: its positional arguments), then spec_bdyupdate of
+    t with ft (index set idx24) and of mu and muts with mu_tend (idx2d, with
+    kds = kde = 0), step dt, in one launch.  Same result as the four calls.
+    Not part of the reference API."""
+    (ww_ori, ww_1, u, u_1, v, v_1, mu_ori, mut, muave_ori, muts_ori, muu, muv, mudf_ori, _, _, _, _, _, _, _, _,
+     uam, vam, wwam, t_ori, t_1, t_ave_ori, ft, mu_tend, rdx, rdy, dts, epssm, dnw, fnm, fnp, rdnw, msfux, msfuy, msfvx,
+     msfvx_inv, msfvy, msftx, msfty, step, *ix) = mt_args
+    g, gz, gz2 = grid(u.shape, tuple(ix)), grid(u.shape, tuple(idx24)), grid(mu_ori.shape, tuple(idx2d))
+    ww, t, t_ave = fresh(ww_ori), fresh(t_ori), fresh(t_ave_ori)
+    muave, muts, mudf, mu = fresh(muave_ori), fresh(muts_ori), fresh(mudf_ori), fresh(mu_ori)
+    call("pywrf_advance_mu_t_zone", g, gz, gz2, ptr(ww_ori), ptr(ww_1), ptr(u), ptr(u_1), ptr(v), ptr(v_1), ptr(mu_ori),
+         ptr(mut), ptr(muave_ori), ptr(muts_ori), ptr(muu), ptr(muv), ptr(mudf_ori), ptr(t_ori), ptr(t_1),
+         ptr(t_ave_ori), ptr(ft), ptr(mu_tend), float(rdx), float(rdy), float(dts), float(epssm), ptr(dnw), ptr(fnm),
+         ptr(fnp), ptr(rdnw), ptr(msfuy), ptr(msfvx_inv), ptr(msftx), ptr(msfty), ptr(ww), ptr(t), ptr(t_ave),
+         ptr(muave), ptr(muts), ptr(mudf), ptr(mu), float(dt), stream())
     return ww, ww_1, t, t_ave, uam, vam, wwam, muave, muts, mudf, mu
 
 
@@ -854,6 +891,26 @@ def sumflux(ru, rv, ww,
          ptr(ru_m), ptr(rv_m), ptr(ww_m), ptr(msfuy), ptr(msfvx_inv), int(iteration), int(number_of_small_timesteps),
          stream())
     return ru_m, rv_m, ww_m
+
+
+def sumflux_zone(sf_args, ph_args, zg_args):
+    """sumflux, then spec_bdyupdate_ph and zero_grad_bdy (wrf_boundary.py:287-405)
+    on two arrays that sumflux does not touch, each given as the tuple of its
+    positional arguments, in one launch; the last two share their index set
+    and zone.  Returns the three calls' results.  Not part of the reference
+    API."""
+    (ru, rv, ww, u_lin, v_lin, ww_lin, muu, muv, _, _, _, _, _, _, _, _, ru_m, rv_m, ww_m, epssm, msfux, msfuy, msfvx,
+     msfvx_inv, msfvy, iteration, nsmall, *ix) = sf_args
+    (ph_save, field, field_tend, mu_tend, muts, _, _, dt, variable_in, spec_zone, *pix) = ph_args
+    (zg_field, zg_variable, zg_zone, *zix) = zg_args
+    if tuple(pix) != tuple(zix) or spec_zone != zg_zone:
+        raise ValueError("sumflux_zone: the boundary calls must share the index set and zone")
+    g, gz = grid(ru.shape, tuple(ix)), grid(ru.shape, tuple(pix))
+    call("pywrf_sumflux_zone", g, gz, ptr(ru), ptr(rv), ptr(ww), ptr(u_lin), ptr(v_lin), ptr(ww_lin), ptr(muu), ptr(muv),
+         ptr(ru_m), ptr(rv_m), ptr(ww_m), ptr(msfuy), ptr(msfvx_inv), int(iteration), int(nsmall), ptr(ph_save),
+         ptr(field), ptr(field_tend), ptr(mu_tend), ptr(muts), float(dt), flag(variable_in), ptr(zg_field),
+         flag(zg_variable), stream())
+    return (ru_m, rv_m, ww_m), field, zg_field
 
 
 def calc_mu_uv_1(mu, muu, muv,
