@@ -382,20 +382,36 @@ extern "C" int pywrf_spec_bdyupdate_ph_zero_grad(const pywrf_grid_t* g, const fl
 // is scaled by r per application, and muts's gathers, down the column, the
 // derivative of f' with respect to muts, carried through the applications in
 // forward mode, and so do those of mu_tend (through r) and of ft (dt / muts
-// per application).  One thread per column of the band; lam holds f''s
+// per application).  16 columns of the band to a block, 32 threads to a column
+// (levels g, g + 32, ...): the band of a 120 x 120 plane is 480 columns, too few
+// to hide a walk of the levels (10 us,
+// 43 with one thread a column); lam holds f''s
 // sensitivity on entry and f's on return; lam_muts and lam_mu_tend are
 // written on the band's columns only, lam_ft on the strips' points only.
-__global__ void k_spec_bdyupdate_ph_adj(Box cols, Dims D, PhStrip a, const float* f_in, float* lam,
-                                        float* lam_muts, float* lam_ft, float* lam_mu_tend, float* lam_ph_save) {
-  int j, i;
-  if (!box_column(cols, j, i)) return;
+#define PA_COLS 16
+#define PA_RUNS 32
+__global__ void __launch_bounds__(PA_COLS * PA_RUNS)
+    k_spec_bdyupdate_ph_adj(Box cols, Dims D, PhStrip a, const float* f_in, float* lam, float* lam_muts, float* lam_ft,
+                            float* lam_mu_tend, float* lam_ph_save) {
+  __shared__ float s_m[PA_RUNS][PA_COLS], s_t[PA_RUNS][PA_COLS];
+  const int lane = threadIdx.x % PA_COLS, g = (int)threadIdx.x / PA_COLS;
+  int j = 0, i = 0;
+  const int c = (int)blockIdx.x * PA_COLS + lane;
+  bool col;
+  if (a.w == 1) {
+    col = edge_at(cols, 1, c, j, i);
+  } else {
+    j = cols.j0 + c / cols.ni(); i = cols.i0 + c % cols.ni();
+    col = j < cols.j1;
+  }
   bool ir = i >= a.ibs && i < a.ibe, jc = j >= a.jbs + 1 && j < a.jbe - 1;
   int n = (j == a.jts && ir) + (j == a.jbe - 1 && ir) + (i == a.ibs && jc) + (i == a.ibe - 1 && jc);
-  if (!n) return;
+  if (!col) n = 0;
+  if (!n) { j = cols.j0; i = cols.i0; }   // a lane without a column: reads, adds and stores nothing below
   const float mt = AT2(a.muts, j, i), mtend = AT2(a.mu_tend, j, i);
   const float mo = mt - a.dt * mtend, r = mo / mt, dr = a.dt * mtend / (mt * mt), drt = -a.dt / mt;
   float gm = 0.0f, gt = 0.0f;
-  for (int k = a.all.k0; k < a.all.k1; ++k) {
+  for (int k = a.all.k0 + g; k < (n ? a.all.k1 : 0); k += PA_RUNS) {
     const long q = D.ix(k, j, i);
     const float ft = a.ft[q], ps = a.ph_save[q];
     const float dc = -a.dt * ft / (mt * mt) + ps * dr;
@@ -415,6 +431,11 @@ __global__ void k_spec_bdyupdate_ph_adj(Box cols, Dims D, PhStrip a, const float
     if (lam_ph_save) lam_ph_save[q] = l * dps;
     lam[q] = l * s;
   }
+  s_m[g][lane] = gm;
+  s_t[g][lane] = gt;
+  __syncthreads();
+  if (g != 0 || !n) return;
+  for (int w = 1; w < PA_RUNS; ++w) { gm += s_m[w][lane]; gt += s_t[w][lane]; }
   AT2(lam_muts, j, i) = gm;
   AT2(lam_mu_tend, j, i) = gt;
 }
@@ -427,8 +448,12 @@ extern "C" int pywrf_spec_bdyupdate_ph_adjoint(const pywrf_grid_t* g, const floa
   PhStrip a;
   if (int e = ph_strip_setup(g, ph_save, nullptr, field_tend, mu_tend, muts, dt, variable_in, a)) return e;
   Box cols = mkbox(0, 1, a.all.j0, a.all.j1, a.all.i0, a.all.i1);
-  PW_LAUNCH_COLS(k_spec_bdyupdate_ph_adj, cols, s, dims_of(g), a, field_in, lam_field, lam_muts, lam_field_tend,
-                 lam_mu_tend, lam_ph_save);
+  if (2 > cols.nj() || 2 > cols.ni()) a.w = 0;   // no band in so small a box: all its columns
+  const long nc = cols.nj() > 0 && cols.ni() > 0 ? (a.w == 1 ? edge_count(cols, 1) : (long)cols.nj() * cols.ni()) : 0;
+  if (nc > 0)
+    hipLaunchKernelGGL(k_spec_bdyupdate_ph_adj, dim3((unsigned)((nc + PA_COLS - 1) / PA_COLS)), dim3(PA_COLS * PA_RUNS), 0,
+                       (hipStream_t)s, cols, dims_of(g), a, field_in, lam_field, lam_muts, lam_field_tend, lam_mu_tend,
+                       lam_ph_save);
   PW_RET();
 }
 

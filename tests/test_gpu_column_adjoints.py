@@ -1,0 +1,56 @@
+"""The column adjoints (64 columns of a row to a block, the levels dealt out to
+its waves) at plane sizes around a block's 63 and 64 columns, against the same
+FP64 oracle gradients as at the stock sizes, and with level arrays kept in LDS
+and, beyond what it holds, in memory."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+import test_gpu_adjoint as stock
+from pywrf_amd.gen import CONFIGS
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [62, 63, 65])
+@pytest.mark.parametrize("which", ["advance_w", "advance_uv", "advance_mu_t"])
+def test_column_adjoints_around_a_block(which, n):
+    fn = {"advance_w": stock.test_advance_w_adjoint_matches_oracle_autograd,
+          "advance_uv": stock.test_advance_uv_adjoint_matches_oracle_autograd,
+          "advance_mu_t": stock.test_advance_mu_t_adjoint_matches_oracle_differences}[which]
+    fn(dict(CONFIGS["bdy24"], n=n))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nz", [58, 59, 64])
+def test_advance_w_adjoint_is_the_same_from_lds_and_memory(nz):
+    """Levels above the model's top (index set unchanged) change nothing at
+    and below it, whichever place the level arrays take."""
+    import pywrf_amd
+    from pywrf_amd import adjoint
+    from pywrf_amd.gen import synthetic_state
+    from pywrf_amd.step import RunConfig, rk3_step
+    s = synthetic_state("bdy24", device="cuda")
+    rec = stock._FirstCall(pywrf_amd.ops(), "advance_w")
+    rk3_step(s, rec, RunConfig())
+    nz0 = s.w.shape[0]
+
+    def padded(a):
+        if not isinstance(a, torch.Tensor) or a.dim() not in (1, 3) or a.shape[0] != nz0:
+            return a
+        out = torch.ones((nz,) + tuple(a.shape[1:]), device=a.device)
+        out[:nz0] = a
+        return out
+
+    D = adjoint.AdvanceW.DIFF + adjoint.AdvanceW.EXTRA
+    from pywrf_amd import wrf_dynamics
+    outs = wrf_dynamics.advance_w(*rec.args)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    lams = [torch.randn(s.w.shape, device="cuda", generator=gen) for _ in outs]
+    grads = []
+    for pad in (lambda a: a, padded):             # the forward takes fewer levels: the backward by itself
+        ctx = SimpleNamespace(args=[pad(a) for a in rec.args], outs=[pad(o) for o in outs[:2]],
+                              needs_input_grad=(True,) * (len(D) + 1))
+        grads.append(adjoint.AdvanceW.backward(ctx, *[pad(l) for l in lams]))
+    for n, a, b in zip(range(len(D) + 1), *grads):
+        assert (a is None and b is None) or torch.equal(a, b[:nz0] if b.dim() == 3 else b), n
