@@ -80,6 +80,11 @@ int pywrf_set_physical_bc3d(const pywrf_grid_t* g, float* dat, char variable, py
 int pywrf_set_physical_bc_group(const pywrf_grid_t* g3, const pywrf_grid_t* g2, int n, void* const* fields,
                                 const char* variables, const int* is2d, pywrf_stream_t s);
 
+/* For each of n jobs f (at most 16): dst[f][q] = src[4 f][q] + src[4 f + 1][q] + ... over its leading non-null
+   sources (one to four), q < counts[f], added in that order, in one launch.  A destination may be one of its own
+   job's sources, and no other job's source or destination. */
+int pywrf_sum_group(int n, void* const* dst, void* const* src, const long long* counts, pywrf_stream_t s);
+
 /* Zero n distinct device arrays of counts[f] floats each in one launch: the
  * runs of tensor.zero_() calls of the reference driver (solver.py:848-851,
  * 975-981).  No counterpart in the reference API: a batching of zero_(). */

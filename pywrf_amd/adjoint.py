@@ -74,6 +74,25 @@ def _f32(t):
     return t.contiguous()
 
 
+def _sums(*jobs):
+    """dst = the sum of its sources, in order, for jobs (dst, sources) of up to
+    four sources each, in one launch; dst may be one of its own sources."""
+    import ctypes
+    n = len(jobs)
+    dst = (ctypes.c_void_p * n)(*[ptr(d).value for d, _ in jobs])
+    srcs = [(list(s) + [None] * 4)[:4] for _, s in jobs]
+    src = (ctypes.c_void_p * (4 * n))(*[None if t is None else ptr(t).value for q in srcs for t in q])
+    counts = (ctypes.c_longlong * n)(*[d.numel() for d, _ in jobs])
+    call("pywrf_sum_group", n, dst, src, counts, stream())
+
+
+def _copies(*tensors):
+    """A copy of each tensor, in one launch."""
+    out = [torch.empty_like(t) for t in tensors]
+    _sums(*[(o, (t,)) for o, t in zip(out, tensors)])
+    return out
+
+
 # ----------------------------------------------------------------------- advection
 def advect_scalar_tendency(field, ru, rv, rom, msftx, fzm, fzp, rdx, rdy, rdzw, idx):
     """The tendency advect_scalar adds to a zeroed array (HIP)."""
@@ -780,43 +799,200 @@ def loop_saved(substeps):
     return [mt[3], mt[5], wa[3], mt[25], wa[22], mt[1]]
 
 
+class AcousticSubstep(torch.autograd.Function):
+    """One acoustic substep (solver.py:1349-1493): advance_uv, the u/v zone
+    update, advance_mu_t, the t/mu/muts zone update, advance_w, sumflux,
+    spec_bdyupdate_ph, zero_grad_bdy, calc_p_rho and the six open-boundary
+    fills, and their adjoints in the opposite order, as one node.  The calls
+    that work in place do so on arrays the substep made itself: what they
+    change (the zone's ring, the halos) is not what the adjoints of the calls
+    before them read, except f_in of spec_bdyupdate_ph, which is kept.  A node
+    per call cost a copy of every such array and an addition for every value
+    that two calls read: 555 launches for a stage of four substeps, forward
+    twice and backward, against 291 (at 120 x 120 x 41 8.8 against 6.1 ms,
+    most of it the host's).
+
+    calls: the nine recorded calls' arguments; given, saved: whether the six
+    tendencies (FORCING order) and the six saved fields (SAVED order) follow
+    the 17 carried fields among the inputs; where not, the recorded ones are
+    used and held fixed."""
+
+    @staticmethod
+    def forward(ctx, calls, given, saved, *inputs):
+        from . import wrf_boundary, wrf_dynamics
+        inputs = [_f32(t) for t in inputs]
+        st = dict(zip(ACOUSTIC_STATE, inputs))
+        uv, z1, mt, z2, wa, sf, pz, cp, bc = [list(c) for c in calls]
+        ph_args, zg_args = list(pz[0]), list(pz[1])
+        n = len(ACOUSTIC_STATE)
+        tends = [it[1] for it in z1[0]] + [it[1] for it in z2[0]]
+        if given:
+            fc = dict(zip(FORCING, inputs[n:]))
+            n += len(FORCING)
+            uv[1], uv[3], mt[27], mt[28] = fc["ru_tend"], fc["rv_tend"], fc["t_tend"], fc["mu_tend"]
+            wa[AdvanceW.RWT], wa[AdvanceW.PHT] = fc["rw_tend"], fc["ph_tend"]
+            ph_args[2], ph_args[3] = fc["ph_tend"], fc["mu_tend"]
+            tends = [fc[k] for k in ("ru_tend", "rv_tend", "t_tend", "mu_tend", "mu_tend")]
+        if saved:
+            sv = dict(zip(SAVED, inputs[n:]))
+            mt[3], mt[5], mt[1], mt[25] = sv["u_save"], sv["v_save"], sv["ww1"], sv["t_save"]
+            wa[AdvanceW.WSAVE], wa[AdvanceW.T1], wa[AdvanceW.PH1] = sv["w_save"], sv["t_save"], sv["ph_save"]
+            sf[3], sf[4], sf[5] = sv["u_save"], sv["v_save"], sv["ww1"]
+            ph_args[0] = sv["ph_save"]
+            cp[5] = sv["t_save"]
+
+        def put(args, places, values):
+            for pos, t in zip(places, values):
+                args[pos] = t
+
+        def zone(call, fields, tends):
+            items, dt, ix24, ix2d = call
+            wrf_boundary.spec_bdyupdate_group([(f, t, it[2], it[3]) for f, t, it in zip(fields, tends, items)], dt,
+                                              ix24, ix2d)
+
+        put(uv, (0, 2, 4, 6, 9, 10, 15), [st[k] for k in ("u", "v", "p", "ph", "al", "mu", "mudf")])
+        u, v = wrf_dynamics.advance_uv(*uv)
+        zone(z1, (u, v), tends[:2])
+        put(mt, (2, 4, 0, 6, 8, 9, 12, 24, 26),
+            [u, v] + [st[k] for k in ("ww", "mu", "muave", "muts", "mudf", "t", "t_ave")])
+        r = wrf_dynamics.advance_mu_t(*mt)
+        ww, t, t_ave, muave, muts, mudf, mu = [r[k] for k in AdvanceMuT.OUT]
+        zone(z2, (t, mu, muts), tends[2:])
+        put(wa, AdvanceW.DIFF, (st["w"], st["ph"], t, t_ave, u, v, muts, muave, ww))
+        t2a, w, ph = wrf_dynamics.advance_w(*wa)
+        f_in, pm1, ru_m, rv_m, ww_m = _copies(ph, st["pm1"], st["ru_m"], st["rv_m"], st["ww_m"])
+        put(sf, SumFlux.DIFF, (u, v, ww, ru_m, rv_m, ww_m))
+        wrf_dynamics.sumflux(*sf)
+        ph_args[1], ph_args[4], zg_args[0] = ph, muts, w
+        if tuple(ph_args[10:]) == tuple(zg_args[3:]) and ph_args[9] == zg_args[2]:
+            wrf_boundary.spec_bdyupdate_ph_zero_grad(tuple(ph_args), tuple(zg_args))
+        else:
+            wrf_boundary.spec_bdyupdate_ph(*ph_args)
+            wrf_boundary.zero_grad_bdy(*zg_args)
+        put(cp, CalcPRho.DIFF, (st["al"], st["p"], ph, t, pm1, mu, muts))
+        al, p, pm1 = wrf_dynamics.calc_p_rho(*cp)
+        items, ix24, ix2d = bc
+        kinds = [(k, two) for _, k, two in items]
+        wrf_dynamics.set_physical_bc_group([(f, k, two) for f, (k, two) in zip((ph, al, p, muts, mu, mudf), kinds)],
+                                           ix24, ix2d)
+        ctx.calls = uv, z1, mt, z2, wa, sf, ph_args, zg_args, cp, (kinds, ix24, ix2d)
+        ctx.kept = ww, t2a, w, f_in, tends
+        ctx.given, ctx.saved = given, saved
+        ctx.set_materialize_grads(False)
+        new = {"u": u, "v": v, "p": p, "ph": ph, "al": al, "mu": mu, "mudf": mudf, "ww": ww, "muave": muave,
+               "muts": muts, "t": t, "t_ave": t2a, "w": w, "pm1": pm1, "ru_m": ru_m, "rv_m": rv_m, "ww_m": ww_m}
+        # aliases: the results get a grad_fn, and what ctx holds must not lead back to it
+        return tuple(new[k].detach() for k in ACOUSTIC_STATE)
+
+    @staticmethod
+    def backward(ctx, *lams):
+        import ctypes
+        from .wrf_dynamics import _cf, zero_group
+        from . import wrf_boundary
+        uv, z1, mt, z2, wa, sf, pz, zg, cp, (kinds, ix24, ix2d) = ctx.calls
+        ww, t2a_out, w_out, f_in, tends = ctx.kept
+        big, flat = uv[0], mt[9]                     # a 3-D field and a plane
+        none = [n for n, l in zip(ACOUSTIC_STATE, lams) if l is None]
+        L = {n: _f32(l) for n, l in zip(ACOUSTIC_STATE, lams) if l is not None}
+        for n in none:
+            L[n] = torch.zeros_like(flat if n in ("mu", "mudf", "muave", "muts") else big)
+        e3 = lambda n: [torch.empty_like(big) for _ in range(n)]
+        e2 = lambda n: [torch.empty_like(flat) for _ in range(n)]
+        g = lambda args: grid(big.shape, tuple(args[-18:]))
+        # the fills, on copies
+        lph, lal, lp, lmuts, lmu, lmudf = own = _copies(*[L[n] for n in ("ph", "al", "p", "muts", "mu", "mudf")])
+        ptrs = (ctypes.c_void_p * 6)(*[ptr(t).value for t in own])
+        two = (ctypes.c_int * 6)(*[1 if t else 0 for _, t in kinds])
+        call("pywrf_set_physical_bc_group_adjoint", grid(big.shape, ix24), grid(flat.shape, ix2d), 6, ptrs,
+             b"".join(v.encode() for v, _ in kinds), two, stream())
+        # calc_p_rho
+        al_p, p_p, pm1_p, ph_p, t_p, t1_p = e3(6)
+        mu_p, muts_p = e2(2)
+        call("pywrf_calc_p_rho_adjoint", g(cp), ptr(lal), ptr(lp), ptr(L["pm1"]), ptr(cp[2]), ptr(cp[3]), ptr(cp[4]),
+             ptr(cp[5]), ptr(cp[6]), ptr(cp[8]), ptr(cp[9]), float(cp[19]), ptr(cp[20]), float(cp[22]), int(cp[24]),
+             ptr(al_p), ptr(p_p), ptr(pm1_p), ptr(ph_p), ptr(t_p), ptr(mu_p), ptr(muts_p), ptr(t1_p), stream())
+        # zero_grad_bdy, spec_bdyupdate_ph (which writes the sums' arrays in its band only)
+        lw, ft_z, ps_z = e3(3)
+        muts_z, mt_z = e2(2)
+        call("pywrf_zero_grad_bdy_adjoint", grid(big.shape, tuple(zg[-24:])), ptr(L["w"]), flag(zg[1]), ptr(lw),
+             stream())
+        _sums((lph, (lph, ph_p)))
+        zero_group([muts_z, mt_z, ft_z, ps_z])
+        call("pywrf_spec_bdyupdate_ph_adjoint", grid(big.shape, tuple(pz[-24:])), ptr(pz[0]), ptr(f_in), ptr(pz[2]),
+             ptr(pz[3]), ptr(pz[4]), float(pz[7]), flag(pz[8]), ptr(lph), ptr(muts_z), ptr(ft_z), ptr(mt_z), ptr(ps_z),
+             stream())
+        # sumflux
+        u_f, v_f, ww_f, ru_m, rv_m, ww_m, ul_f, vl_f, wwl_f = e3(9)
+        call("pywrf_sumflux_adjoint", g(sf), ptr(L["ru_m"]), ptr(L["rv_m"]), ptr(L["ww_m"]), int(sf[25]), int(sf[26]),
+             ptr(u_f), ptr(v_f), ptr(ww_f), ptr(ru_m), ptr(rv_m), ptr(ww_m), ptr(sf[6]), ptr(sf[7]), ptr(sf[21]),
+             ptr(sf[23]), ptr(ul_f), ptr(vl_f), ptr(wwl_f), stream())
+        # advance_w
+        w_w, ph_w, t_w, ta_w, u_w, v_w, ww_w, rw_w, pht_w, ws_w, t1_w, ph1_w, work, work2 = e3(14)
+        muts_w, muave_w = e2(2)
+        cf, _keep = _cf(wa[43], wa[44], wa[45])
+        call("pywrf_advance_w_adjoint", g(wa), ptr(L["t_ave"]), ptr(lw), ptr(lph), ptr(wa[7]), ptr(wa[9]), ptr(wa[20]),
+             ptr(wa[22]), ptr(wa[23]), ptr(wa[26]), ptr(wa[27]), ptr(wa[28]), ptr(wa[30]), ptr(wa[31]), ptr(wa[32]),
+             float(wa[35]), float(wa[36]), float(wa[37]), ptr(wa[41]), ptr(wa[42]), ptr(wa[47]), ptr(t2a_out),
+             ptr(w_out), ptr(wa[25]), ptr(wa[46]), cf, float(wa[33]), float(wa[34]), ptr(wa[39]), ptr(wa[40]),
+             ptr(w_w), ptr(ph_w), ptr(t_w), ptr(ta_w), ptr(u_w), ptr(v_w), ptr(muts_w), ptr(muave_w), ptr(ww_w),
+             ptr(rw_w), ptr(pht_w), ptr(ws_w), ptr(t1_w), ptr(wa[2]), ptr(wa[3]), ptr(ph1_w), ptr(work), ptr(work2),
+             stream())
+        # what advance_mu_t's results hand on
+        _sums((t_w, (L["t"], t_p, t_w)), (ww_w, (L["ww"], ww_f, ww_w)), (muts_w, (lmuts, muts_p, muts_z, muts_w)),
+              (muave_w, (L["muave"], muave_w)), (lmu, (lmu, mu_p)))
+        u_m, v_m, ww_i, t_m, ta_m, ft_m, u1_m, v1_m, ww1_m, t1_m = e3(10)
+        mu_m, muave_m, muts_m, mudf_m, mut_m = e2(5)
+        call("pywrf_advance_mu_t_adjoint", g(mt), ptr(ww_w), ptr(t_w), ptr(ta_w), ptr(muave_w), ptr(muts_w), ptr(lmudf),
+             ptr(lmu), ptr(mt[25]), ptr(mt[42]), ptr(mt[43]), ptr(mt[33]), ptr(mt[34]), ptr(mt[35]), ptr(mt[36]),
+             float(mt[29]), float(mt[30]), float(mt[31]), float(mt[32]), ptr(ww_i), ptr(u_m), ptr(v_m), ptr(mu_m),
+             ptr(muave_m), ptr(muts_m), ptr(mudf_m), ptr(t_m), ptr(ta_m), ptr(ft_m), ptr(mut_m), ptr(ww), ptr(mt[2]),
+             ptr(mt[4]), ptr(mt[10]), ptr(mt[11]), ptr(mt[38]), ptr(mt[40]), ptr(u1_m), ptr(v1_m), ptr(ww1_m),
+             ptr(t1_m), stream())
+        # advance_uv
+        _sums((u_w, (L["u"], u_f, u_w, u_m)), (v_w, (L["v"], v_f, v_w, v_m)))
+        u, v, p_u, ph_u, al_u, ru_u, rv_u = e3(7)
+        mu_u, mudf_u = e2(2)
+        cf, _keep2 = _cf(uv[32], uv[33], uv[34])
+        call("pywrf_advance_uv_adjoint", g(uv), ptr(u_w), ptr(v_w), ptr(uv[5]), ptr(uv[7]), ptr(uv[8]), ptr(uv[11]),
+             ptr(uv[12]), ptr(uv[13]), ptr(uv[14]), ptr(uv[24]), ptr(uv[25]), ptr(uv[26]), ptr(uv[27]), ptr(uv[28]),
+             float(uv[29]), float(uv[30]), float(uv[31]), cf, ptr(uv[35]), ptr(uv[36]), float(uv[37]), ptr(uv[38]),
+             int(uv[39]), ptr(u), ptr(v), ptr(p_u), ptr(ph_u), ptr(al_u), ptr(mu_u), ptr(mudf_u), ptr(ru_u), ptr(rv_u),
+             stream())
+        last = [(p_u, (p_u, p_p)), (ph_u, (ph_u, ph_w)), (al_u, (al_u, al_p)), (mu_u, (mu_u, mu_m)),
+                (mudf_u, (mudf_u, mudf_m))]
+        if ctx.given:
+            # the zone updates' shares: their tendencies enter like the field's own ring, dt times over
+            for call_, fields, lam in ((z1, (ru_u, rv_u), (u_w, v_w)), (z2, (ft_m, mut_m), (t_w, lmu))):
+                items, dt, i24, i2d = call_
+                wrf_boundary.spec_bdyupdate_group([(f, l, it[2], it[3]) for f, l, it in zip(fields, lam, items)], dt,
+                                                  i24, i2d)
+            items, dt, i24, i2d = z2
+            wrf_boundary.spec_bdyupdate_group([(mt_z, muts_w, items[2][2], items[2][3])], dt, i24, i2d)
+            last += [(pht_w, (pht_w, ft_z)), (mut_m, (mut_m, mt_z))]
+        if ctx.saved:
+            last += [(u1_m, (u1_m, ul_f)), (v1_m, (v1_m, vl_f)), (t1_m, (t1_m, t1_w, t1_p)), (ph1_w, (ph1_w, ps_z)),
+                     (ww1_m, (ww1_m, wwl_f))]
+        _sums(*last)
+        out = {"u": u, "v": v, "p": p_u, "ph": ph_u, "al": al_u, "mu": mu_u, "mudf": mudf_u, "ww": ww_i,
+               "muave": muave_m, "muts": muts_m, "t": t_m, "t_ave": ta_m, "w": w_w, "pm1": pm1_p, "ru_m": ru_m,
+               "rv_m": rv_m, "ww_m": ww_m}
+        res = [out[n] for n in ACOUSTIC_STATE]
+        if ctx.given:
+            res += [ru_u, rv_u, rw_w, ft_m, pht_w, mut_m]
+        if ctx.saved:
+            res += [u1_m, v1_m, ws_w, t1_m, ph1_w, ww1_m]
+        return (None, None, None, *res)
+
+
 def acoustic_substep(x, calls, forcing=None, saved=None):
-    """One acoustic substep (solver.py:1349-1493) as autograd Functions:
-    advance_uv, the u/v zone update, advance_mu_t, the t/mu/muts zone update,
-    advance_w, sumflux, spec_bdyupdate_ph, zero_grad_bdy, calc_p_rho and the
-    six open-boundary fills.  x: the 17 carried fields (ACOUSTIC_STATE
-    order); calls: the nine recorded calls' arguments; forcing: None, or the
-    six large-step tendencies (FORCING order) to use, and differentiate, in
-    place of the recorded ones wherever the substep reads them; saved: the
-    same for the six saved fields (SAVED order).  Returns the 17 fields
-    after the substep."""
-    st = dict(zip(ACOUSTIC_STATE, x))
-    uv, z1, mt, z2, wa, sf, pz, cp, bc = calls
-    fc = dict(zip(FORCING, forcing)) if forcing is not None else {
-        "ru_tend": uv[1], "rv_tend": uv[3], "rw_tend": None, "t_tend": mt[27], "ph_tend": None, "mu_tend": mt[28]}
-    given = forcing is not None
-    sv = dict(zip(SAVED, saved)) if saved is not None else dict.fromkeys(SAVED)
-    u1, v1 = AdvanceUV.apply(st["u"], fc["ru_tend"], st["v"], fc["rv_tend"], st["p"], st["ph"], st["al"], st["mu"],
-                             st["mudf"], uv)
-    u2, v2 = SpecBdyUpdateGroup.apply(z1, u1, v1, *((fc["ru_tend"], fc["rv_tend"]) if given else (None, None)))
-    ww, t, t_ave, muave, muts, mudf, mu = AdvanceMuT.apply(
-        u2, v2, st["ww"], st["mu"], st["muave"], st["muts"], st["mudf"], st["t"], st["t_ave"], fc["t_tend"],
-        fc["mu_tend"], mt, sv["u_save"], sv["v_save"], sv["ww1"], sv["t_save"])
-    t2, mu2, muts2 = SpecBdyUpdateGroup.apply(z2, t, mu, muts, *((fc["t_tend"], fc["mu_tend"], fc["mu_tend"])
-                                                                 if given else (None, None, None)))
-    t2a, w, ph = AdvanceW.apply(st["w"], st["ph"], t2, t_ave, u2, v2, muts2, muave, ww, wa, fc["rw_tend"],
-                                fc["ph_tend"], sv["w_save"], sv["t_save"], sv["ph_save"])
-    ru_m, rv_m, ww_m = SumFlux.apply(u2, v2, ww, st["ru_m"], st["rv_m"], st["ww_m"], sf, sv["u_save"],
-                                     sv["v_save"], sv["ww1"])
-    ph = SpecBdyUpdatePh.apply(ph, muts2, pz[0], fc["ph_tend"], fc["mu_tend"] if given else None, sv["ph_save"])
-    w = ZeroGradBdy.apply(w, pz[1])
-    al, p, pm1 = CalcPRho.apply(st["al"], st["p"], ph, t2, st["pm1"], mu2, muts2, cp, sv["t_save"])
-    items, ix24, ix2d = bc
-    ph, al, p, muts2, mu2, mudf = OpenBoundaryFill.apply([(v, two) for _, v, two in items], ix24, ix2d, ph, al, p,
-                                                         muts2, mu2, mudf)
-    new = {"u": u2, "v": v2, "p": p, "ph": ph, "al": al, "mu": mu2, "mudf": mudf, "ww": ww, "muave": muave,
-           "muts": muts2, "t": t2, "t_ave": t2a, "w": w, "pm1": pm1, "ru_m": ru_m, "rv_m": rv_m, "ww_m": ww_m}
-    return [new[n] for n in ACOUSTIC_STATE]
+    """One acoustic substep (AcousticSubstep).  x: the 17 carried fields
+    (ACOUSTIC_STATE order); calls: the nine recorded calls' arguments;
+    forcing: None, or the six large-step tendencies (FORCING order) to use,
+    and differentiate, in place of the recorded ones wherever the substep
+    reads them; saved: the same for the six saved fields (SAVED order).
+    Returns the 17 fields after the substep."""
+    return list(AcousticSubstep.apply(calls, forcing is not None, saved is not None, *x, *(forcing or ()),
+                                      *(saved or ())))
 
 
 STAGE_IN = ("u_2", "v_2", "w_2", "t_2", "ph_2", "mu_2", "u_1", "v_1", "w_1", "t_1", "ph_1", "mu_1", "ww", "mudf",

@@ -74,6 +74,65 @@ extern "C" int pywrf_zero_group(int n, void* const* fields, const long long* cou
   return (int)hipGetLastError();
 }
 
+// ------------------------------------------------------------------ sum_group
+// dst = the sum of up to four arrays, for several jobs in one launch: bound by
+// its reads and writes (16 bytes a lane where the arrays allow it).
+#define PW_SUM_MAX 16
+struct SumJobs {
+  float* d[PW_SUM_MAX];
+  const float* s[PW_SUM_MAX][4];
+  long n[PW_SUM_MAX];
+  int vec[PW_SUM_MAX];
+};
+
+__global__ void k_sum_group(SumJobs J) {
+  const int f = blockIdx.y;
+  float* d = J.d[f];
+  const float *a = J.s[f][0], *b = J.s[f][1], *c = J.s[f][2], *e = J.s[f][3];
+  const long t = (long)blockIdx.x * PW_BLOCK + threadIdx.x, step = (long)gridDim.x * PW_BLOCK;
+  const long n4 = J.vec[f] ? J.n[f] / 4 : 0;
+  for (long q = t; q < n4; q += step) {
+    float4 x = ((const float4*)a)[q];
+    if (b) { const float4 y = ((const float4*)b)[q]; x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w; }
+    if (c) { const float4 y = ((const float4*)c)[q]; x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w; }
+    if (e) { const float4 y = ((const float4*)e)[q]; x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w; }
+    ((float4*)d)[q] = x;
+  }
+  for (long q = 4 * n4 + t; q < J.n[f]; q += step) {
+    float x = a[q];
+    if (b) x += b[q];
+    if (c) x += c[q];
+    if (e) x += e[q];
+    d[q] = x;
+  }
+}
+
+extern "C" int pywrf_sum_group(int n, void* const* dst, void* const* src, const long long* counts,
+                               pywrf_stream_t s) {
+  if (n < 0 || n > PW_SUM_MAX || (n > 0 && (!dst || !src || !counts))) return PYWRF_E_ARG;
+  SumJobs J;
+  long most = 0;
+  for (int f = 0; f < n; ++f) {
+    if (!dst[f] || !src[4 * f] || counts[f] < 0) return PYWRF_E_ARG;
+    J.d[f] = (float*)dst[f];
+    J.n[f] = (long)counts[f];
+    size_t bits = (size_t)dst[f];
+    for (int m = 0; m < 4; ++m) {
+      J.s[f][m] = m && !J.s[f][m - 1] ? nullptr : (const float*)src[4 * f + m];
+      bits |= (size_t)J.s[f][m];
+    }
+    J.vec[f] = bits % sizeof(float4) == 0;
+    for (int h = 0; h < f; ++h)
+      if (J.d[h] == J.d[f]) return PYWRF_E_ARG;
+    most = J.n[f] > most ? J.n[f] : most;
+  }
+  if (n == 0 || most == 0) return 0;
+  long blocks = (most / 4 + PW_BLOCK - 1) / PW_BLOCK;
+  blocks = blocks > 2048 ? 2048 : blocks < 1 ? 1 : blocks;
+  hipLaunchKernelGGL(k_sum_group, dim3((unsigned)blocks, (unsigned)n), dim3(PW_BLOCK), 0, (hipStream_t)s, J);
+  return (int)hipGetLastError();
+}
+
 // ------------------------------------------------------------------ rk_scalar_tend
 extern "C" int pywrf_rk_scalar_tend(const pywrf_grid_t* g, int scs, int sce, int rk_step, const float* ru,
                                     const float* rv, const float* ww, const float* mut, const float* alt,

@@ -1,7 +1,7 @@
 """The column adjoints (64 columns of a row to a block, the levels dealt out to
 its waves) at plane sizes around a block's 63 and 64 columns, against the same
 FP64 oracle gradients as at the stock sizes, and with level arrays kept in LDS
-and, beyond what it holds, in memory."""
+and, beyond what it holds, in memory; and the grouped sum."""
 from types import SimpleNamespace
 
 import pytest
@@ -54,3 +54,18 @@ def test_advance_w_adjoint_is_the_same_from_lds_and_memory(nz):
         grads.append(adjoint.AdvanceW.backward(ctx, *[pad(l) for l in lams]))
     for n, a, b in zip(range(len(D) + 1), *grads):
         assert (a is None and b is None) or torch.equal(a, b[:nz0] if b.dim() == 3 else b), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 4, 4099])
+def test_sum_group_adds_in_order(n):
+    from pywrf_amd.adjoint import _sums
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    t = [torch.randn(n + 1, device="cuda", generator=gen) for _ in range(6)]
+    a, b, c, d = (x[:n].clone() for x in t[:4])
+    off = t[4][1:]                                # not 16-byte aligned
+    x, y, z = torch.empty_like(a), torch.empty_like(off), t[5][:n].clone()
+    want = ((a + b) + c) + d, off + b, z + a       # the last into its own source
+    _sums((x, (a, b, c, d)), (y, (off, b)), (z, (z, a)))
+    for got, w in zip((x, y, z), want):
+        assert torch.equal(got, w)
