@@ -310,58 +310,83 @@ struct AdvUV {
   int kde;
 };
 
-__device__ inline float uv_dpn(const Dims& D, const AdvUV& a, int k, int j, int i, int dj, int di) {
-  auto P = [&](int kk, int jj, int ii) { return AT(a.p, kk, jj, ii); };
-  if (k == 0)
-    return 0.5f * (a.cf[0] * (P(0, j, i) + P(0, j + dj, i + di)) + a.cf[1] * (P(1, j, i) + P(1, j + dj, i + di)) +
-                   a.cf[2] * (P(2, j, i) + P(2, j + dj, i + di)));
-  if (k == a.kde - 1) return 0.0f;
-  return 0.5f * (a.fnm[k] * (P(k, j, i) + P(k, j + dj, i + di)) + a.fnp[k] * (P(k - 1, j, i) + P(k - 1, j + dj, i + di)));
-}
-
-__device__ inline float uv_dpxy(const Dims& D, const AdvUV& a, int k, int j, int i, int dj, int di, const float* mv,
-                                const float* mx, const float* my, float rd) {
-  int jd = j + dj, id = i + di;
-  float r = AT2(mx, j, i) / AT2(my, j, i);
-  float d = r * 0.5f * rd * AT2(mv, j, i) *
-            (((AT(a.ph, k + 1, j, i) - AT(a.ph, k + 1, jd, id)) + (AT(a.ph, k, j, i) - AT(a.ph, k, jd, id))) +
-             (AT(a.alt, k, j, i) + AT(a.alt, k, jd, id)) * (AT(a.p, k, j, i) - AT(a.p, k, jd, id)) +
-             (AT(a.al, k, j, i) + AT(a.al, k, jd, id)) * (AT(a.pb, k, j, i) - AT(a.pb, k, jd, id)));
-  return d + r * rd * (AT(a.php, k, j, i) - AT(a.php, k, jd, id)) *
-                 (a.rdnw[k] * (uv_dpn(D, a, k + 1, j, i, dj, di) - uv_dpn(D, a, k, j, i, dj, di)) -
-                  0.5f * (AT2(a.mu, jd, id) + AT2(a.mu, j, i)));
-}
-
+// A thread marches up kc levels of its column, the values of the plane formed
+// once, p, ph and the pressure on w levels taken over from level to level, all
+// loads before the branches (neighbours clamped into the plane; what lies
+// outside a box is not used).
+//
 // ZONE: the specified zone's update of u and v (zu, zv: the ring around bu, bv)
-// on the points the boxes leave out.  46.2 us at 240 x 240 x 41 against 45.5 us
-// and a further launch of 5.2 us; with the tendencies loaded inside the branch
-// the ring's lanes made it 50.4.
+// on the points the boxes leave out.  240 x 240 x 41: 33.7 us, one
+// point a thread 46.2; the zone's update adds 0.5 us, as a launch of its own 5.2.
 template <bool ZONE>
-__global__ void k_advance_uv(Box all, Dims D, AdvUV a, Box bu, Box bv, UpdJob zu, UpdJob zv) {
-  int k, j, i;
-  if (!box_point(all, k, j, i)) return;
-  long q = D.ix(k, j, i);
-  float u = a.u_in[q];
-  const float tu = a.ru_tend[q], tv = a.rv_tend[q];   // before the branches: the ring's lanes wait for no load of their own
-  if (bu.has(k, j, i)) {
-    u = u + a.dts * tu;
-    float mxy = a.dfx * (AT2(a.mudf, j, i) - AT2(a.mudf, j, i - 1)) / AT2(a.msfuy, j, i);
-    float d = uv_dpxy(D, a, k, j, i, 0, -1, a.muu, a.msfux, a.msfuy, a.rdx);
-    u = u - a.dts * a.cqu[q] * d + mxy;
-  } else if (ZONE) {
-    u = spec_upd_value(zu, k, j, i, u, tu);
+__global__ void __launch_bounds__(PW_BLOCK) k_advance_uv(Box all, Dims D, AdvUV a, Box bu, Box bv, UpdJob zu, UpdJob zv,
+                                                         int kc) {
+  const int i = all.i0 + (int)(blockIdx.x * PW_TX + threadIdx.x), j = all.j0 + (int)(blockIdx.y * PW_TY + threadIdx.y);
+  if (i >= all.i1 || j >= all.j1) return;
+  const int ka = all.k0 + (int)blockIdx.z * kc, kb = imin(ka + kc, all.k1);
+  const unsigned C = D.ob2(j, i), W = D.ob2(j, imax(i - 1, 0)), S = D.ob2(imax(j - 1, 0), i);
+  const unsigned plane = (unsigned)D.plane() * 4u;
+  const bool u2 = bu.has2(j, i), v2 = bv.has2(j, i);
+  const float msfuy = at_b(a.msfuy, C), muc = at_b(a.mu, C), dfc = at_b(a.mudf, C);
+  const float rx = at_b(a.msfux, C) / msfuy, ry = at_b(a.msfvy, C) / at_b(a.msfvx, C);
+  const float Au = rx * 0.5f * a.rdx * at_b(a.muu, C), Bu = rx * a.rdx, Mu = 0.5f * (at_b(a.mu, W) + muc);
+  const float Av = ry * 0.5f * a.rdy * at_b(a.muv, C), Bv = ry * a.rdy, Mv = 0.5f * (at_b(a.mu, S) + muc);
+  const float mxu = a.dfx * (dfc - at_b(a.mudf, W)) / msfuy, mxv = a.dfy * (dfc - at_b(a.mudf, S)) * at_b(a.msfvx_inv, C);
+  unsigned o = (unsigned)ka * plane;
+  float pc = at_b(a.p, o + C), pw = at_b(a.p, o + W), ps = at_b(a.p, o + S);
+  float phc = at_b(a.ph, o + C), phw = at_b(a.ph, o + W), phs = at_b(a.ph, o + S);
+  float du = 0.0f, dv = 0.0f;   // the pressure on w level k at the u and v faces
+  if (ka == 0) {
+    const unsigned p1 = imin(1, D.nz - 1) * plane, p2 = imin(2, D.nz - 1) * plane;
+    const float c1 = at_b(a.p, p1 + C), c2 = at_b(a.p, p2 + C);
+    const float f0 = level(a.cf, 0), f1 = level(a.cf, 1), f2 = level(a.cf, 2);
+    du = 0.5f * (f0 * (pc + pw) + f1 * (c1 + at_b(a.p, p1 + W)) + f2 * (c2 + at_b(a.p, p2 + W)));
+    dv = 0.5f * (f0 * (pc + ps) + f1 * (c1 + at_b(a.p, p1 + S)) + f2 * (c2 + at_b(a.p, p2 + S)));
+  } else if (ka < a.kde - 1) {
+    const unsigned m = o - plane;
+    const float fm = level(a.fnm, ka), fp = level(a.fnp, ka), pmc = at_b(a.p, m + C);
+    du = 0.5f * (fm * (pc + pw) + fp * (pmc + at_b(a.p, m + W)));
+    dv = 0.5f * (fm * (pc + ps) + fp * (pmc + at_b(a.p, m + S)));
   }
-  float v = a.v_in[q];
-  if (bv.has(k, j, i)) {
-    v = v + a.dts * tv;
-    float mxy = a.dfy * (AT2(a.mudf, j, i) - AT2(a.mudf, j - 1, i)) * AT2(a.msfvx_inv, j, i);
-    float d = uv_dpxy(D, a, k, j, i, -1, 0, a.muv, a.msfvy, a.msfvx, a.rdy);
-    v = v - a.dts * a.cqv[q] * d + mxy;
-  } else if (ZONE) {
-    v = spec_upd_value(zv, k, j, i, v, tv);
+  for (int k = ka; k < kb; ++k) {
+    const unsigned t = o + C, up = k + 1 < D.nz ? o + plane : o;
+    float u = at_b(a.u_in, t), v = at_b(a.v_in, t);
+    const float tu = at_b(a.ru_tend, t), tv = at_b(a.rv_tend, t);
+    if (k < bu.k1) {   // bu, bv: the same levels
+      const bool lev = k >= bu.k0, inu = u2 && lev, inv = v2 && lev;
+      const float cqu = at_b(a.cqu, t), cqv = at_b(a.cqv, t);
+      const float pnc = at_b(a.p, up + C), pnw = at_b(a.p, up + W), pns = at_b(a.p, up + S);
+      const float pcc = at_b(a.ph, up + C), pcw = at_b(a.ph, up + W), pcs = at_b(a.ph, up + S);
+      const float ac = at_b(a.alt, t), aw = at_b(a.alt, o + W), as = at_b(a.alt, o + S);
+      const float lc = at_b(a.al, t), lw = at_b(a.al, o + W), ls = at_b(a.al, o + S);
+      const float bc = at_b(a.pb, t), bw = at_b(a.pb, o + W), bs = at_b(a.pb, o + S);
+      const float hc = at_b(a.php, t), hw = at_b(a.php, o + W), hs = at_b(a.php, o + S);
+      float dun = 0.0f, dvn = 0.0f;
+      if (k + 1 != a.kde - 1) {
+        const float fm = level(a.fnm, k + 1), fp = level(a.fnp, k + 1);
+        dun = 0.5f * (fm * (pnc + pnw) + fp * (pc + pw));
+        dvn = 0.5f * (fm * (pnc + pns) + fp * (pc + ps));
+      }
+      const float rd = level(a.rdnw, k);
+      const float xu = Au * (((pcc - pcw) + (phc - phw)) + (ac + aw) * (pc - pw) + (lc + lw) * (bc - bw)) +
+                       Bu * (hc - hw) * (rd * (dun - du) - Mu);
+      const float xv = Av * (((pcc - pcs) + (phc - phs)) + (ac + as) * (pc - ps) + (lc + ls) * (bc - bs)) +
+                       Bv * (hc - hs) * (rd * (dvn - dv) - Mv);
+      if (inu) u = (u + a.dts * tu) - a.dts * cqu * xu + mxu;
+      else if (ZONE) u = spec_upd_value(zu, k, j, i, u, tu);
+      if (inv) v = (v + a.dts * tv) - a.dts * cqv * xv + mxv;
+      else if (ZONE) v = spec_upd_value(zv, k, j, i, v, tv);
+      du = dun; dv = dvn;
+      pc = pnc; pw = pnw; ps = pns;
+      phc = pcc; phw = pcw; phs = pcs;
+    } else if (ZONE) {
+      u = spec_upd_value(zu, k, j, i, u, tu);
+      v = spec_upd_value(zv, k, j, i, v, tv);
+    }
+    at_b(a.u, t) = u;
+    at_b(a.v, t) = v;
+    o += plane;
   }
-  a.u[q] = u;   // stores last: no load waits on them
-  a.v[q] = v;
 }
 
 // gz non-null: also spec_bdyupdate of u with ru_tend and of v with rv_tend, step zdt
@@ -395,8 +420,12 @@ static int advance_uv(const pywrf_grid_t* g, const float* u_in, const float* ru_
     if (e) return e;
     ring = spec_upd_rings(zu, bu) && spec_upd_rings(zv, bv);
   }
-  if (ring) PW_LAUNCH_BOX(k_advance_uv<true>, whole(g), s, dims_of(g), a, bu, bv, zu, zv);
-  else PW_LAUNCH_BOX(k_advance_uv<false>, whole(g), s, dims_of(g), a, bu, bv, zu, zv);
+  const Box all = whole(g);
+  const int kc = march_levels(all);
+  dim3 grid((unsigned)((all.ni() + PW_TX - 1) / PW_TX), (unsigned)((all.nj() + PW_TY - 1) / PW_TY),
+            (unsigned)((all.nk() + kc - 1) / kc));
+  hipLaunchKernelGGL(ring ? k_advance_uv<true> : k_advance_uv<false>, grid, dim3(PW_TX, PW_TY), 0, (hipStream_t)s, all,
+                     dims_of(g), a, bu, bv, zu, zv, kc);
   if (gz && !ring) {
     int e = pywrf_spec_bdyupdate(gz, u_out, ru_tend, zdt, 'u', s);
     return e ? e : pywrf_spec_bdyupdate(gz, v_out, rv_tend, zdt, 'v', s);

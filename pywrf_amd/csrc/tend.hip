@@ -441,38 +441,144 @@ struct PgBuoy {
   int kde;
 };
 
-__global__ void k_pgf_buoy_cor(Box b, Dims D, Hpg h, Box hbv, Box hbu, PgBuoy pg, Box pbox, Cor a, Curv c, Box bu,
-                               Box bv, Box bw) {
-  int k, j, i;
-  if (!box_point(b, k, j, i)) return;
-  const int q = D.ix(k, j, i);
-  float u0 = a.ru_tend[q], v0 = a.rv_tend[q], w0 = a.rw_tend[q];
-  const bool gv = hbv.has(k, j, i), gu = hbu.has(k, j, i), gb = pbox.has(k, j, i);
-  if (gv) v0 = v0 - h.cqv[q] * hpg_dpx(D, h, k, j, i, -1, 0, h.muv, h.msfvy, h.msfvx, h.rdy);
-  if (gu) u0 = u0 - h.cqu[q] * hpg_dpx(D, h, k, j, i, 0, -1, h.muu, h.msfux, h.msfuy, h.rdx);
-  float cq1 = 0.0f, wtop = 0.0f;
-  const bool top = gb && k == pg.kde - 2;
-  if (gb) {
-    const float cqo = pg.cqw[q];
-    const float rmsf = 1.0f / AT2(pg.msfty, j, i);
-    if (top) {
-      const float c1 = 1.0f / (1.0f + cqo), c2 = cqo * c1;
-      wtop = AT(pg.rw_tend, pg.kde - 1, j, i) + rmsf * pg.g * (c1 * 2.0f * pg.rdnw[pg.kde - 2] * (-pg.p[q]) -
-                                                               AT2(pg.muf, j, i) - c2 * AT2(pg.mubf, j, i));
-    }
-    cq1 = 1.0f / (1.0f + cqo);
-    const float cq2 = cqo * cq1;
-    w0 = w0 + rmsf * pg.g * (cq1 * pg.rdn[k] * (pg.p[q] - AT(pg.p, k - 1, j, i)) - AT2(pg.muf, j, i) -
-                             cq2 * AT2(pg.mubf, j, i));
+// A thread marches up kc levels of its column: the map factor ratios and every
+// other value of the plane are formed once, the pressure on w levels, the sums
+// of the fluxes a level below, ph, p and rw a level above are taken over from
+// level to level.  One point a thread, the kernel formed 13 ratios and sums of
+// the plane at each of its points, twice the pressures, and its four branches
+// waited for memory in turn.  All loads here precede the branches, from
+// neighbours clamped into the plane; what lies outside a call's box is not
+// stored.  240 x 240 x 41: 61 us,
+// one point a thread 101.
+__global__ void __launch_bounds__(PW_BLOCK) k_pgf_buoy_cor(Box b, Dims D, Hpg h, Box hbv, Box hbu, PgBuoy pg, Box pbox,
+                                                           Cor a, Curv c, Box bu, Box bv, Box bw, int kc) {
+  const int i = b.i0 + (int)(blockIdx.x * PW_TX + threadIdx.x), j = b.j0 + (int)(blockIdx.y * PW_TY + threadIdx.y);
+  if (i >= b.i1 || j >= b.j1) return;
+  const int ka = b.k0 + (int)blockIdx.z * kc, kb = imin(ka + kc, b.k1);
+  const float rr = F(pw::reradius);
+  const int im = imax(i - 1, 0), ip = imin(i + 1, D.nx - 1), jm = imax(j - 1, 0), jp = imin(j + 1, D.ny - 1);
+  // the column, its neighbours to the west, east, south and north, and two diagonal ones (byte offsets in the plane)
+  const unsigned C = D.ob2(j, i), W = D.ob2(j, im), E = D.ob2(j, ip), S = D.ob2(jm, i), N = D.ob2(jp, i),
+                 SE = D.ob2(jm, ip), NW = D.ob2(jp, im), plane = (unsigned)D.plane() * 4u;
+  const bool gv2 = hbv.has2(j, i), gu2 = hbu.has2(j, i), gb2 = pbox.has2(j, i);
+  const bool hu2 = bu.has2(j, i), hv2 = bv.has2(j, i), hw2 = bw.has2(j, i);
+  // the plane's values
+  const float msfuy = at_b(a.msfuy, C), msfvx = at_b(a.msfvx, C), muc = at_b(h.mu, C);
+  const float ru_r = at_b(a.msfux, C) / msfuy, rv_r = at_b(a.msfvy, C) / msfvx;
+  const float Au = ru_r * 0.5f * h.rdx * at_b(h.muu, C), Bu = ru_r * h.rdx, Mu = 0.5f * (at_b(h.mu, W) + muc);
+  const float Av = rv_r * 0.5f * h.rdy * at_b(h.muv, C), Bv = rv_r * h.rdy, Mv = 0.5f * (at_b(h.mu, S) + muc);
+  const float fc = at_b(a.f, C), ec = at_b(a.e, C), cosa = at_b(a.cosa, C), sina = at_b(a.sina, C);
+  const float Fu = ru_r * 0.5f * (fc + at_b(a.f, W)) * 0.25f, Fv = rv_r * 0.5f * (fc + at_b(a.f, S)) * 0.25f;
+  const float Eu = 0.5f * (ec + at_b(a.e, W)) * 0.5f * (cosa + at_b(a.cosa, W)) * 0.25f;
+  const float Ev = rv_r * 0.5f * (ec + at_b(a.e, S)) * 0.5f * (sina + at_b(a.sina, S)) * 0.25f;
+  const float msfty = at_b(a.msfty, C), mr = at_b(a.msftx, C) / msfty, rmsf = 1.0f / msfty;
+  const float Cw = cosa * 0.5f, Sw = mr * sina * 0.5f, Gw = rmsf * pg.g, mub = at_b(pg.mubf, C);
+  const float vw = at_b(c.msfvx, W), vs = at_b(c.msfvx, S), uw = at_b(c.msfuy, W), us = at_b(c.msfuy, S);
+  const float xc = at_b(c.msfvx, N) - msfvx, yc = at_b(c.msfuy, E) - msfuy;
+  const float xw = at_b(c.msfvx, NW) - vw, yw = msfuy - uw, xs = msfvx - vs, ys = at_b(c.msfuy, SE) - us;
+  // values taken over from the level below
+  float pmc = 0.0f, pmw = 0.0f, pms = 0.0f, sru = 0.0f, srv = 0.0f, su = 0.0f, sv = 0.0f;
+  unsigned o = (unsigned)ka * plane;
+  if (ka > 0) {
+    const unsigned m = o - plane;
+    pmc = at_b(h.p, m + C); pmw = at_b(h.p, m + W); pms = at_b(h.p, m + S);
+    sru = at_b(a.ru, m + C) + at_b(a.ru, m + E); srv = at_b(a.rv, m + C) + at_b(a.rv, m + N);
+    su = at_b(c.u, m + C) + at_b(c.u, m + E); sv = at_b(c.v, m + C) + at_b(c.v, m + N);
   }
-  const bool hu = bu.has(k, j, i), hv = bv.has(k, j, i), hw = bw.has(k, j, i);
-  float tu, tv, tw;
-  cor_curv_point(D, a, c, hu, hv, hw, k, j, i, u0, v0, w0, tu, tv, tw);
-  if (hu || gu) a.ru_tend[q] = hu ? tu : u0;
-  if (hv || gv) a.rv_tend[q] = hv ? tv : v0;
-  if (hw || gb) a.rw_tend[q] = hw ? tw : w0;
-  if (gb) pg.cqw[q] = cq1;
-  if (top) AT(pg.rw_tend, pg.kde - 1, j, i) = wtop;
+  float pc = at_b(h.p, o + C), pw = at_b(h.p, o + W), ps = at_b(h.p, o + S);
+  float phc = at_b(h.ph, o + C), phw = at_b(h.ph, o + W), phs = at_b(h.ph, o + S);
+  float rwc = at_b(a.rw, o + C), rww = at_b(a.rw, o + W), rws = at_b(a.rw, o + S);
+  float du = 0.0f, dv = 0.0f;   // the pressure on w level k at the u and v faces
+  if (ka == 0) {
+    const unsigned p1 = imin(1, D.nz - 1) * plane, p2 = imin(2, D.nz - 1) * plane;
+    const float c1 = at_b(h.p, p1 + C), c2 = at_b(h.p, p2 + C);
+    const float f0 = level(h.cf, 0), f1 = level(h.cf, 1), f2 = level(h.cf, 2);
+    du = 0.5f * (f0 * (pw + pc) + f1 * (at_b(h.p, p1 + W) + c1) + f2 * (at_b(h.p, p2 + W) + c2));
+    dv = 0.5f * (f0 * (ps + pc) + f1 * (at_b(h.p, p1 + S) + c1) + f2 * (at_b(h.p, p2 + S) + c2));
+  } else if (ka < h.kde - 1) {
+    const float fm = level(h.fnm, ka), fp = level(h.fnp, ka);
+    du = 0.5f * (fm * (pw + pc) + fp * (pmw + pmc));
+    dv = 0.5f * (fm * (ps + pc) + fp * (pms + pmc));
+  }
+  for (int k = ka; k < kb; ++k) {
+    const unsigned t = o + C, up = k + 1 < D.nz ? o + plane : o;
+    float u0 = at_b(a.ru_tend, t), v0 = at_b(a.rv_tend, t), w0 = at_b(a.rw_tend, t);
+    const float cqu = at_b(h.cqu, t), cqv = at_b(h.cqv, t), cqw = at_b(pg.cqw, t);
+    const float pnc = at_b(h.p, up + C), pnw = at_b(h.p, up + W), pns = at_b(h.p, up + S);
+    const float pcc = at_b(h.ph, up + C), pcw = at_b(h.ph, up + W), pcs = at_b(h.ph, up + S);
+    const float rnc = at_b(a.rw, up + C), rnw = at_b(a.rw, up + W), rns = at_b(a.rw, up + S);
+    const float ac = at_b(h.alt, t), aw = at_b(h.alt, o + W), as = at_b(h.alt, o + S);
+    const float lc = at_b(h.al, t), lw = at_b(h.al, o + W), ls = at_b(h.al, o + S);
+    const float bc = at_b(h.pb, t), bbw = at_b(h.pb, o + W), bs = at_b(h.pb, o + S);
+    const float hc = at_b(h.php, t), hhw = at_b(h.php, o + W), hs = at_b(h.php, o + S);
+    const float ruc = at_b(a.ru, t), rue = at_b(a.ru, o + E), rus = at_b(a.ru, o + S), ruse = at_b(a.ru, o + SE);
+    const float rvc = at_b(a.rv, t), rvn = at_b(a.rv, o + N), rvw = at_b(a.rv, o + W), rvnw = at_b(a.rv, o + NW);
+    const float uc = at_b(c.u, t), ue = at_b(c.u, o + E), uww = at_b(c.u, o + W), uss = at_b(c.u, o + S),
+                use = at_b(c.u, o + SE);
+    const float vc = at_b(c.v, t), vn = at_b(c.v, o + N), vww = at_b(c.v, o + W), vnw = at_b(c.v, o + NW),
+                vss = at_b(c.v, o + S);
+    const bool lev = k >= hbv.k0 && k < hbv.k1;      // hbv, hbu: the same levels
+    const bool gv = gv2 && lev, gu = gu2 && lev, gb = gb2 && k >= pbox.k0 && k < pbox.k1;
+    if (lev) {
+      float dun = 0.0f, dvn = 0.0f;
+      if (k + 1 < h.kde - 1) {
+        const float fm = level(h.fnm, k + 1), fp = level(h.fnp, k + 1);
+        dun = 0.5f * (fm * (pnw + pnc) + fp * (pw + pc));
+        dvn = 0.5f * (fm * (pns + pnc) + fp * (ps + pc));
+      }
+      const float rd = level(h.rdnw, k);
+      const float xv = Av * ((pcc - pcs + phc - phs) + (ac + as) * (pc - ps) + (lc + ls) * (bc - bs)) +
+                       Bv * (hc - hs) * (rd * (dvn - dv) - Mv);
+      const float xu = Au * ((pcc - pcw + phc - phw) + (ac + aw) * (pc - pw) + (lc + lw) * (bc - bbw)) +
+                       Bu * (hc - hhw) * (rd * (dun - du) - Mu);
+      if (gv) v0 = v0 - cqv * xv;
+      if (gu) u0 = u0 - cqu * xu;
+      du = dun; dv = dvn;
+    }
+    const bool top = gb && k == pg.kde - 2;
+    const float cq1 = 1.0f / (1.0f + cqw), cq2 = cqw * cq1;
+    float wtop = 0.0f;
+    if (top)
+      wtop = at_b(pg.rw_tend, t + plane) +
+             Gw * (cq1 * 2.0f * level(pg.rdnw, pg.kde - 2) * (-pc) - muc - cq2 * mub);
+    if (gb) w0 = w0 + Gw * (cq1 * level(pg.rdn, k) * (pc - pmc) - muc - cq2 * mub);
+    const bool cl = k >= bu.k0 && k < bu.k1;          // bu, bv: the same levels
+    const bool hu = hu2 && cl, hv = hv2 && cl, hw = hw2 && k >= bw.k0 && k < bw.k1;
+    // vxgm here and at the neighbours the faces reach back to; beyond the interior it is the nearest inner value
+    const float gc = 0.5f * (uc + ue) * xc * c.rdy - 0.5f * (vc + vn) * yc * c.rdx;
+    const float gw = 0.5f * (uww + uc) * xw * c.rdy - 0.5f * (vww + vnw) * yw * c.rdx;
+    const float gs = 0.5f * (uss + use) * xs * c.rdy - 0.5f * (vss + vc) * ys * c.rdx;
+    const float qc = i > c.ite - 2 ? gw : j > c.jte - 2 ? gs : gc;
+    const float qw = i - 1 < c.its ? gc : gw, qs = j - 1 < c.jts ? gc : gs;
+    float tu, tv, tw = 0.0f;
+    {
+      const float rv4 = rvnw + rvn + rvw + rvc, rw4 = rnw + rww + rnc + rwc;
+      const float x = u0 + Fu * rv4 - Eu * rw4;
+      tu = x + 0.5f * (qc + qw) * 0.25f * rv4 - uc * rr * 0.25f * rw4;
+    }
+    {
+      const float ru4 = ruc + rue + rus + ruse, rw4 = rns + rws + rnc + rwc;
+      const float x = v0 - Fv * ru4 + Ev * rw4;
+      tv = x - 0.5f * (qc + qs) * 0.25f * ru4 - rv_r * vc * rr * 0.25f * rw4;
+    }
+    const float sru1 = ruc + rue, srv1 = rvc + rvn, su1 = uc + ue, sv1 = vc + vn;
+    if (k >= bw.k0 && k < bw.k1) {
+      const float fm = level(a.fzm, k), fp = level(a.fzp, k);
+      const float fru = fm * sru1 + fp * sru, frv = fm * srv1 + fp * srv, fu = fm * su1 + fp * su, fv = fm * sv1 + fp * sv;
+      const float x = w0 + ec * (Cw * fru - Sw * frv);
+      tw = x + rr * (0.5f * fru * 0.5f * fu + mr * 0.5f * frv * 0.5f * fv);
+    }
+    if (hu || gu) at_b(a.ru_tend, t) = hu ? tu : u0;
+    if (hv || gv) at_b(a.rv_tend, t) = hv ? tv : v0;
+    if (hw || gb) at_b(a.rw_tend, t) = hw ? tw : w0;
+    if (gb) at_b(pg.cqw, t) = cq1;
+    if (top) at_b(pg.rw_tend, t + plane) = wtop;
+    sru = sru1; srv = srv1; su = su1; sv = sv1;
+    pmc = pc; pc = pnc; pw = pnw; ps = pns;
+    phc = pcc; phw = pcw; phs = pcs;
+    rwc = rnc; rww = rnw; rws = rns;
+    o += plane;
+  }
 }
 
 extern "C" int pywrf_coriolis_curvature(const pywrf_grid_t* g, const float* ru, const float* rv, const float* rw,
@@ -837,6 +943,12 @@ extern "C" int pywrf_pgf_buoy_coriolis_curvature(
   Box b = mkbox(imin(hb.k0, imin(pbox.k0, cb.k0)), imax(hb.k1, imax(pbox.k1, cb.k1)),
                 imin(hb.j0, imin(pbox.j0, cb.j0)), imax(hb.j1, imax(pbox.j1, cb.j1)),
                 imin(hb.i0, imin(pbox.i0, cb.i0)), imax(hb.i1, imax(pbox.i1, cb.i1)));
-  PW_LAUNCH_BOX(k_pgf_buoy_cor, b, s, dims_of(g), h, hbv, hbu, pg, pbox, a, c, bu, bv, bw);
+  if (b.size() > 0) {
+    const int kc = march_levels(b);
+    dim3 grid((unsigned)((b.ni() + PW_TX - 1) / PW_TX), (unsigned)((b.nj() + PW_TY - 1) / PW_TY),
+              (unsigned)((b.nk() + kc - 1) / kc));
+    hipLaunchKernelGGL(k_pgf_buoy_cor, grid, dim3(PW_TX, PW_TY), 0, (hipStream_t)s, b, dims_of(g), h, hbv, hbu, pg,
+                       pbox, a, c, bu, bv, bw, kc);
+  }
   PW_RET();
 }
