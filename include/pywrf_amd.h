@@ -66,6 +66,16 @@ int pywrf_calc_alt(const pywrf_grid_t* g, float* alt, const float* al, const flo
 /* calc_php, wrf_dynamics.py:150-159 */
 int pywrf_calc_php(const pywrf_grid_t* g, float* php, const float* ph, const float* phb, pywrf_stream_t s);
 
+/* An RK stage's preparation in one launch: calculate_full, calc_mu_uv, couple_momentum, calc_ww_cp, calc_cq,
+ * calc_alt and calc_php with common index sets.  The arrays written must be distinct from all the arrays read.
+ * No counterpart in the reference: a batching of the seven calls above. */
+int pywrf_stage_prep(const pywrf_grid_t* g, float* mut, const float* mub, const float* mu, float* muu, float* muv,
+                     float* ru, const float* u, const float* msfu, float* rv, const float* v, const float* msfvx_inv,
+                     float* rw, const float* w, const float* msft, float* ww, const float* c1h, double rdx, double rdy,
+                     const float* msftx, const float* msfuy, const float* dnw, const float* moist, int n_moist,
+                     float* cqu, float* cqv, float* cqw, float* alt, const float* al, const float* alb, float* php,
+                     const float* ph, const float* phb, pywrf_stream_t s);
+
 /* ---- open lateral boundaries: wrf_dynamics.py:164-278 ------------------- */
 /* set_physical_bc2d, wrf_dynamics.py:164-212 (variable: u v w t x y r p, any case) */
 int pywrf_set_physical_bc2d(const pywrf_grid_t* g, float* dat, char variable, pywrf_stream_t s);

@@ -285,6 +285,159 @@ extern "C" int pywrf_calc_php(const pywrf_grid_t* g, float* php, const float* ph
   PW_RET();
 }
 
+// ---------------------------------------------------------------- the stage's preparation in one launch
+// calculate_full, calc_mu_uv, couple_momentum, calc_ww_cp, calc_cq, calc_alt
+// and calc_php.  Each is bound by its loads, and on a small plane by the
+// latency of one round of them, so they run side by side: the first blocks
+// take calc_ww_cp's columns (the longest chain), the others calc_cq's tiles,
+// which also couple the winds and form alt and php at their points.  What one
+// call hands to another (mut, muu, muv) is formed again where it is used, by
+// the same expressions.  us at
+// 240 x 240 x 41 and 40 x 40 x 41: 72 and 12, against 93 and 34 for the seven launches
+// (and 4 to 5 us of each launch's own in a graph of small kernels).
+struct StagePrep {
+  const float *mub, *mu, *u, *v, *w, *msfu, *msfvx_inv, *msft, *moist, *al, *alb, *ph, *phb;
+  float *mut, *muu, *muv, *ru, *rv, *rw, *cqu, *cqv, *cqw, *alt, *php;
+  int n, jts, jtf, jte, its, itf, ite;
+  Box b, bu, bv, bw, cu, cv, cw, bm;   // all tiles; couple_momentum's, calc_cq's; alt and php
+  WwCp ww;
+  Box wb;
+  int nww, nbx, ntx, nty;              // calc_ww_cp's blocks, its blocks a row; tiles along i and j
+};
+
+// calc_mu_uv's muu and muv at a point of their boxes
+__device__ inline float prep_muu(const Dims& D, const StagePrep& a, int j, int i) {
+  const int im = imax(i - 1, 0);
+  const float m = AT2(a.mu, j, i), w = AT2(a.mu, j, im), mb = AT2(a.mub, j, i), wb = AT2(a.mub, j, im);
+  return i == a.ite - 1 ? w + wb : i == a.its ? m + mb : 0.5f * (m + w + mb + wb);
+}
+__device__ inline float prep_muv(const Dims& D, const StagePrep& a, int j, int i) {
+  const int jm = imax(j - 1, 0);
+  const float m = AT2(a.mu, j, i), s = AT2(a.mu, jm, i), mb = AT2(a.mub, j, i), sb = AT2(a.mub, jm, i);
+  return j == a.jte - 1 ? s + sb : j == a.jts ? m + mb : 0.5f * (m + s + mb + sb);
+}
+
+__device__ inline void prep_ww(const Dims& D, const StagePrep& a, float* s_dv, float* s_dc) {
+  for (int t = threadIdx.x; t < D.nz; t += WW_TB) s_dc[t] = a.ww.dnw[t] * a.ww.c1h[t];
+  const int lane = threadIdx.x % WW_TI, grp = threadIdx.x / WW_TI;
+  const int j = a.wb.j0 + (int)blockIdx.x / a.nbx, i = a.wb.i0 + (int)blockIdx.x % a.nbx * WW_TI + lane;
+  const bool ok = i < a.wb.i1;
+  if (ok) {
+    const float ue = prep_muu(D, a, j, i + 1), uw = prep_muu(D, a, j, i), vn = prep_muv(D, a, j + 1, i),
+                vs = prep_muv(D, a, j, i);
+    const float fe = AT2(a.ww.msfuy, j, i + 1), fw = AT2(a.ww.msfuy, j, i), xn = AT2(a.ww.msfvx_inv, j + 1, i),
+                xs = AT2(a.ww.msfvx_inv, j, i), mx = AT2(a.ww.msftx, j, i);
+#pragma unroll 6
+    for (int k = grp; k < D.nz; k += WW_TG) {
+      const float e = ue * AT(a.ww.u, k, j, i + 1) / fe, w = uw * AT(a.ww.u, k, j, i) / fw;
+      const float n = vn * AT(a.ww.v, k, j + 1, i) * xn, s = vs * AT(a.ww.v, k, j, i) * xs;
+      s_dv[k * WW_TI + lane] =
+          k >= a.wb.k0 && k < a.wb.k1 ? mx * a.ww.dnw[k] * (a.ww.rdx * (e - w) + a.ww.rdy * (n - s)) : 0.0f;
+    }
+  }
+  __syncthreads();
+  if (!ok || grp != 0) return;
+  const float dmdt = torch_outer_sum(D.nz, [&](int k) { return s_dv[k * WW_TI + lane]; });
+  float wk = AT(a.ww.ww, 0, j, i);
+  for (int k = 0; k < a.wb.k1 - 1; ++k) {
+    wk = wk - s_dc[k] * dmdt - s_dv[k * WW_TI + lane];
+    AT(a.ww.ww, k + 1, j, i) = wk;
+  }
+}
+
+__global__ void __launch_bounds__(WW_TB) k_stage_prep(Dims D, StagePrep a) {
+  extern __shared__ float s_dv[];   // [nz][WW_TI]
+  __shared__ float s_dc[256];
+  if ((int)blockIdx.x < a.nww) {
+    prep_ww(D, a, s_dv, s_dc);
+    return;
+  }
+  const int t = (int)blockIdx.x - a.nww, tx = t % a.ntx, ty = t / a.ntx % a.nty, tz = t / a.ntx / a.nty;
+  const int lane = threadIdx.x % WW_TI;
+  const int i = a.b.i0 - 1 + tx * CQ_OX + lane, j = a.b.j0 + ty * WW_TG + (int)threadIdx.x / WW_TI;
+  if (j >= a.b.j1) return;                    // a whole wave (one row) leaves together
+  const int k0 = a.b.k0 + tz * CQ_KC, k1 = imin(k0 + CQ_KC, a.b.k1);
+  const bool live = i < a.b.i1, own = lane >= 1 && live;
+  // every load of the tile first
+  const int ic = imin(i, D.nx - 1);
+  const float muu = prep_muu(D, a, j, ic), muv = prep_muv(D, a, j, ic), mut = AT2(a.mub, j, ic) + AT2(a.mu, j, ic);
+  const float mfu = AT2(a.msfu, j, ic), mfv = AT2(a.msfvx_inv, j, ic), mft = AT2(a.msft, j, ic);
+  const bool cq0 = live && k0 >= 1 && k0 - 1 < a.cu.k1;
+  float sdown = cq0 ? qsum(D, a.moist, a.n, k0 - 1, j, i) : 0.0f;
+  float s[CQ_KC], sn[CQ_KC], u[CQ_KC], v[CQ_KC], w[CQ_KC], al[CQ_KC], alb[CQ_KC], ph[CQ_KC + 1], phb[CQ_KC + 1];
+#pragma unroll
+  for (int kk = 0; kk <= CQ_KC; ++kk) {
+    const int k = k0 + kk, kc = imin(k, D.nz - 1);
+    ph[kk] = AT(a.ph, kc, j, ic);
+    phb[kk] = AT(a.phb, kc, j, ic);
+    if (kk == CQ_KC) break;
+    s[kk] = (live && k < a.cu.k1) ? qsum(D, a.moist, a.n, k, j, i) : 0.0f;
+    sn[kk] = (own && a.cv.has(k, j, i)) ? qsum(D, a.moist, a.n, k, j - 1, i) : 0.0f;
+    u[kk] = AT(a.u, kc, j, ic); v[kk] = AT(a.v, kc, j, ic); w[kk] = AT(a.w, kc, j, ic);
+    al[kk] = AT(a.al, kc, j, ic); alb[kk] = AT(a.alb, kc, j, ic);
+  }
+  if (tz == 0 && own) {
+    if (j < a.jtf && i < a.itf) AT2(a.mut, j, i) = mut;
+    if (j < a.jtf) AT2(a.muu, j, i) = muu;
+    if (i < a.itf) AT2(a.muv, j, i) = muv;
+  }
+#pragma unroll
+  for (int kk = 0; kk < CQ_KC; ++kk) {
+    const int k = k0 + kk;
+    if (k >= k1) break;                       // uniform across the wave
+    const float s0 = s[kk], sw = __shfl_up(s0, 1, WW_TI);
+    if (own) {
+      const int p = D.ix(k, j, i);
+      if (a.cu.has(k, j, i)) a.cqu[p] = 1.0f / (1.0f + 0.5f * (s0 + sw));
+      if (a.cv.has(k, j, i)) a.cqv[p] = 1.0f / (1.0f + 0.5f * (s0 + sn[kk]));
+      if (a.cw.has(k, j, i)) a.cqw[p] = 0.5f * (s0 + sdown);
+      if (a.bu.has(k, j, i)) a.ru[p] = u[kk] * muu / mfu;
+      if (a.bv.has(k, j, i)) a.rv[p] = v[kk] * muv * mfv;
+      if (a.bw.has(k, j, i)) a.rw[p] = w[kk] * mut / mft;
+      if (a.bm.has(k, j, i)) {
+        a.alt[p] = al[kk] + alb[kk];
+        a.php[p] = 0.5f * (phb[kk] + phb[kk + 1] + ph[kk] + ph[kk + 1]);
+      }
+    }
+    sdown = s0;
+  }
+}
+
+extern "C" int pywrf_stage_prep(const pywrf_grid_t* g, float* mut, const float* mub, const float* mu, float* muu,
+                                float* muv, float* ru, const float* u, const float* msfu, float* rv, const float* v,
+                                const float* msfvx_inv, float* rw, const float* w, const float* msft, float* ww,
+                                const float* c1h, double rdx, double rdy, const float* msftx, const float* msfuy,
+                                const float* dnw, const float* moist, int n_moist, float* cqu, float* cqv, float* cqw,
+                                float* alt, const float* al, const float* alb, float* php, const float* ph,
+                                const float* phb, pywrf_stream_t s) {
+  if (!pw_size_ok(g)) return PYWRF_E_RANGE;
+  CHECK(g, 1);
+  if (n_moist < 1) return PYWRF_E_ARG;
+  const int ktf = imin(g->kte, g->kde - 1), jtf = imin(g->jte, g->jde - 1), itf = imin(g->ite, g->ide - 1);
+  if (ktf + 1 > g->nz || g->kts != 0) return PYWRF_E_RANGE;
+  const size_t lds = (size_t)g->nz * WW_TI * sizeof(float);
+  if (lds > 60 * 1024 || g->nz > 256) return PYWRF_E_RANGE;
+  StagePrep a = {mub, mu, u, v, w, msfu, msfvx_inv, msft, moist, al, alb, ph, phb, mut, muu, muv, ru, rv, rw, cqu, cqv,
+                 cqw, alt, php, n_moist, g->jts, jtf, g->jte, g->its, itf, g->ite};
+  a.b = mkbox(0, g->kte, g->jts, g->jte, g->its, g->ite);
+  a.bu = mkbox(0, ktf, g->jts, jtf, g->its, g->ite);
+  a.bv = mkbox(0, ktf, g->jts, g->jte, g->its, itf);
+  a.bw = mkbox(0, g->kte, g->jts, jtf, g->its, itf);
+  a.cu = a.bu; a.cv = a.bv;
+  a.cw = mkbox(1, ktf, g->jts, jtf, g->its, itf);
+  a.bm = mkbox(0, ktf, g->jts, jtf, g->its, itf);
+  a.ww = {u, v, nullptr, nullptr, c1h, msftx, msfuy, msfvx_inv, dnw, ww, F(rdx), F(rdy)};
+  a.wb = a.bm;
+  if (a.b.size() <= 0 || a.wb.size() <= 0) return PYWRF_E_RANGE;
+  a.nbx = (a.wb.ni() + WW_TI - 1) / WW_TI;
+  a.nww = a.nbx * a.wb.nj();
+  a.ntx = (a.b.ni() + CQ_OX - 1) / CQ_OX;
+  a.nty = (a.b.nj() + WW_TG - 1) / WW_TG;
+  const long blocks = a.nww + (long)a.ntx * a.nty * ((a.b.nk() + CQ_KC - 1) / CQ_KC);
+  hipLaunchKernelGGL(k_stage_prep, dim3((unsigned)blocks), dim3(WW_TB), lds, (hipStream_t)s, dims_of(g), a);
+  PW_RET();
+}
+
 // ---------------------------------------------------------------- set_physical_bc3d / bc2d
 __global__ void k_open_bc(Dims D, float* dat, int k0, BcSpec c) {
   open_bc_plane(dat + (long)(k0 + (int)blockIdx.x) * D.plane(), D.nx, c);

@@ -217,15 +217,23 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
         else:
             dt_rk, dts_rk, nsmall = dtm, dts, cfg.soundsteps
         # rk_step_prep (solver.py:736-778)
-        s.mut = o.calculate_full(s.mut, s.mub, s.mu, *I18)
-        s.muu, s.muv = o.calc_mu_uv(s.mu, s.mub, s.muu, s.muv, *I18)
-        s.ru, s.rv, s.rw = o.couple_momentum(s.muu, s.ru, s.u, s.msfu, s.muv, s.rv, s.v, s.msfv, s.msfvx_inv,
-                                             s.mut, s.rw, s.w, s.msft, s.c1h, s.c2h, s.c1f, s.c2f, *I18)
-        s.ww = o.calc_ww_cp(s.u, s.v, s.mu, s.mub, s.muu, s.muv, s.c1h, s.c2h, s.ww, rdx, rdy, s.msftx, s.msfty,
-                            s.msfux, s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.dnw, *I18)
-        s.cqu, _cuv, s.cqw = o.calc_cq(s.moist, s.cqu, s.cqv, s.cqw, N_MOIST, *I18)
-        s.alt = o.calc_alt(s.alt, s.al, s.alb, *I18)
-        s.php = o.calc_php(s.php, s.ph, s.phb, *I18)
+        prep = ((s.mut, s.mub, s.mu, *I18), (s.mu, s.mub, s.muu, s.muv, *I18),
+                (s.muu, s.ru, s.u, s.msfu, s.muv, s.rv, s.v, s.msfv, s.msfvx_inv, s.mut, s.rw, s.w, s.msft, s.c1h,
+                 s.c2h, s.c1f, s.c2f, *I18),
+                (s.u, s.v, s.mu, s.mub, s.muu, s.muv, s.c1h, s.c2h, s.ww, rdx, rdy, s.msftx, s.msfty, s.msfux,
+                 s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.dnw, *I18),
+                (s.moist, s.cqu, s.cqv, s.cqw, N_MOIST, *I18), (s.alt, s.al, s.alb, *I18), (s.php, s.ph, s.phb, *I18))
+        if merged:
+            o.stage_prep(*prep)
+        else:
+            full, mass, couple, omega, cq, alt, php = prep
+            s.mut = o.calculate_full(*full)
+            s.muu, s.muv = o.calc_mu_uv(*mass)
+            s.ru, s.rv, s.rw = o.couple_momentum(*couple)
+            s.ww = o.calc_ww_cp(*omega)
+            s.cqu, _cuv, s.cqw = o.calc_cq(*cq)
+            s.alt = o.calc_alt(*alt)
+            s.php = o.calc_php(*php)
         # rk_phys_bc_dry_1 (solver.py:781-843)
         (s.ru, s.rv, s.rw, s.ww, s.php, s.alt, s.p, s.muu, s.muv, s.mut, s.al, s.ph) = bcs(
             (s.ru, 'u', 0), (s.rv, 'v', 0), (s.rw, 'w', 0), (s.ww, 'w', 0), (s.php, 'w', 0), (s.alt, 't', 0),

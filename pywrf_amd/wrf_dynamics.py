@@ -108,6 +108,33 @@ def calc_php(php, ph, phb,
     return php
 
 
+def stage_prep(full_args, mass_args, couple_args, ww_args, cq_args, alt_args, php_args):
+    """calculate_full, calc_mu_uv, couple_momentum, calc_ww_cp, calc_cq,
+    calc_alt and calc_php (the sequence of solver.py:736-778), each given as
+    the tuple of its positional arguments, in one launch.  The calls must share
+    their operands as that sequence does, and their index set.  Returns the
+    seven calls' results.  Not part of the reference API."""
+    mut, mub, mu, *ix = full_args
+    mu_, mub_, muu, muv, *ix1 = mass_args
+    muu_, ru, u, msfu, muv_, rv, v, _, msfvx_inv, mut_, rw, w, msft, _, _, _, _, *ix2 = couple_args
+    (wu, wv, wmu, wmub, wmuu, wmuv, c1h, _, ww, rdx, rdy, msftx, _, _, msfuy, _, winv, _, dnw, *ix3) = ww_args
+    moist, cqu, cqv, cqw, _, *ix4 = cq_args
+    alt, al, alb, *ix5 = alt_args
+    php, ph, phb, *ix6 = php_args
+    same = [(mu_, mu), (mub_, mub), (muu_, muu), (muv_, muv), (mut_, mut), (wu, u), (wv, v), (wmu, mu), (wmub, mub),
+            (wmuu, muu), (wmuv, muv), (winv, msfvx_inv)]
+    if not all(x is y for x, y in same) or any(tuple(q) != tuple(ix) for q in (ix1, ix2, ix3, ix4, ix5, ix6)):
+        raise ValueError("stage_prep: the calls do not share their common arguments")
+    read = {t.data_ptr() for t in (mub, mu, u, v, w, moist, al, alb, ph, phb)}
+    if any(t.data_ptr() in read for t in (mut, muu, muv, ru, rv, rw, ww, cqu, cqv, cqw, alt, php)):
+        raise ValueError("stage_prep: an array is both read and written")
+    call("pywrf_stage_prep", grid(u.shape, tuple(ix)), ptr(mut), ptr(mub), ptr(mu), ptr(muu), ptr(muv), ptr(ru), ptr(u),
+         ptr(msfu), ptr(rv), ptr(v), ptr(msfvx_inv), ptr(rw), ptr(w), ptr(msft), ptr(ww), ptr(c1h), float(rdx),
+         float(rdy), ptr(msftx), ptr(msfuy), ptr(dnw), ptr(moist), int(moist.shape[0]), ptr(cqu), ptr(cqv), ptr(cqw),
+         ptr(alt), ptr(al), ptr(alb), ptr(php), ptr(ph), ptr(phb), stream())
+    return mut, (muu, muv), (ru, rv, rw), ww, (cqu, cqv, cqw), alt, php
+
+
 def set_physical_bc2d(dat, variable_in,
                       ids, ide, jds, jde,
                       ims, ime, jms, jme,
