@@ -301,6 +301,14 @@ int pywrf_calc_p_rho(const pywrf_grid_t* g, const float* al_in, const float* p_i
                      const float* alt, const float* t_2, const float* t_1, const float* c2a, float* pm1,
                      const float* mu, const float* mut, double t0, const float* rdnw, double smdiv, int step,
                      float* al_out, float* p_out, pywrf_stream_t s);
+/* calc_p_rho past step 0 (pm1 out of place), then the open-boundary fills of ph, al_out, p_out, mut, mu and mudf
+ * (variables: their six flags, the second and third the same; g3, g2: the fills' 3-D and 2-D index sets), in one
+ * launch.  No counterpart in the reference: a batching of the seven calls. */
+int pywrf_calc_p_rho_bc(const pywrf_grid_t* g, const pywrf_grid_t* g3, const pywrf_grid_t* g2, const float* al_in,
+                        const float* p_in, float* ph, const float* alt, const float* t_2, const float* t_1,
+                        const float* c2a, const float* pm1_in, float* mu, float* mut, double t0, const float* rdnw,
+                        double smdiv, int step, float* mudf, const char* variables, float* al_out, float* p_out,
+                        float* pm1_out, pywrf_stream_t s);
 /* calc_coef_w, wrf_dynamics.py:3316-3388 */
 int pywrf_calc_coef_w(const pywrf_grid_t* g, float* a, float* alpha, float* gamma, const float* mut,
                       const float* cqw, const float* rdn, const float* rdnw, const float* c2a, double dts,

@@ -130,6 +130,22 @@ struct BcJob {
   BcSpec c;
 };
 
+// The cell whose value a cell holds after the fill (itself where nothing is
+// copied to it): the y-copy's source, then the x-copy's.
+__device__ inline void open_bc_source(const BcSpec& c, int& j, int& i) {
+  const int yh0 = c.vstag ? c.jde : c.jde - 1;
+  if (i >= c.yc0 && i < c.yc1) {
+    if (j >= c.jds - 3 && j < c.jds) j = c.jds;
+    else if (j >= yh0 && j < yh0 + 3) j = yh0 - 1;
+  }
+  const int r0 = c.ustag ? c.ur0 : c.xr0, r1 = c.ustag ? c.ur1 : c.xr1, xh0 = c.ustag ? c.ide : c.ide - 1;
+  if (i >= c.ids - 3 && i < c.ids) {
+    if (j >= c.xr0 && j < c.xr1) i = c.ids;
+  } else if (i >= xh0 && i < xh0 + 3) {
+    if (j >= r0 && j < r1) i = xh0 - 1;
+  }
+}
+
 static inline char lower(char v) { return (v >= 'A' && v <= 'Z') ? (char)(v - 'A' + 'a') : v; }
 static inline bool in(char v, const char* set) { for (; *set; ++set) if (*set == v) return true; return false; }
 

@@ -382,10 +382,9 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
             s.muv, s.muvs, s.mut, s.muts, s.mudf, s.c1h, s.c2h, s.c1f, s.c2f, s.c3h, s.c4h, s.c3f, s.c4f,
             s.u_save, s.v_save, s.w_save, s.t_save, s.ph_save, s.mu_save, s.ww, s.ww1, s.c2a, s.pb, s.p, s.alt,
             s.msfux, s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.msftx, s.msfty, rdx, rdy, rk_step, *I18)
-        cpr = lambda step: o.calc_p_rho(s.al, s.p, s.ph, s.alt, s.t, s.t_save, s.c2a, s.pm1, s.mu, s.muts, s.c1h,
-                                        s.c2h, s.c1f, s.c2f, s.c3h, s.c4h, s.c3f, s.c4f, s.znu, T0, s.rdnw, s.dnw,
-                                        SMDIV, True, step, *I18)
-        s.al, s.p, s.pm1 = cpr(0)
+        pr_args = lambda step: (s.al, s.p, s.ph, s.alt, s.t, s.t_save, s.c2a, s.pm1, s.mu, s.muts, s.c1h, s.c2h, s.c1f,
+                                s.c2f, s.c3h, s.c4h, s.c3f, s.c4f, s.znu, T0, s.rdnw, s.dnw, SMDIV, True, step, *I18)
+        s.al, s.p, s.pm1 = o.calc_p_rho(*pr_args(0))
         s.a, s.alpha, s.gamma = o.calc_coef_w(s.a, s.alpha, s.gamma, s.mut, s.c1h, s.c2h, s.c1f, s.c2f, s.c3h,
                                               s.c4h, s.c3f, s.c4f, s.cqw, s.rdn, s.rdnw, s.c2a, dts_rk, G, EPSSM,
                                               False, *I18)
@@ -442,9 +441,12 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
                 else:
                     s.ph = o.spec_bdyupdate_ph(*ph_args)
                     s.w = o.zero_grad_bdy(*zg_args)
-            s.al, s.p, s.pm1 = cpr(iteration)
-            s.ph, s.al, s.p, s.muts, s.mu, s.mudf = bcs((s.ph, 'w', 0), (s.al, 'p', 0), (s.p, 'p', 0),
-                                                        (s.muts, 't', 1), (s.mu, 't', 1), (s.mudf, 't', 1))
+            if merged:
+                s.al, s.p, s.pm1 = o.calc_p_rho_bc(pr_args(iteration), s.mudf, 'wppttt', I24, I2)
+            else:
+                s.al, s.p, s.pm1 = o.calc_p_rho(*pr_args(iteration))
+                s.ph, s.al, s.p, s.muts, s.mu, s.mudf = bcs((s.ph, 'w', 0), (s.al, 'p', 0), (s.p, 'p', 0),
+                                                            (s.muts, 't', 1), (s.mu, 't', 1), (s.mudf, 't', 1))
         # back to full variables (solver.py:1496-1543)
         s.muus, s.muvs = o.calc_mu_uv_1(s.muts, s.muus, s.muvs, *I18)
         s.u, s.v, s.w, s.ph, s.ww, s.t, s.mu = o.small_step_finish(

@@ -766,6 +766,22 @@ def calc_p_rho(al_ori, p_ori, ph,
     return al, p, pm1
 
 
+def calc_p_rho_bc(pr_args, mudf, variables, idx24, idx2d):
+    """calc_p_rho (pr_args: its positional arguments, step not 0), then the
+    open-boundary fills of ph, al, p, mut, mu and mudf (variables: their six
+    flags, al's and p's the same; idx24 / idx2d as in set_physical_bc_group),
+    in one launch.  Same result as the calls in order, pm1 in a fresh array.
+    Returns (al, p, pm1).  Not part of the reference API."""
+    (al_ori, p_ori, ph, alt, t_2, t_1, c2a, pm1, mu, mut, _, _, _, _, _, _, _, _, _, t0, rdnw, _, smdiv, _, step,
+     *ix) = pr_args
+    al, p, pm = fresh(al_ori), fresh(p_ori), fresh(pm1)
+    call("pywrf_calc_p_rho_bc", grid(p_ori.shape, tuple(ix)), grid(p_ori.shape, tuple(idx24)),
+         grid(mu.shape, tuple(idx2d)), ptr(al_ori), ptr(p_ori), ptr(ph), ptr(alt), ptr(t_2), ptr(t_1), ptr(c2a),
+         ptr(pm1), ptr(mu), ptr(mut), float(t0), ptr(rdnw), float(smdiv), int(step), ptr(mudf), variables.encode(),
+         ptr(al), ptr(p), ptr(pm), stream())
+    return al, p, pm
+
+
 def calc_coef_w(a, alpha, gamma,
                 mut,
                 c1h, c2h, c1f, c2f,
