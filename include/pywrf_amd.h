@@ -466,6 +466,14 @@ int pywrf_relax_bdytend_dtbc_dev(const pywrf_grid_t* g, const float* field, floa
 int pywrf_spec_bdytend(const pywrf_grid_t* g, float* field_tend, const float* btxs, const float* btxe,
                        const float* btys, const float* btye, char variable_in, pywrf_stream_t s);
 
+/* n (at most 8) relax_bdytend calls on distinct tendencies in one launch: fields[f], tends[f], variables[f] and
+ * bdys[8 f .. 8 f + 7] as in pywrf_relax_bdytend, is2d[f] selects the index set g2 over g3; masses[f] non-null: the
+ * field is first multiplied by that plane on mass_weight's box (index set gw).  No counterpart in the reference: a
+ * batching. */
+int pywrf_relax_group_dtbc_dev(const pywrf_grid_t* g3, const pywrf_grid_t* g2, const pywrf_grid_t* gw, int n,
+                               void* const* fields, void* const* masses, void* const* tends, void* const* bdys,
+                               const char* variables, const int* is2d, const float* dtbc, const float* fcx,
+                               const float* gcx, pywrf_stream_t s);
 /* n consecutive spec_bdytend calls on distinct tendencies (solver.py:
  * 1220-1254) in one launch: tends[f], variables[f] as in pywrf_spec_bdytend,
  * bdy_tends[4f .. 4f+3] its btxs, btxe, btys, btye, is2d[f] selects the index

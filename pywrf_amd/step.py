@@ -343,19 +343,25 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
             # relax_bdy_dry (solver.py:1146-1203)
             rb = lambda fld, tend, key, var, ix=I24: o.relax_bdytend(
                 fld, tend, *b[key], var, SPEC_BDY_WIDTH, SPEC_ZONE, RELAX_ZONE, dtbc, s.fcx, s.gcx, *ix)
-            s.u_save = rb(s.ru, s.u_save, 'u', 'u')
-            s.v_save = rb(s.rv, s.v_save, 'v', 'v')
             i_start, i_end = max(its - 1, ids), min(ite + 1, ide - 1)
             j_start, j_end = max(jts - 1, jds), min(jte + 1, jde - 1)
             mw = (ids, ide, jds, jde, kds, kde, ims, ime, jms, jme, kms, kme,
                   its - 1, ite + 1, jts - 1, jte + 1, kts, kte, i_start, i_end, j_start, j_end, kts, kte)
-            s.rfield = o.mass_weight(s.ph, s.mut, s.rfield, s.c1f, s.c2f, *mw)
-            s.ph_save = rb(s.rfield, s.ph_save, 'ph', 'h')
-            s.rfield = o.mass_weight(s.t, s.mut, s.rfield, s.c1h, s.c2h, *mw)
-            s.t_save = rb(s.rfield, s.t_save, 't', 't')
             ix_mu = (ids, ide, jds, jde, 0, 1, ims, ime, jms, jme, 0, 1, ips, ipe, jps, jpe, 0, 1,
                      its, ite, jts, jte, 0, 1)
-            mu_tend_e = rb(mu_e, mu_tend_e, 'mu', 'm', ix_mu)
+            if merged:
+                o.relax_group([(s.ru, None, s.u_save, b['u'], 'u', False), (s.rv, None, s.v_save, b['v'], 'v', False),
+                               (s.ph, s.mut, s.ph_save, b['ph'], 'h', False), (s.t, s.mut, s.t_save, b['t'], 't', False),
+                               (mu_e, None, mu_tend_e, b['mu'], 'm', True)], dtbc, s.fcx, s.gcx, I24, ix_mu, mw)
+                s.rfield = o.mass_weight(s.t, s.mut, s.rfield, s.c1h, s.c2h, *mw)   # the driver leaves it so
+            else:
+                s.u_save = rb(s.ru, s.u_save, 'u', 'u')
+                s.v_save = rb(s.rv, s.v_save, 'v', 'v')
+                s.rfield = o.mass_weight(s.ph, s.mut, s.rfield, s.c1f, s.c2f, *mw)
+                s.ph_save = rb(s.rfield, s.ph_save, 'ph', 'h')
+                s.rfield = o.mass_weight(s.t, s.mut, s.rfield, s.c1h, s.c2h, *mw)
+                s.t_save = rb(s.rfield, s.t_save, 't', 't')
+                mu_tend_e = rb(mu_e, mu_tend_e, 'mu', 'm', ix_mu)
             s.mu_tend = mu_tend_e[0, :, :] + 0.
         s.ru_tend, s.rv_tend, s.rw_tend, s.ph_tend, s.t_tend, s.mu_tend = o.rk_addtend_dry(
             s.ru_tend, s.rv_tend, s.rw_tend, s.ph_tend, s.t_tend, s.ru_tendf, s.rv_tendf, s.rw_tendf, s.ph_tendf,

@@ -316,6 +316,36 @@ def spec_bdytend_group(items, idx24, idx2d):
     call("pywrf_spec_bdytend_group", g3, g2, n, tends, bt, flags, kinds, stream())
 
 
+def relax_group(items, dtbc, fcx, gcx, idx24, idx2d, weight_idx24):
+    """A run of relax_bdytend calls on distinct tendencies in one launch.
+    items: [(field, mass, field_tend, (bxs, bxe, bys, bye, btxs, btxe, btys,
+    btye), variable, is_2d)], mass None or the plane that mass_weight (index
+    set weight_idx24) multiplies the field by first; dtbc a one-value device
+    tensor; idx24 / idx2d: the index tuples the individual calls would take.
+    Same result as the calls in order.  Not part of the reference API."""
+    import ctypes
+    n = len(items)
+    if not _on_device(dtbc):
+        raise TypeError("relax_group: dtbc must be a device tensor")
+    f3 = next(f for f, _, _, _, _, two in items if not two)
+    g3 = grid(f3.shape, _I24(*idx24))
+    g2 = grid((1,) + tuple(f3.shape[-2:]), _I24(*idx2d))
+    gw = grid(f3.shape, _I24(*weight_idx24))
+    for f, m, t, _, _, two in items:
+        check_operands("relax_group", (g2 if two else g3).contents, ("field", "tend"), (ptr(f), ptr(t)))
+        if m is not None and tuple(m.shape) != tuple(f3.shape[-2:]):
+            raise ValueError("relax_group: a mass plane of shape %s" % (tuple(m.shape),))
+    fields = (ctypes.c_void_p * n)(*[ptr(f).value for f, _, _, _, _, _ in items])
+    masses = (ctypes.c_void_p * n)(*[None if m is None else ptr(m).value for _, m, _, _, _, _ in items])
+    tends = (ctypes.c_void_p * n)(*[ptr(t).value for _, _, t, _, _, _ in items])
+    bps = [p for _, _, _, arrs, _, two in items for p in _bdy(g2 if two else g3, tuple(arrs))]
+    bdys = (ctypes.c_void_p * (8 * n))(*[p.value for p in bps])
+    flags = b"".join(v.encode() for _, _, _, _, v, _ in items)
+    kinds = (ctypes.c_int * n)(*[1 if two else 0 for _, _, _, _, _, two in items])
+    call("pywrf_relax_group_dtbc_dev", g3, g2, gw, n, fields, masses, tends, bdys, flags, kinds, ptr(dtbc), ptr(fcx),
+         ptr(gcx), stream())
+
+
 def spec_bdy_final_group(items, dtbc, idx24):
     """A run of spec_bdy_final calls on distinct fields in one launch.
     items: [(field, mu, msf, (bxs, bxe, bys, bye, btxs, btxe, btys, btye),
