@@ -160,6 +160,27 @@ class NanFlag:
                                      % (self.WHERE.get(code, code), count, k, j, i))
 
 
+# the calls that the merged forms stand for, by the module of the library that has them
+MERGED_CALLS = {
+    "stage_prep": ("calculate_full", "calc_mu_uv", "couple_momentum", "calc_ww_cp", "calc_cq", "calc_alt", "calc_php",
+                   "advance_uv", "advance_mu_t", "sumflux", "calc_p_rho", "set_physical_bc3d", "set_physical_bc2d",
+                   "set_physical_bc_group", "advance_uv_zone", "advance_mu_t_zone", "sumflux_zone", "calc_p_rho_bc"),
+    "relax_group": ("spec_bdyupdate", "spec_bdyupdate_group", "spec_bdyupdate_ph", "zero_grad_bdy",
+                    "spec_bdyupdate_ph_zero_grad", "relax_bdytend", "mass_weight"),
+}
+
+
+def offers_merged(ops):
+    """Whether ops has the merged calls and, beside them, the library's own
+    versions of every call they stand for: where a caller has replaced or
+    wrapped one of those, the step makes the calls one by one."""
+    for name, calls in MERGED_CALLS.items():
+        own = getattr(getattr(ops, name, None), "__globals__", None)
+        if own is None or any(getattr(ops, c, None) is not own.get(c) for c in calls):
+            return False
+    return True
+
+
 def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
     """Advance state `s` (a namespace of tensors, see pywrf_amd.state) by one
     RK3 step using the functions in `ops`.  solver.py:454-1910.  With a
@@ -179,7 +200,7 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
     grouped_upd = hasattr(o, "spec_bdyupdate_group")
     # the forms that merge several calls: where the launch itself counts (a graph's node is about 5 us), and only
     # there, so that a step made call by call keeps the calls that a caller may replace or record
-    merged = clock is not None and hasattr(o, "advance_uv_zone")
+    merged = clock is not None and offers_merged(o)
 
     def bcs(*items):
         """A run of consecutive open-boundary fills, items (tensor, flag, is_2d);
