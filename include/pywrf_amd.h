@@ -174,6 +174,13 @@ int pywrf_advect_v_fresh(const pywrf_grid_t* g, const float* v, float* tendency,
 int pywrf_advect_w_fresh(const pywrf_grid_t* g, const float* w, float* tendency, const float* ru, const float* rv,
                          const float* rom, const float* msftx, const float* fzm, const float* fzp, double rdx,
                          double rdy, const float* rdzu, pywrf_stream_t s);
+/* advect_u_fresh, advect_v_fresh and advect_w_fresh (distinct tendencies) in one launch; rdzw as in the first two,
+ * rdzu as in the third.  No counterpart in the reference: a batching. */
+int pywrf_advect_uvw_fresh(const pywrf_grid_t* g, const float* u, float* u_tend, const float* v, float* v_tend,
+                           const float* w, float* w_tend, const float* ru, const float* rv, const float* rom,
+                           const float* msfux, const float* msfvx, const float* msfvy, const float* msftx,
+                           const float* fzm, const float* fzp, double rdx, double rdy, const float* rdzw,
+                           const float* rdzu, pywrf_stream_t s);
 int pywrf_advect_scalar_fresh(const pywrf_grid_t* g, const float* field, float* tendency, const float* ru,
                               const float* rv, const float* rom, const float* msftx, const float* fzm,
                               const float* fzp, double rdx, double rdy, const float* rdzw, pywrf_stream_t s);

@@ -721,7 +721,7 @@ SUBSTEP_CALLS = ("advance_uv", "spec_bdyupdate_group", "advance_mu_t", "spec_bdy
 
 # calls that merge several of the recorded ones; a recorder does not offer them, so the step makes each call itself
 MERGED = frozenset(("advance_uv_zone", "advance_mu_t_zone", "sumflux_zone", "stage_prep",
-                    "calc_p_rho_bc", "relax_group"))
+                    "calc_p_rho_bc", "relax_group", "advect_uvw_fresh"))
 
 
 class _LoopRecorder:

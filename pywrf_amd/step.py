@@ -164,7 +164,9 @@ class NanFlag:
 MERGED_CALLS = {
     "stage_prep": ("calculate_full", "calc_mu_uv", "couple_momentum", "calc_ww_cp", "calc_cq", "calc_alt", "calc_php",
                    "advance_uv", "advance_mu_t", "sumflux", "calc_p_rho", "set_physical_bc3d", "set_physical_bc2d",
-                   "set_physical_bc_group", "advance_uv_zone", "advance_mu_t_zone", "sumflux_zone", "calc_p_rho_bc"),
+                   "set_physical_bc_group", "advance_uv_zone", "advance_mu_t_zone", "sumflux_zone", "calc_p_rho_bc",
+                   "advect_u", "advect_v", "advect_w", "advect_u_fresh", "advect_v_fresh", "advect_w_fresh",
+                   "advect_uvw_fresh"),
     "relax_group": ("spec_bdyupdate", "spec_bdyupdate_group", "spec_bdyupdate_ph", "zero_grad_bdy",
                     "spec_bdyupdate_ph_zero_grad", "relax_bdytend", "mass_weight"),
 }
@@ -306,9 +308,13 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
         adv_u, adv_v, adv_w, adv_s, rhs = ((o.advect_u_fresh, o.advect_v_fresh, o.advect_w_fresh,
                                             o.advect_scalar_fresh, o.rhs_ph_fresh) if fresh else
                                            (o.advect_u, o.advect_v, o.advect_w, o.advect_scalar, o.rhs_ph))
-        s.ru_tend = adv_u(s.u, s.u, s.ru_tend, s.ru, s.rv, s.ww, *adv, s.rdnw, *I18)
-        s.rv_tend = adv_v(s.v, s.v, s.rv_tend, s.ru, s.rv, s.ww, *adv, s.rdnw, *I18)
-        s.rw_tend = adv_w(s.w, s.w, s.rw_tend, s.ru, s.rv, s.ww, *adv, s.rdn, *I18)
+        winds = ((s.u, s.u, s.ru_tend, s.ru, s.rv, s.ww, *adv, s.rdnw, *I18),
+                 (s.v, s.v, s.rv_tend, s.ru, s.rv, s.ww, *adv, s.rdnw, *I18),
+                 (s.w, s.w, s.rw_tend, s.ru, s.rv, s.ww, *adv, s.rdn, *I18))
+        if merged:
+            o.advect_uvw_fresh(*winds)
+        else:
+            s.ru_tend, s.rv_tend, s.rw_tend = adv_u(*winds[0]), adv_v(*winds[1]), adv_w(*winds[2])
         s.t_tend = adv_s(s.t, s.t, s.t_tend, s.ru, s.rv, s.ww, *adv, s.rdnw, *I18)
         s.ph_tend = rhs(s.ph_tend, s.u, s.v, s.ww, s.ph, s.ph, s.phb, s.w, s.mut, s.muu, s.muv, s.c1f, s.c2f,
                         s.fnm, s.fnp, s.rdnw, s.cfn, s.cfn1, rdx, rdy, s.msfux, s.msfuy, s.msfvx, s.msfvx_inv,

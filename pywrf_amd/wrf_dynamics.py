@@ -370,6 +370,25 @@ def advect_w_fresh(*args):
     return _advect_w("pywrf_advect_w_fresh", **vars(_bind(advect_w, args)))
 
 
+def advect_uvw_fresh(u_args, v_args, w_args):
+    """advect_u_fresh, advect_v_fresh and advect_w_fresh, each given as the
+    tuple of its positional arguments, in one launch; the mass fluxes, map
+    factors, grid and index set must be the same.  Returns the three calls'
+    results.  Not part of the reference API."""
+    a, b, c = _bind(advect_u, u_args), _bind(advect_v, v_args), _bind(advect_w, w_args)
+    shared = ("ru", "rv", "rom", "msfux", "msfvx", "msfvy", "msftx", "fzm", "fzp")
+    idx = ("rdx", "rdy", "ids", "ide", "jds", "jde", "kds", "kde", "ims", "ime", "jms", "jme", "kms", "kme", "its",
+           "ite", "jts", "jte", "kts", "kte")
+    if (any(getattr(a, n) is not getattr(b, n) or getattr(a, n) is not getattr(c, n) for n in shared)
+            or any(getattr(a, n) != getattr(b, n) or getattr(a, n) != getattr(c, n) for n in idx) or a.rdzw is not b.rdzw):
+        raise ValueError("advect_uvw_fresh: the three calls do not share their common arguments")
+    call("pywrf_advect_uvw_fresh", grid(a.u.shape, tuple(getattr(a, n) for n in idx[2:])), ptr(a.u), ptr(a.tendency),
+         ptr(b.v), ptr(b.tendency), ptr(c.w), ptr(c.tendency), ptr(a.ru), ptr(a.rv), ptr(a.rom), ptr(a.msfux),
+         ptr(a.msfvx), ptr(a.msfvy), ptr(a.msftx), ptr(a.fzm), ptr(a.fzp), float(a.rdx), float(a.rdy), ptr(a.rdzw),
+         ptr(c.rdzu), stream())
+    return a.tendency, b.tendency, c.tendency
+
+
 def advect_scalar(field, field_old, tendency,
                   ru, rv, rom,
                   c1, c2,
