@@ -634,6 +634,14 @@ __global__ void __launch_bounds__(TB) k_advance_mu_t(Dims D, AdvMuT a, UpdJob zt
       a.t[q] = ZONE ? spec_upd_value(zt, k, j, i, y[m], t[m]) : y[m];
       a.t_ave[q] = z[m];
     }
+    // LPT is chosen for the kte - 1 levels of the box; the arrays may hold more
+    for (int k = grp + (LPT + 1) * TG; k < nz; k += TG) {
+      const long q = D.ix(k, j, i);
+      const float wk = a.ww_in[q], tk = a.t_in[q], ak = a.t_ave_in[q];
+      a.ww[q] = wk;
+      a.t[q] = ZONE ? spec_upd_value(zt, k, j, i, tk, a.ft[q]) : tk;
+      a.t_ave[q] = ak;
+    }
   }
   if (!row) return;   // the whole block
   const int ic = imin(imax(i, a.i0), a.i1 - 1);   // lanes outside the box load (and drop) its edge column's values

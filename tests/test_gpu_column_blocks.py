@@ -59,3 +59,48 @@ def test_level_and_row_edges(name, nz, nx):
     bound = 0.0 if name == "advance_mu_t" else 1e-4
     for n, (x, y) in enumerate(zip(got, want)):
         assert rel_err(x.cpu(), y) <= bound, (name, n)
+
+
+def _poison(*tensors):
+    """Fill the allocator's free blocks of the tensors' sizes with NaN, so that a point a call leaves
+    unwritten in its fresh results does not hold an earlier result."""
+    blocks = [torch.full_like(t, float("nan")) for _ in range(4) for t in tensors]
+    torch.cuda.synchronize()
+    del blocks
+
+
+def _same(x, y):
+    x, y = x.cpu(), y.cpu()
+    return torch.equal(torch.nan_to_num(x, nan=3e38), torch.nan_to_num(y, nan=3e38))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nz,kte", [(49, 41), (60, 41), (73, 65), (80, 60), (128, 17), (128, 66)])
+def test_arrays_with_more_levels_than_the_index_set(nz, kte):
+    """advance_mu_t copies every level of the columns it does not update, and those above kte of the others:
+    its results against the oracle's, and with the zone's updates against the four single calls."""
+    import oracle
+    import pywrf_amd
+    from pywrf_amd.step import Grid
+    from pywrf_amd.step import SPEC_ZONE
+    ny, nx = 27, 69
+    ops, fn = pywrf_amd.ops(), oracle.ops().advance_mu_t
+    g = Grid(nz, ny, nx)
+    g.kde = g.kte = g.kpe = kte
+    args = _args(fn, nz, ny, nx, 7 * nz + kte)[:-18] + list(g.ix18)
+    dev = [a.cuda() if isinstance(a, torch.Tensor) else a for a in args]
+    want = fn(*[a.clone() if isinstance(a, torch.Tensor) else a for a in args])
+    _poison(dev[0], dev[6])
+    got = ops.advance_mu_t(*dev)
+    for n, (x, y) in enumerate(zip(got, want)):
+        assert rel_err(x.cpu(), y) == 0.0, n
+    ix2d = tuple(0 if n in (4, 5, 10, 11, 16, 17, 22, 23) else v for n, v in enumerate(g.ix24))
+    dt, t, muts, mu = 13.5, got[2], got[8], got[10]
+    ft, mu_tend = dev[27], dev[28]
+    ops.spec_bdyupdate(t, ft, dt, "t", SPEC_ZONE, *g.ix24)
+    ops.spec_bdyupdate(mu, mu_tend, dt, "m", SPEC_ZONE, *ix2d)
+    ops.spec_bdyupdate(muts, mu_tend, dt, "m", SPEC_ZONE, *ix2d)
+    _poison(dev[0], dev[6])
+    zone = ops.advance_mu_t_zone(tuple(dev), dt, g.ix24, ix2d)
+    for n, (x, y) in enumerate(zip(zone, got)):
+        assert _same(x, y), n
