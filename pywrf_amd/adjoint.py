@@ -807,7 +807,9 @@ class AcousticSubstep(torch.autograd.Function):
     fills, and their adjoints in the opposite order, as one node.  The calls
     that work in place do so on arrays the substep made itself: what they
     change (the zone's ring, the halos) is not what the adjoints of the calls
-    before them read, except f_in of spec_bdyupdate_ph, which is kept.  A node
+    before them read, except f_in of spec_bdyupdate_ph, which is kept.  Of the
+    results w, ph, mu and muts, which a caller may write into, the backward
+    reads copies of its own.  A node
     per call cost a copy of every such array and an addition for every value
     that two calls read: 555 launches for a stage of four substeps, forward
     twice and backward, against 291 (at 120 x 120 x 41 8.8 against 6.1 ms,
@@ -820,6 +822,10 @@ class AcousticSubstep(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, calls, given, saved, *inputs):
+        return AcousticSubstep._run(ctx, calls, given, saved, inputs, copies=True)
+
+    @staticmethod
+    def _run(ctx, calls, given, saved, inputs, copies):
         from . import wrf_boundary, wrf_dynamics
         inputs = [_f32(t) for t in inputs]
         st = dict(zip(ACOUSTIC_STATE, inputs))
@@ -861,23 +867,28 @@ class AcousticSubstep(torch.autograd.Function):
         zone(z2, (t, mu, muts), tends[2:])
         put(wa, AdvanceW.DIFF, (st["w"], st["ph"], t, t_ave, u, v, muts, muave, ww))
         t2a, w, ph = wrf_dynamics.advance_w(*wa)
-        f_in, pm1, ru_m, rv_m, ww_m = _copies(ph, st["pm1"], st["ru_m"], st["rv_m"], st["ww_m"])
+        # what is updated in place below and, with copies, what the backward reads of w, mu and muts
+        own = (w, mu, muts)
+        f_in, pm1, ru_m, rv_m, ww_m, *kept = _copies(ph, st["pm1"], st["ru_m"], st["rv_m"], st["ww_m"],
+                                                     *(own if copies else ()))
+        w_kept, mu_kept, muts_kept = kept or own
         put(sf, SumFlux.DIFF, (u, v, ww, ru_m, rv_m, ww_m))
         wrf_dynamics.sumflux(*sf)
-        ph_args[1], ph_args[4], zg_args[0] = ph, muts, w
+        wa[AdvanceW.MUTS] = muts_kept
+        ph_args[1], ph_args[4], zg_args[0] = ph, muts_kept, w
         if tuple(ph_args[10:]) == tuple(zg_args[3:]) and ph_args[9] == zg_args[2]:
             wrf_boundary.spec_bdyupdate_ph_zero_grad(tuple(ph_args), tuple(zg_args))
         else:
             wrf_boundary.spec_bdyupdate_ph(*ph_args)
             wrf_boundary.zero_grad_bdy(*zg_args)
-        put(cp, CalcPRho.DIFF, (st["al"], st["p"], ph, t, pm1, mu, muts))
+        put(cp, CalcPRho.DIFF, (st["al"], st["p"], ph.clone() if copies else ph, t, pm1, mu_kept, muts_kept))
         al, p, pm1 = wrf_dynamics.calc_p_rho(*cp)
         items, ix24, ix2d = bc
         kinds = [(k, two) for _, k, two in items]
         wrf_dynamics.set_physical_bc_group([(f, k, two) for f, (k, two) in zip((ph, al, p, muts, mu, mudf), kinds)],
                                            ix24, ix2d)
         ctx.calls = uv, z1, mt, z2, wa, sf, ph_args, zg_args, cp, (kinds, ix24, ix2d)
-        ctx.kept = ww, t2a, w, f_in, tends
+        ctx.kept = ww, t2a, w_kept, f_in, tends
         ctx.given, ctx.saved = given, saved
         ctx.set_materialize_grads(False)
         new = {"u": u, "v": v, "p": p, "ph": ph, "al": al, "mu": mu, "mudf": mudf, "ww": ww, "muave": muave,
@@ -985,15 +996,23 @@ class AcousticSubstep(torch.autograd.Function):
         return (None, None, None, *res)
 
 
-def acoustic_substep(x, calls, forcing=None, saved=None):
+class _InnerSubstep(AcousticSubstep):
+    """AcousticSubstep without copies: for a chain whose results no caller
+    gets hold of before its backward has run (the checkpointed forms')."""
+
+    @staticmethod
+    def forward(ctx, calls, given, saved, *inputs):
+        return AcousticSubstep._run(ctx, calls, given, saved, inputs, copies=False)
+
+
+def acoustic_substep(x, calls, forcing=None, saved=None, _node=AcousticSubstep):
     """One acoustic substep (AcousticSubstep).  x: the 17 carried fields
     (ACOUSTIC_STATE order); calls: the nine recorded calls' arguments;
     forcing: None, or the six large-step tendencies (FORCING order) to use,
     and differentiate, in place of the recorded ones wherever the substep
     reads them; saved: the same for the six saved fields (SAVED order).
     Returns the 17 fields after the substep."""
-    return list(AcousticSubstep.apply(calls, forcing is not None, saved is not None, *x, *(forcing or ()),
-                                      *(saved or ())))
+    return list(_node.apply(calls, forcing is not None, saved is not None, *x, *(forcing or ()), *(saved or ())))
 
 
 STAGE_IN = ("u_2", "v_2", "w_2", "t_2", "ph_2", "mu_2", "u_1", "v_1", "w_1", "t_1", "ph_1", "mu_1", "ww", "mudf",
@@ -1046,7 +1065,7 @@ def record_acoustic_stage(s, ops, cfg, stage=2):
     return x, calls
 
 
-def acoustic_stage(x, calls):
+def acoustic_stage(x, calls, _node=AcousticSubstep):
     """The acoustic part of an RK stage past the first, as autograd Functions
     (small_step_prep, calc_p_rho at step 0, the open-boundary fills, the
     acoustic substeps, calc_mu_uv_1, small_step_finish); x: STAGE_IN, calls:
@@ -1069,7 +1088,7 @@ def acoustic_stage(x, calls):
           v["ww_m"]]
     saved = [us, vs, ws, ts, ps, ww1]
     for c in subs:
-        st = acoustic_substep(st, c, None, saved)
+        st = acoustic_substep(st, c, None, saved, _node)
     st = dict(zip(ACOUSTIC_STATE, st))
     muus, muvs = CalcMuUV1.apply(st["muts"], muus, muvs, mc)
     uo, vo, wo, pho, wwo, to, muo = SmallStepFinish.apply(
@@ -1109,7 +1128,7 @@ class AcousticLoop(torch.autograd.Function):
         n, m = len(ACOUSTIC_STATE), len(ACOUSTIC_STATE) + len(FORCING)
         x, forcing, saved = list(inputs[:n]), inputs[n:m] or None, inputs[m:] or None
         for calls in substeps:
-            x = acoustic_substep(x, calls, forcing, saved)
+            x = acoustic_substep(x, calls, forcing, saved, _InnerSubstep)
         return x
 
     @staticmethod
@@ -1276,14 +1295,14 @@ class AcousticStage(torch.autograd.Function):
         ctx.calls = calls
         ctx.save_for_backward(*x)
         with torch.no_grad():
-            y = acoustic_stage(list(x), calls)
+            y = acoustic_stage(list(x), calls, _InnerSubstep)
         return tuple(y)
 
     @staticmethod
     def backward(ctx, *lams):
         x = [t.detach().requires_grad_() for t in ctx.saved_tensors]
         with torch.enable_grad():
-            y = acoustic_stage(x, ctx.calls)
+            y = acoustic_stage(x, ctx.calls, _InnerSubstep)
             pairs = [(o, l) for o, l in zip(y, lams) if l is not None]
             grads = torch.autograd.grad([o for o, _ in pairs], x, [l for _, l in pairs], allow_unused=True)
         return (None, *grads)
