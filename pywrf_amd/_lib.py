@@ -9,6 +9,7 @@ ImportError at import time -- there is no fallback path.
 import ctypes
 import os
 import re
+import weakref
 
 import torch
 
@@ -288,7 +289,8 @@ def boundary_layout(t, kind, kz, n):
     (kz, 5, n)) as a contiguous (5, kz, n) array -- the layout of the
     driver's own permuted views (solver.py:468-703), which are used in place.
     Arrays in any other layout are copied into that layout; the copy is kept
-    while the array's data and version are unchanged."""
+    while the array (or the tensor it is a view of) lives and its version is
+    unchanged: after that another array may have its address."""
     _require_device(t)
     want = (kz, n, 5) if kind == "x" else (kz, 5, n)
     if t.shape != want:
@@ -297,14 +299,15 @@ def boundary_layout(t, kind, kz, n):
     if t.stride() == strides or t.numel() == 0:
         return t
     key = (t.data_ptr(), tuple(t.stride()), kind)
+    owner = t if t._base is None else t._base
     hit = _bdy_copies.get(key)
-    if hit is not None and hit[0] == t._version:
-        return hit[1]
+    if hit is not None and hit[0]() is owner and hit[1] == t._version:
+        return hit[2]
     c = (t.permute(2, 0, 1) if kind == "x" else t.permute(1, 0, 2)).contiguous()
     c = c.permute(1, 2, 0) if kind == "x" else c.permute(1, 0, 2)
     if len(_bdy_copies) > 256:
         _bdy_copies.clear()
-    _bdy_copies[key] = (t._version, c)
+    _bdy_copies[key] = (weakref.ref(owner), t._version, c)
     return c
 
 
