@@ -323,8 +323,9 @@ __device__ inline void prep_ww(const Dims& D, const StagePrep& a, float* s_dv, f
   const int j = a.wb.j0 + (int)blockIdx.x / a.nbx, i = a.wb.i0 + (int)blockIdx.x % a.nbx * WW_TI + lane;
   const bool ok = i < a.wb.i1;
   if (ok) {
-    const float ue = prep_muu(D, a, j, i + 1), uw = prep_muu(D, a, j, i), vn = prep_muv(D, a, j + 1, i),
-                vs = prep_muv(D, a, j, i);
+    // the faces beyond a tile that ends inside the domain are not calc_mu_uv's: what the arrays hold there
+    const float ue = i + 1 < a.ite ? prep_muu(D, a, j, i + 1) : AT2(a.muu, j, i + 1), uw = prep_muu(D, a, j, i);
+    const float vn = j + 1 < a.jte ? prep_muv(D, a, j + 1, i) : AT2(a.muv, j + 1, i), vs = prep_muv(D, a, j, i);
     const float fe = AT2(a.ww.msfuy, j, i + 1), fw = AT2(a.ww.msfuy, j, i), xn = AT2(a.ww.msfvx_inv, j + 1, i),
                 xs = AT2(a.ww.msfvx_inv, j, i), mx = AT2(a.ww.msftx, j, i);
 #pragma unroll 6
