@@ -788,6 +788,8 @@ __global__ void __launch_bounds__(CA_THREADS) k_advance_mu_t_adj(Box b, Dims D, 
     r.u = at_b(a.u, o); r.ue = at_b(a.u, oe); r.v = at_b(a.v, o); r.vn = at_b(a.v, on);
     return r;
   };
+  // a share of nothing, whatever the other factor holds: the forward does not read it there
+  auto times = [](float share, float x) { return share != 0.0f ? share * x : 0.0f; };
   const int kt = imin(ka + L, D.nz);   // the run's top, above the mass levels too
   if (ka >= kt) return;
   MuTLevel x = load(kt - 1), y = load(kt - 2);
@@ -812,16 +814,16 @@ __global__ void __launch_bounds__(CA_THREADS) k_advance_mu_t_adj(Box b, Dims D, 
     const float duw = lane_below(du), qw = lane_below(q);
     const float hx = 0.5f * a.rdx, hy = 0.5f * a.rdy;
     // t_1 in the horizontal theta fluxes, and in the vertical flux wdtn[k] = ww'[k] (fnm[k] t_1[k] + fnp[k] t_1[k-1])
-    float gt1 = hx * ((qw - q) * x.u + (q - qe) * x.ue) + hy * ((qs - q) * x.v + (q - qn) * x.vn);
+    float gt1 = hx * (times(qw - q, x.u) + times(q - qe, x.ue)) + hy * (times(qs - q, x.v) + times(q - qn, x.vn));
     const float wl = lwd * x.wwo;
     if (inl) gt1 += (k >= 1 ? wl * level(a.fnm, k) : 0.0f) + up;
     up = k >= 1 ? wl * level(a.fnp, k) : 0.0f;
     if (own) {
       const long p = D.ix(k, j, i);
-      a.gu[p] = (duw - du) + (qw - q) * hx * (x.t1 + x.t1w);
-      a.gv[p] = (dvs - dv) + (qs - q) * hy * (x.t1 + x.t1s);
-      a.gu1[p] = (duw - du) * uc;
-      a.gv1[p] = (dvs - dv) * vc;
+      a.gu[p] = (duw - du) + times((qw - q) * hx, x.t1 + x.t1w);
+      a.gv[p] = (dvs - dv) + times((qs - q) * hy, x.t1 + x.t1s);
+      a.gu1[p] = times(duw - du, uc);
+      a.gv1[p] = times(dvs - dv, vc);
       a.gt1[p] = gt1;
       a.gww[p] = inl ? (k == 0 ? R : 0.0f) : x.lww;
       a.gww1[p] = inl ? -lwk : 0.0f;             // ww' = ww - ww_1

@@ -69,3 +69,33 @@ def test_sum_group_adds_in_order(n):
     _sums((x, (a, b, c, d)), (y, (off, b)), (z, (z, a)))
     for got, w in zip((x, y, z), want):
         assert torch.equal(got, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx", [24, 69])
+def test_advance_mu_t_adjoint_of_values_the_forward_never_reads(nx):
+    """NaN around the columns advance_mu_t updates and above its levels reaches no gradient."""
+    import oracle
+    from pywrf_amd import adjoint
+    from pywrf_amd.step import Grid
+    from test_gpu_column_blocks import _args
+    nz, ny = 11, 27
+    g = Grid(nz, ny, nx)
+    args = [a.cuda() if isinstance(a, torch.Tensor) else a
+            for a in _args(oracle.ops().advance_mu_t, nz, ny, nx, nx)]
+    read = torch.zeros(nz, ny, nx, dtype=torch.bool, device="cuda")
+    read[:nz - 1, g.jds:g.jde - 1, g.ids:g.ide - 1] = True     # the box's columns and their neighbours
+    gen = torch.Generator(device="cuda").manual_seed(nx)
+    D, E = adjoint.AdvanceMuT.DIFF, adjoint.AdvanceMuT.EXTRA
+    grads = []
+    for fill in (0.0, float("nan")):
+        a = list(args)
+        for n in (1, 2, 3, 4, 5, 10, 11, 25, 27):              # ww_1, u, u_1, v, v_1, muu, muv, t_1, ft
+            a[n] = torch.where(read if a[n].dim() == 3 else read[0], a[n], fill)
+        x = [a[n].clone().requires_grad_() for n in D + E]
+        out = adjoint.AdvanceMuT.apply(*x[:len(D)], a, *x[len(D):])
+        if not grads:
+            lams = [torch.randn(o.shape, device="cuda", generator=gen) for o in out]
+        grads.append(torch.autograd.grad(out, x, lams))
+    for n, p, q in zip(D + E, *grads):
+        assert torch.equal(p, q), n
