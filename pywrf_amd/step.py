@@ -240,23 +240,24 @@ def rk3_step(s, ops, cfg, check_nan=False, clock=None, nan_flag=None):
         else:
             dt_rk, dts_rk, nsmall = dtm, dts, cfg.soundsteps
         # rk_step_prep (solver.py:736-778)
-        prep = ((s.mut, s.mub, s.mu, *I18), (s.mu, s.mub, s.muu, s.muv, *I18),
-                (s.muu, s.ru, s.u, s.msfu, s.muv, s.rv, s.v, s.msfv, s.msfvx_inv, s.mut, s.rw, s.w, s.msft, s.c1h,
-                 s.c2h, s.c1f, s.c2f, *I18),
-                (s.u, s.v, s.mu, s.mub, s.muu, s.muv, s.c1h, s.c2h, s.ww, rdx, rdy, s.msftx, s.msfty, s.msfux,
-                 s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.dnw, *I18),
-                (s.moist, s.cqu, s.cqv, s.cqw, N_MOIST, *I18), (s.alt, s.al, s.alb, *I18), (s.php, s.ph, s.phb, *I18))
+        full = lambda: (s.mut, s.mub, s.mu, *I18)
+        mass = lambda: (s.mu, s.mub, s.muu, s.muv, *I18)
+        couple = lambda: (s.muu, s.ru, s.u, s.msfu, s.muv, s.rv, s.v, s.msfv, s.msfvx_inv, s.mut, s.rw, s.w, s.msft,
+                          s.c1h, s.c2h, s.c1f, s.c2f, *I18)
+        omega = lambda: (s.u, s.v, s.mu, s.mub, s.muu, s.muv, s.c1h, s.c2h, s.ww, rdx, rdy, s.msftx, s.msfty, s.msfux,
+                         s.msfuy, s.msfvx, s.msfvx_inv, s.msfvy, s.dnw, *I18)
+        cq = lambda: (s.moist, s.cqu, s.cqv, s.cqw, N_MOIST, *I18)
+        alt, php = lambda: (s.alt, s.al, s.alb, *I18), lambda: (s.php, s.ph, s.phb, *I18)
         if merged:
-            o.stage_prep(*prep)
+            o.stage_prep(full(), mass(), couple(), omega(), cq(), alt(), php())
         else:
-            full, mass, couple, omega, cq, alt, php = prep
-            s.mut = o.calculate_full(*full)
-            s.muu, s.muv = o.calc_mu_uv(*mass)
-            s.ru, s.rv, s.rw = o.couple_momentum(*couple)
-            s.ww = o.calc_ww_cp(*omega)
-            s.cqu, _cuv, s.cqw = o.calc_cq(*cq)
-            s.alt = o.calc_alt(*alt)
-            s.php = o.calc_php(*php)
+            s.mut = o.calculate_full(*full())
+            s.muu, s.muv = o.calc_mu_uv(*mass())
+            s.ru, s.rv, s.rw = o.couple_momentum(*couple())
+            s.ww = o.calc_ww_cp(*omega())
+            s.cqu, _cuv, s.cqw = o.calc_cq(*cq())
+            s.alt = o.calc_alt(*alt())
+            s.php = o.calc_php(*php())
         # rk_phys_bc_dry_1 (solver.py:781-843)
         (s.ru, s.rv, s.rw, s.ww, s.php, s.alt, s.p, s.muu, s.muv, s.mut, s.al, s.ph) = bcs(
             (s.ru, 'u', 0), (s.rv, 'v', 0), (s.rw, 'w', 0), (s.ww, 'w', 0), (s.php, 'w', 0), (s.alt, 't', 0),
