@@ -175,10 +175,11 @@ MERGED_CALLS = {
 def offers_merged(ops):
     """Whether ops has the merged calls and, beside them, the library's own
     versions of every call they stand for: where a caller has replaced or
-    wrapped one of those, the step makes the calls one by one."""
+    wrapped one of those, in ops or in the module it comes from, the step
+    makes the calls one by one."""
     for name, calls in MERGED_CALLS.items():
-        own = getattr(getattr(ops, name, None), "__globals__", None)
-        if own is None or any(getattr(ops, c, None) is not own.get(c) for c in calls):
+        own = getattr(getattr(ops, name, None), "__globals__", {}).get("_OWN")
+        if own is None or any(getattr(ops, c, None) is not own.get(c) for c in (name, *calls)):
             return False
     return True
 

@@ -418,3 +418,7 @@ def boundary_epilogue(bc_items, final_items, dtbc, idx24, idx2d):
     else:
         call("pywrf_boundary_epilogue", g3, g2, n, fields, flags, kinds, m, fin, mus, msfs, bdys, fflags,
              float(dtbc), stream())
+
+
+# the functions as defined above, whatever a program puts in their place later (step.offers_merged)
+_OWN = {n: f for n, f in list(globals().items()) if getattr(f, "__module__", None) == __name__}

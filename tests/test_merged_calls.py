@@ -36,3 +36,19 @@ def test_the_recorders_and_the_oracle_do_not_offer_them():
     assert not offers_merged(_LoopRecorder(pywrf_amd.ops(), 1))
     assert not offers_merged(_StageRecorder(pywrf_amd.ops(), 2))
     assert not offers_merged(oracle.ops())
+
+
+@pytest.mark.parametrize("name", _names())
+def test_a_call_replaced_in_its_module_is_called(name, monkeypatch):
+    """ops() takes its functions from the modules: a wrapper put there is the ops' and the module's alike."""
+    import functools
+    import pywrf_amd
+    from pywrf_amd import wrf_boundary, wrf_dynamics
+    from pywrf_amd.step import offers_merged
+    mod = next(m for m in (wrf_dynamics, wrf_boundary) if hasattr(m, name))
+    own = getattr(mod, name)
+    monkeypatch.setattr(mod, name, functools.wraps(own)(lambda *a: own(*a)))
+    assert getattr(pywrf_amd.ops(), name) is not own
+    assert not offers_merged(pywrf_amd.ops())
+    monkeypatch.undo()
+    assert offers_merged(pywrf_amd.ops())
