@@ -1258,6 +1258,7 @@ class SurrogateNet(torch.autograd.Function):
         M = X.shape[0]
         if M % 32:
             raise ValueError("batch size must be a multiple of 32")
+        X = X.expand(M, _sg.FIN)       # raises for another width (the conversion below pads a narrower one with zeros)
         bf = dict(dtype=torch.bfloat16, device=X.device)
         H1, H2 = torch.empty(M, _sg.HID, **bf), torch.empty(M, _sg.HID, **bf)
         Y = torch.empty(M, _sg.FOUT, device=X.device)

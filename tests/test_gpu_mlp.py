@@ -190,3 +190,11 @@ def test_mse_rows_of_any_length(N, ldy):
     want = (2.0 * w[:N] * (Y - T)[:, :N] * 0.01)
     assert float((dY[:, :N].float() - want).abs().max()) <= 2 ** -8 * float(want.abs().max())
     assert bool((dY[:, N:] == 0).all())
+
+
+@pytest.mark.parametrize("shape", [(32, 368), (32, 370), (32, 384), (64, 2), (32, 369, 1), (32,)])
+def test_column_network_refuses_other_widths(shape):
+    from pywrf_amd import adjoint, surrogate as sg
+    net = sg.MLP(seed=1)
+    with pytest.raises((ValueError, RuntimeError)):
+        adjoint.SurrogateNet.apply(torch.zeros(shape, device="cuda"), net)
