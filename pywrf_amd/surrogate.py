@@ -210,14 +210,24 @@ def forward(net, X, ws):
     return ws.Y[:M]
 
 
+def weight_splits(M):
+    """Splits of a weight gradient's sum over a batch of M columns.  A
+    workgroup's time is its chain of 64-column slabs, M / 64 / splits of them,
+    plus the splits' atomic adds to its tile, which meet in memory: least near
+    the square root of the slabs.  From 32 splits of 12 to 16 tiles on every CU
+    has its workgroups, and more splits only add.  us a product, the mean of the
+    three layers': 1024 columns 1 split 17.0, 4 7.7, 8 8.2; 8192 columns 8 19.1,
+    12 17.2, 32 26.3; 65536 columns 8 106, 32 62, 64 77; 262144 columns 8 517,
+    32 207, 64 215."""
+    return max(1, min(32, math.isqrt(max(M // 64 - 1, 0)) + 1))
+
+
 def backward(net, X, T, w, ws, wsum, ksplit=None):
     """Loss and parameter gradients (ws.gW, ws.gb) of one batch: the weighted
     mean squared error sum_n w[n] (Y - T)^2 / (M wsum) of the forward pass
     just run on X (standardised targets T, FP32 [M x 288]; wsum = sum w)."""
     M = ws.M
-    # splits of a weight gradient's sum over the batch: each adds its tiles with atomics, so no more than give half
-    # the CUs a workgroup (16 tiles of 128 x 128; 8192 columns: 26.8 us a product with 32 splits, 19.5 with 8)
-    ks = ksplit or max(1, min(8, M // 256))
+    ks = ksplit or weight_splits(M)
     zero_group([ws.loss, *ws.gW])
     call("pywrf_mlp_mse", M, FOUT, _vp(ws.Y), NO, _vp(T), NO, _vp(w), 1.0 / (M * wsum), _vp(ws.dY), NO,
          _vp(ws.loss), stream())

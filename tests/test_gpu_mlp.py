@@ -198,3 +198,21 @@ def test_column_network_refuses_other_widths(shape):
     net = sg.MLP(seed=1)
     with pytest.raises((ValueError, RuntimeError)):
         adjoint.SurrogateNet.apply(torch.zeros(shape, device="cuda"), net)
+
+
+@pytest.mark.parametrize("M,splits", [(32, 1), (96, 1), (1024, 4), (4128, 8), (70048, 32)])
+def test_weight_gradients_in_any_number_of_splits(M, splits):
+    from pywrf_amd import surrogate as sg
+    assert sg.weight_splits(M) == splits
+    net, ws, w = sg.MLP(seed=2), sg.Workspace(M), sg.loss_weights()
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    X = _bf(torch.randn(M, sg.KIN, device="cuda", generator=gen))
+    T = torch.randn(M, sg.NO, device="cuda", generator=gen)
+    sg.forward(net, X, ws)
+    sg.backward(net, X, T, w, ws, float(w.sum()))
+    got = [g.clone() for g in ws.gW]
+    sg.backward(net, X, T, w, ws, float(w.sum()), ksplit=1)
+    for n, (a, b) in enumerate(zip(got, ws.gW)):
+        # FP32 sums over M terms in two orders: within sqrt(M) eps / 2 of the terms' root of summed squares each,
+        # here over whole matrices of such sums
+        assert float((a - b).norm()) <= 2 * M ** 0.5 * 6e-8 * float(b.norm()), n
