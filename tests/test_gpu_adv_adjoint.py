@@ -1,7 +1,10 @@
-"""The advection adjoints at sizes where a wave's columns, rows and levels run
-out (58 columns, two rows, eight levels), and with values the forward never
+"""The advection adjoints at sizes where a wave's 58 columns, a workgroup's four
+rows and a march of 3 or of 8 levels run out, and with values the forward never
 reads set to NaN: <A(q), lam> = <q, A^T lam> (u and v: A is homogeneous in q,
 its upwind choices those of q itself)."""
+import os
+import re
+
 import pytest
 import torch
 
@@ -22,9 +25,29 @@ def _case(nz, ny, nx, seed):
     return g, f
 
 
+def _march(nz, ny, nx):
+    """Levels a wave marches at that size, from the dispatch's own line."""
+    import pywrf_amd
+    from pywrf_amd.step import Grid
+    src = open(os.path.join(os.path.dirname(pywrf_amd.__file__), "csrc", "adv_adj.hip")).read()
+    line, = re.findall(r"const int kc = \(long\)gx \* \(\(a\.j1 - a\.j0 \+ AA_R - 1\) / AA_R\) \* "
+                       r"\(\(g->nz \+ 7\) / 8\) >= (\d+) \? 8 : 3;", src)
+    assert re.search(r"#define AA_R 1\b", src)
+    g = Grid(nz, ny, nx)
+    return 8 if -(-(g.ide - g.ids) // 58) * (g.jde - g.jds) * ((nz + 7) // 8) >= int(line) else 3
+
+
+SIZES = {(9, 24, 24): 3, (41, 27, 69): 3, (17, 69, 136): 3, (40, 131, 126): 3, (41, 237, 243): 8, (48, 240, 242): 8}
+
+
+@pytest.mark.parametrize("size", list(SIZES))
+def test_the_sizes_take_both_marches(size):
+    assert _march(*size) == SIZES[size]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["scalar", "u", "v", "w"])
-@pytest.mark.parametrize("nz,ny,nx", [(9, 24, 24), (41, 27, 69), (17, 69, 136), (40, 131, 126)])
+@pytest.mark.parametrize("nz,ny,nx", list(SIZES))
 def test_transpose(kind, nz, ny, nx):
     from pywrf_amd import adjoint
     g, f = _case(nz, ny, nx, nz + ny + nx)
