@@ -35,12 +35,10 @@ COPY_REF_FLOATS = 64 * 1024 * 1024   # 256 MiB copy used to scale the HBM byte c
 # 256 MiB copy), from profiles/measured_kernels_240x240x41_hbm_bytes.md and
 # profiles/scalar_transport_240x240x41_hbm_bytes.md.  Only valid at that size; the species transport
 # figure is its later-stage launch (six moisture and two tracer species, advection only).
-TRAFFIC_240 = {"advance_w": 213.9e6, "advance_uv": 194.8e6, "advance_uv_zone": 194.8e6, "advance_mu_t": 131.8e6,
-               "advance_mu_t_zone": 131.8e6, "microphysics_driver": 159.1e6,
-               "advect_scalar_fresh": 101.0e6, "rk_scalar_tend_pair": 778.2e6}
+TRAFFIC_240 = {"advance_w": 190.0e6, "advance_uv": 200.7e6, "advance_mu_t": 112.3e6, "microphysics_driver": 159.1e6,
+               "advect_scalar_fresh": 89.7e6, "rk_scalar_tend_pair": 690.8e6}
 # the HIP kernel each function launches
 KERNEL_OF = {"advance_w": "k_advance_w", "advance_uv": "k_advance_uv", "advance_mu_t": "k_advance_mu_t",
-             "advance_uv_zone": "k_advance_uv", "advance_mu_t_zone": "k_advance_mu_t",
              "microphysics_driver": "k_wsm6", "pgf_buoy_coriolis_curvature": "k_pgf_buoy_cor",
              "advect_scalar_fresh": "k_scalar_adv", "rk_scalar_tend_pair": "k_scalar_adv"}
 FIELD_PASSES_PER_STEP = 700          # algorithmic 3-D field passes per RK3 step (7 acoustic substeps included)
@@ -117,9 +115,6 @@ def call_bytes(name, rk_call, g):
         "advance_w": 20 * n3 + 6 * n2,
         "advance_uv": 14 * n3 + 6 * n2,
         "advance_mu_t": 13 * n3 + 12 * n2,
-        # the zone updates beside them touch rings only
-        "advance_uv_zone": 14 * n3 + 6 * n2,
-        "advance_mu_t_zone": 13 * n3 + 12 * n2,
         "microphysics_driver": 18 * n3 + 7 * n2,
         # pressure gradient + buoyancy + Coriolis + curvature: 15 fields read, 3 tendencies read and written
         "pgf_buoy_coriolis_curvature": 21 * n3 + 12 * n2,

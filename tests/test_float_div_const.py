@@ -1,8 +1,10 @@
 """The flux5 / flux3 face values divide by 60 and 12 through a product by the
-rounded reciprocal plus one fma correction (div_const in csrc/common.h).  This
-runs the exhaustive proof that the form equals the IEEE quotient on every float
-it takes (tests/float_div_const.c); subnormal and infinite inputs and
-subnormal or NaN results take the true division instead."""
+rounded reciprocal plus one fma correction (div_const2 in csrc/common.h).  This
+runs the exhaustive proof that, with the sign of x copied onto it, the form
+equals the IEEE quotient bit for bit on every float that is neither subnormal
+nor infinite and gives no subnormal or NaN (tests/float_div_const.c).  The
+kernels test the result alone and drop a zero's sign: test_float_div_value.py
+has the proof of that."""
 import os
 import shutil
 import subprocess
