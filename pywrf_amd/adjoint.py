@@ -9,7 +9,7 @@ transpose of a linear part of the step:
 * AdvectScalar -- advect_scalar (wrf_dynamics.py:1841-2028) as a function of
   the field, the mass fluxes held fixed.  Backward: pywrf_advect_scalar_adjoint.
 * AdvectU -- advect_u (wrf_dynamics.py:1112-1307) as a function of u, the
-  mass fluxes held fixed.  Backward: pywrf_advect_u_adjoint (scatter form).
+  mass fluxes held fixed.  Backward: pywrf_advect_u_adjoint (gather form).
 * AdvectV, AdvectW -- advect_v (1332-1532) and advect_w (1535-1838) likewise.
 * AdvanceW -- the vertical acoustic step advance_w (wrf_dynamics.py:3641-3796)
   as a function of w, ph, t_2, t_2ave, u, v, muts, muave and ww.  Backward: pywrf_advance_w_adjoint
@@ -17,8 +17,8 @@ transpose of a linear part of the step:
   geopotential right-hand side, in reverse).
 * AdvanceUV -- the horizontal acoustic step advance_uv
   (wrf_dynamics.py:3391-3525) as a function of u, v, ru_tend, rv_tend, p, ph,
-  al, mu and mudf.  Backward: pywrf_advance_uv_adjoint (each u or v column
-  adds its sensitivities into the two columns its differences read).
+  al, mu and mudf.  Backward: pywrf_advance_uv_adjoint (each column takes the
+  shares of the u and v points whose differences read it).
 * AdvanceMuT -- the column-mass and theta acoustic step advance_mu_t
   (wrf_dynamics.py:3528-3638) as a function of u, v, ww, mu, muave, muts,
   mudf, t, t_ave, ft and mu_tend.  Backward: pywrf_advance_mu_t_adjoint (the
@@ -28,8 +28,10 @@ transpose of a linear part of the step:
   spec_bdyupdate_ph (wrf_boundary.py:287-358), zero_grad_bdy (361-405),
   calc_p_rho (wrf_dynamics.py:3269-3313) and a run of open-boundary fills
   (164-278), each on copies of its in-place operands.  With the three above
-  and the zone updates (fixed increments) they chain into the gradient of the
-  whole acoustic loop.
+  and the zone updates (fixed increments) a caller can chain them into the
+  gradient of the whole acoustic loop.
+* AcousticSubstep -- the same nine calls and their adjoints as one node, which
+  is what the loop and stage forms below chain.
 * SmallStepPrep, CalcMuUV1, SmallStepFinish -- small_step_prep past the
   first stage (wrf_dynamics.py:3152-3266), calc_mu_uv_1 (3844-3860) and
   small_step_finish (3863-3978); with the loop they make acoustic_stage, an
@@ -809,11 +811,10 @@ class AcousticSubstep(torch.autograd.Function):
     change (the zone's ring, the halos) is not what the adjoints of the calls
     before them read, except f_in of spec_bdyupdate_ph, which is kept.  Of the
     results w, ph, mu and muts, which a caller may write into, the backward
-    reads copies of its own.  A node
-    per call cost a copy of every such array and an addition for every value
-    that two calls read: 555 launches for a stage of four substeps, forward
-    twice and backward, against 291 (at 120 x 120 x 41 8.8 against 6.1 ms,
-    most of it the host's).
+    reads copies of its own.  A node per call cost a copy of every such array
+    and an addition for every value that two calls read: 555 launches for a
+    stage of four substeps, forward twice and backward, against 291 (at 120 x
+    120 x 41 8.8 against 6.0 to 6.5 ms, most of it the host's).
 
     calls: the nine recorded calls' arguments; given, saved: whether the six
     tendencies (FORCING order) and the six saved fields (SAVED order) follow

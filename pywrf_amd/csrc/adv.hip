@@ -495,9 +495,13 @@ struct ScalarTend {
 // same in a whole wave, so which rule a y- or z-face follows is decided in
 // scalar registers.  The arithmetic and its order are those of the reference.
 //
-// What bounds it is VALU work (a 5th-order face is 26 operations): 2 + (R+1)/R
-// faces a point with R rows against 4 with one row a wave.  Eight species at
-// 240x240x41: 128 -> 102 us a launch, theta 21.5 -> 20.4 us; the six launches of a step at 40x40x41 15.1 -> 8.8 us each.
+// It is near two limits at once.  Eight species at 240x240x41 with four rows
+// issue in 70 % of the VALU slots (a 5th-order face is 26 operations, 2 +
+// (R+1)/R faces a point with R rows against 4 with one row a wave) and move 691
+// MB a launch, halo rows and mass fluxes fetched again for each species
+// included, at 6.7 TB/s; theta, one row, 63 % and 4.5 TB/s.  Eight species
+// 128 -> 102 us a launch, theta 21.5 -> 20.4; the six launches of a step at
+// 40x40x41 15.1 -> 8.8 us each.
 #define SA_OX 58
 #define SA_KC 8   // levels a wave (14 and 21: 0.4-0.8 % of a step slower)
 
@@ -604,10 +608,15 @@ static void pw_launch_scalar_adv(const pywrf_grid_t* g, const ScalarTend& a, pyw
   const bool any = b.size() > 0, fill = a.h_t || a.bzero.size() > imax(0, (int)b.size());
   if (!any && !fill) return;
   // Rows a wave: more rows share more y-faces but make fewer, longer waves, so
-  // four need eight waves for each of the 1024 SIMDs and two need four (eight
-  // species at 240x240x41: 4 rows 28 us a step faster than 2, 12 than 1; six at
-  // 203x237x41: 2 rows 62 us a launch, 4 rows 67, 1 row 69); below that one row,
-  // and half as many levels a wave (a step at 40x40x41: 925 -> 899 us).
+  // four need eight waves for each of the 1024 SIMDs and two need four.  us a
+  // launch with one, two and four rows, the operands in cache (flushed): one
+  // species at 240x240x41 21.8, 21.6, 28.4 (26.8, 29.9, 35.5); eight at
+  // 120x120x41 28.7, 28.4, 32.9 (32.1, 32.0, 38.6), at 320x320x41 241, 215, 191
+  // (243, 216, 195); in a step at 240x240x41 four rows take 28 us less than two
+  // and 12 less than one.  Around the lines the forms differ by 10 % either way
+  // (six species at 240x240x41 80, 89, 83; eight at 203x237x41 90, 86, 76).
+  // Below them one row, and half as many levels a wave (a step at 40x40x41: 925
+  // -> 899 us).
   auto waves = [&](int R, int kc) {
     return (long)((b.ni() + SA_OX - 1) / SA_OX) * ((b.nj() + R - 1) / R) * ((b.nk() + kc - 1) / kc) * nsp;
   };

@@ -13,13 +13,14 @@
 // scalar transport does: lane l holds column i0 - 3 + l, the x-faces are formed
 // once by their own lane and read by DPP lane shifts, the six y-faces around
 // the row are formed from its neighbours, and the six z-faces around a level
-// slide up in registers.  A face is held as two numbers, its weighted sensitivity under the upwind choice it
-// took and zero under the other, so a 5th-order face costs a point two
-// multiply-adds.  Scattering the shares with atomic adds instead (up to 21 a
-// point) was bound by the L2's atomics: u, v, w at 120x120x41 52, 47 and 59 us
-// with the zeroing beside them, here 16 us; the scalar form that gathered
-// with one thread a point 94.5 us at 240x240x41, here 28 us (2.0 TB/s of its six
-// arrays): what is left is each level's load latency with 3 to 5 waves a SIMD.
+// slide up in registers.  A face is held as two numbers, its weighted
+// sensitivity under the upwind choice it took and zero under the other, so a
+// 5th-order face costs a point two multiply-adds.  Scattering the shares with
+// atomic adds instead (up to 21 a point) was bound by the L2's atomics: u, v, w
+// at 120x120x41 52, 47 and 59 us with the zeroing beside them, here 13, 15 and
+// 15 us (32, 36 and 35 at 240x240x41); the scalar form that gathered with one
+// thread a point 94.5 us at 240x240x41, here 28 us (2.0 TB/s of its six arrays):
+// what is left is each level's load latency with 3 to 5 waves a SIMD.
 #include "common.h"
 #include "consts.h"
 
