@@ -228,7 +228,7 @@ _grid_cache = {}
 def grid(shape, idx):
     """pywrf_grid_t for an array shape and an index tuple of 16, 18 or 24 ints
     (the reference's 2-D, tile-only and patch+tile argument lists)."""
-    key = (shape, idx) if type(idx) is tuple else (tuple(shape), tuple(idx))
+    key = (shape, idx) if type(idx) is tuple and type(shape) is not list else (tuple(shape), tuple(idx))
     g = _grid_cache.get(key)
     if g is not None:
         return g

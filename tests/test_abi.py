@@ -97,6 +97,16 @@ def test_grid_packing():
     assert (g2.nz, g2.kds, g2.kde, g2.jte) == (1, 0, 1, 235)
 
 
+def test_grid_takes_any_sequence():
+    from pywrf_amd import _lib
+    from pywrf_amd.step import Grid
+    gr = Grid(41, 40, 50)
+    g = _lib.grid((41, 40, 50), gr.ix18)
+    for shape in ((41, 40, 50), [41, 40, 50]):
+        for idx in (gr.ix18, list(gr.ix18)):
+            assert _lib.grid(shape, idx) is g
+
+
 def test_physics_hooks_leave_the_state_alone():
     """pbl_driver and sixth_order_diffusion are hooks with no arithmetic in the
     reference (wrf_dynamics.py:413-415, 3088-3097: None returned, tendency
